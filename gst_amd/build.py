@@ -128,7 +128,7 @@ def build_oracle():
     """The checker libraries (not part of the product)."""
     oracle = os.path.join(ROOT, "oracle")
     _run(["make", "-s", "-B", "-C", oracle, os.path.join(oracle, "liboracle_gst.so")])
-    if os.path.isdir(REFERENCE):
+    if os.path.exists(os.path.join(REFERENCE, "codec", "encoder.cpp")):
         _run(["make", "-s", "-C", oracle, "ref"])
 
 
