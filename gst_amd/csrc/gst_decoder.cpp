@@ -162,12 +162,7 @@ StageConfig DefaultStageConfig(bool rgb) {
 void SetAnsForm(StageConfig *s, uint32_t form, bool pair = true) {
   s->ans_auto = (form == GST_ANS_FORM_PAIRED || form == GST_ANS_FORM_AUTO) ? 1 : 0;
   s->ans_pair_short = (form == GST_ANS_FORM_PAIRED || (form == GST_ANS_FORM_AUTO && pair)) ? 1 : 0;
-}
-
-uint32_t AnsFormOf(const StageConfig &s) {
-  if (!s.ans_build_tables || s.ans_waves != 4 || s.ans_groups_per_wave != 2) return 0;
-  if (!s.ans_auto) return GST_ANS_FORM_PLAIN;
-  return s.ans_pair_short ? GST_ANS_FORM_PAIRED : GST_ANS_FORM_AUTO;
+  s->ans_chain = 0;
 }
 
 // Whether GST_ANS_FORM_AUTO pairs short remainders for these images: only when their
@@ -181,9 +176,39 @@ bool AutoPairs(const ImageDesc *descs, uint32_t n) {
   return units > 6 * cus;
 }
 
+// Whether GST_ANS_FORM_AUTO takes AnsChainKernel: while its work-groups of four groups fit
+// the device in one pass (four a CU, by LDS).  Up to there it is faster throughout (one
+// image 16.9 against 33.0 us, 4,080 groups 34.5 against 44.1); with a second pass the two
+// meet (4,620 groups 43.5 against 44.5) and AnsAutoKernel, whose waves carry two groups,
+// is ahead (7,200 groups 48.8 against 55.0).
+bool ChainFits(const ImageDesc *descs, uint32_t n) {
+  uint64_t units = 0;
+  for (uint32_t i = 0; i < n; ++i) units += gst::ChainUnitsOf(descs[i]);
+  const uint64_t cus = static_cast<uint64_t>(G().cu_count > 0 ? G().cu_count : 256);
+  return units <= 4 * cus;
+}
+
+// GST_ANS_FORM_AUTO for these images: AnsChainKernel, or AnsAutoKernel with short
+// remainders paired where that saves a pass.
+void SetAutoForm(StageConfig *s, const ImageDesc *descs, uint32_t n) {
+  SetAnsForm(s, GST_ANS_FORM_AUTO, AutoPairs(descs, n));
+  s->ans_chain = ChainFits(descs, n) ? 1 : 0;
+}
+
+uint32_t AnsFormOf(const StageConfig &s) {
+  if (!s.ans_build_tables || s.ans_waves != 4 || s.ans_groups_per_wave != 2) return 0;
+  if (!s.ans_auto) return GST_ANS_FORM_PLAIN;
+  return s.ans_pair_short ? GST_ANS_FORM_PAIRED : GST_ANS_FORM_AUTO;
+}
+
 // Groups per rANS unit, with gst::kAnsPairShort when short remainders pair up.
 uint32_t AnsUnitCode(const StageConfig &s) {
   return s.ans_waves * s.ans_groups_per_wave | (s.ans_pair_short ? gst::kAnsPairShort : 0u);
+}
+
+// The kind of work units a stage's launch strides over.
+uint32_t UnitKind(uint32_t stage, const StageConfig &s) {
+  return stage == gst::kStageAns && s.ans_chain ? gst::kStageChain : stage;
 }
 
 uint32_t *ErrWord(hipStream_t s) {
@@ -264,14 +289,14 @@ class PinnedRing {
 // The used part of a plan of n <= cap images (layout in gst_internal.h): its size is
 // PlanUsedBytes(cap, n).
 void BuildPlan(const std::vector<ImageDesc> &descs, uint32_t cap, uint32_t ans_unit_code,
-               std::vector<uint8_t> *blob, uint32_t units_out[gst::kNumStages]) {
+               std::vector<uint8_t> *blob, uint32_t units_out[gst::kNumUnitKinds]) {
   const uint32_t n = static_cast<uint32_t>(descs.size());
   blob->assign(gst::PlanUsedBytes(cap, n), 0);
   PlanHeader *ph = reinterpret_cast<PlanHeader *>(blob->data());
   ImageDesc *im = reinterpret_cast<ImageDesc *>(blob->data() + gst::PlanImagesOffset(cap));
   ph->n_images = n;
   ph->ans_unit_code = ans_unit_code;
-  for (uint32_t st = 0; st < gst::kNumStages; ++st) {
+  for (uint32_t st = 0; st < gst::kNumUnitKinds; ++st) {
     uint32_t *pre = reinterpret_cast<uint32_t *>(blob->data() + gst::PlanPrefixOffset(cap, st));
     uint32_t acc = 0;
     for (uint32_t i = 0; i < n; ++i) {
@@ -388,7 +413,7 @@ int DecodeStaging(const gst_header *hdrs, uint32_t n, hipStream_t s, const void 
     in_off += StreamBytes(hdrs[i]);
     out_off += rgb ? 3ull * hdrs[i].width * hdrs[i].height : hdrs[i].width * hdrs[i].height / 2ull;
   }
-  SetAnsForm(&cfg, GST_ANS_FORM_AUTO, AutoPairs(descs.data(), n));
+  SetAutoForm(&cfg, descs.data(), n);
   uint32_t *tables = reinterpret_cast<uint32_t *>(sc.ptr + L.tables);
   uint32_t *status = reinterpret_cast<uint32_t *>(sc.ptr + L.status);
   uint32_t grids[gst::kNumStages];
@@ -401,17 +426,17 @@ int DecodeStaging(const gst_header *hdrs, uint32_t n, hipStream_t s, const void 
     a.tables = tables;
     a.table_status = status;
     for (uint32_t st = 0; st < gst::kNumStages; ++st)
-      grids[st] = gst::SinglePassGrid(st, gst::StageUnitsOf(descs[0], st, AnsUnitCode(cfg)), cfg);
+      grids[st] = gst::SinglePassGrid(st, gst::StageUnitsOf(descs[0], UnitKind(st, cfg), AnsUnitCode(cfg)), cfg);
     rc = LaunchAll(a, grids, cfg, s);
   } else {
     std::vector<uint8_t> blob;
-    uint32_t units[gst::kNumStages];
+    uint32_t units[gst::kNumUnitKinds];
     BuildPlan(descs, n, AnsUnitCode(cfg), &blob, units);
     uint8_t *d_blob = sc.ptr + L.plan;
     rc = PinnedRing::Get().Upload(d_blob, blob.data(), blob.size(), s);
     if (rc == GST_OK) {
       const KernelArgs a = PlanArgs(d_blob, n, err, tables, status);
-      for (uint32_t st = 0; st < gst::kNumStages; ++st) grids[st] = gst::SinglePassGrid(st, units[st], cfg);
+      for (uint32_t st = 0; st < gst::kNumStages; ++st) grids[st] = gst::SinglePassGrid(st, units[UnitKind(st, cfg)], cfg);
       rc = LaunchAll(a, grids, cfg, s);
     }
   }
@@ -650,12 +675,12 @@ int gst_load_compressed_dxt_noalloc(const gst_header *hdr, gst_stream stream, co
   memset(&a, 0, sizeof(a));
   FillDesc(*hdr, cmp + offsets_bytes, cmp + offsets_bytes + 2048, base, c, 0, static_cast<uint8_t *>(d_out),
            false, &a.single);
-  SetAnsForm(&cfg, GST_ANS_FORM_AUTO, AutoPairs(&a.single, 1));
+  SetAutoForm(&cfg, &a.single, 1);
   a.ans_unit_code = AnsUnitCode(cfg);
   a.err = d_err_bits;
   uint32_t grids[gst::kNumStages];
   for (uint32_t st = 0; st < gst::kNumStages; ++st)
-    grids[st] = gst::SinglePassGrid(st, gst::StageUnitsOf(a.single, st, AnsUnitCode(cfg)), cfg);
+    grids[st] = gst::SinglePassGrid(st, gst::StageUnitsOf(a.single, UnitKind(st, cfg), AnsUnitCode(cfg)), cfg);
   return LaunchAll(a, grids, cfg, static_cast<hipStream_t>(stream));
 }
 
@@ -740,8 +765,9 @@ struct gst_batch {
   size_t blob_bytes = 0;
   hipEvent_t blob_ev = nullptr;
   bool blob_pending = false;
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t exec = nullptr;
+  uint32_t grid_chain = 0;   // the rANS stage's grid when it runs AnsChainKernel
+  hipGraph_t graph[2] = {};  // [ans_chain]: a bind may move between the two rANS kernels
+  hipGraphExec_t exec[2] = {};
   uint32_t n_bound = 0;
   std::vector<ImageDesc> bound;  // descriptors of the bound images (for re-planning)
   bool auto_form = false;        // GST_ANS_FORM_AUTO: the rANS form is chosen at each bind
@@ -758,7 +784,7 @@ KernelArgs BatchArgs(gst_batch *b) {
 
 // Builds the plan of the bound images for the batch's rANS work-unit size and
 // copies it to the device on `s` through the pinned staging buffer.
-int UploadPlan(gst_batch *b, hipStream_t s, uint32_t units[gst::kNumStages]) {
+int UploadPlan(gst_batch *b, hipStream_t s, uint32_t units[gst::kNumUnitKinds]) {
   std::vector<uint8_t> blob;
   BuildPlan(b->bound, b->cfg.capacity_images, AnsUnitCode(b->stage), &blob, units);
   if (b->blob_pending) GST_HIP(hipEventSynchronize(b->blob_ev));
@@ -775,19 +801,25 @@ int UploadPlan(gst_batch *b, hipStream_t s, uint32_t units[gst::kNumStages]) {
 }
 
 void DropGraph(gst_batch *b) {
-  if (b->exec) (void)hipGraphExecDestroy(b->exec);
-  if (b->graph) (void)hipGraphDestroy(b->graph);
-  b->exec = nullptr;
-  b->graph = nullptr;
+  for (int i = 0; i < 2; ++i) {
+    if (b->exec[i]) (void)hipGraphExecDestroy(b->exec[i]);
+    if (b->graph[i]) (void)hipGraphDestroy(b->graph[i]);
+    b->exec[i] = nullptr;
+    b->graph[i] = nullptr;
+  }
 }
 
-// Captures the five stage launches on `s` into *exec.
-int CaptureStages(gst_batch *b, hipStream_t s, hipGraph_t *graph, hipGraphExec_t *exec) {
+uint32_t GridOf(const gst_batch *b, uint32_t stage, const StageConfig &cfg) {
+  return stage == gst::kStageAns && cfg.ans_chain ? b->grid_chain : b->grids[stage];
+}
+
+// Captures the stage launches of shape `cfg` on `s` into *exec.
+int CaptureStages(gst_batch *b, const StageConfig &cfg, hipStream_t s, hipGraph_t *graph, hipGraphExec_t *exec) {
   GST_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
   const KernelArgs a = BatchArgs(b);
   hipError_t e = hipSuccess;
   for (uint32_t st = 0; st < gst::kNumStages && e == hipSuccess; ++st)
-    e = gst::LaunchStage(st, a, b->grids[st], b->stage, s);
+    e = gst::LaunchStage(st, a, GridOf(b, st, cfg), cfg, s);
   hipGraph_t g = nullptr;
   const hipError_t end = hipStreamEndCapture(s, &g);
   if (e == hipSuccess) e = end;
@@ -866,6 +898,7 @@ int gst_batch_create(const gst_batch_config *cfg, gst_batch **out) {
   const uint32_t cus = static_cast<uint32_t>(G().cu_count > 0 ? G().cu_count : 256);
   b->grids[gst::kStageTables] = 4 * cfg->capacity_images;
   b->grids[gst::kStageAns] = cfg->grid_ans ? cfg->grid_ans : cus * 8;
+  b->grid_chain = b->grids[gst::kStageAns];
   b->grids[gst::kStageIndices] = cfg->grid_indices ? cfg->grid_indices : cus * 4;
   b->grids[gst::kStageWavelet] = cfg->grid_wavelet ? cfg->grid_wavelet : cus * 16;
   // 16 per CU: past the 6 fused work-groups a CU holds at once, so the hardware keeps
@@ -925,9 +958,9 @@ int gst_batch_bind(gst_batch *b, const gst_header *hdrs, uint32_t n, const void 
     off += c.total;
   }
   // The form travels in the plan, so a captured graph replays whichever one a bind picks.
-  if (b->auto_form) SetAnsForm(&b->stage, GST_ANS_FORM_AUTO, AutoPairs(descs.data(), n));
+  if (b->auto_form) SetAutoForm(&b->stage, descs.data(), n);
   b->bound = std::move(descs);
-  uint32_t units[gst::kNumStages];
+  uint32_t units[gst::kNumUnitKinds];
   const int rc = UploadPlan(b, s, units);
   if (rc != GST_OK) return rc;
   b->n_bound = n;
@@ -944,14 +977,14 @@ int gst_batch_autotune(gst_batch *b, gst_stream stream, uint32_t reps, gst_tune_
   StageConfig best = b->stage;
   uint32_t grids[gst::kNumStages];
   memcpy(grids, b->grids, sizeof(grids));
-  uint32_t units[gst::kNumStages];
+  uint32_t units[gst::kNumUnitKinds];
   int rc;
   float ms = 0.f;
 
   // Tables as their own launch (one work-group per table); the rANS shapes that load
   // them are charged this time, the ones that build their table in LDS are not.
   best.ans_build_tables = 0;
-  best.ans_auto = best.ans_pair_short = 0;
+  best.ans_auto = best.ans_pair_short = best.ans_chain = 0;
   grids[gst::kStageTables] = 4 * b->n_bound;
   float t_tables = 0.f;
   if ((rc = TimeStage(b, gst::kStageTables, grids[gst::kStageTables], best, s, reps, &t_tables)) != GST_OK)
@@ -959,24 +992,28 @@ int gst_batch_autotune(gst_batch *b, gst_stream stream, uint32_t reps, gst_tune_
 
   // rANS: streams per wavefront (32 = one group per wave, 64 = two) x waves per
   // work-group x table source (mode 0: loaded, 1: built in LDS; 2 and 3: AnsAutoKernel
-  // with and without short remainders paired, 4 waves x 2 groups) x persistent grid;
-  // each shape needs its own plan (units of W*GPW groups).
+  // with and without short remainders paired, 4 waves x 2 groups; 4: AnsChainKernel, only
+  // where GST_ANS_FORM_AUTO may pick it) x persistent grid; each shape needs its own plan
+  // (units of W*GPW groups).
   static const uint32_t kAnsShapes[][2] = {{1, 2}, {1, 4}, {1, 8}, {2, 1}, {2, 2}, {2, 4}, {2, 8}};
   float best_ms = 1e30f, best_ans = 0.f;
   for (const auto &shape : kAnsShapes) {
-    for (uint32_t mode = 0; mode < 4; ++mode) {
+    for (uint32_t mode = 0; mode < 5; ++mode) {
       const uint32_t build = mode >= 1 ? 1u : 0u;
       if (build && shape[1] < 4) continue;  // the LDS build needs 256 threads
       if (mode >= 2 && !(shape[0] == 2 && shape[1] == 4)) continue;
+      if (mode == 4 && !(b->auto_form && ChainFits(b->bound.data(), b->n_bound))) continue;
       StageConfig c = best;
       c.ans_groups_per_wave = shape[0];
       c.ans_waves = shape[1];
       c.ans_build_tables = build;
       c.ans_auto = mode >= 2 ? 1u : 0u;
       c.ans_pair_short = mode == 2 ? 1u : 0u;
+      c.ans_chain = mode == 4 ? 1u : 0u;
       b->stage = c;
       if ((rc = UploadPlan(b, s, units)) != GST_OK) return rc;
-      const uint32_t cand[] = {cus, 2 * cus, 4 * cus, 8 * cus, units[gst::kStageAns]};
+      const uint32_t cand[] = {cus, 2 * cus, 4 * cus, 8 * cus,
+                               gst::SinglePassGrid(gst::kStageAns, units[UnitKind(gst::kStageAns, c)], c)};
       for (uint32_t g : cand) {
         if ((rc = TimeStage(b, gst::kStageAns, g, c, s, reps, &ms)) != GST_OK) return rc;
         ++res.candidates;
@@ -989,6 +1026,7 @@ int gst_batch_autotune(gst_batch *b, gst_stream stream, uint32_t reps, gst_tune_
           best.ans_build_tables = build;
           best.ans_auto = c.ans_auto;
           best.ans_pair_short = c.ans_pair_short;
+          best.ans_chain = c.ans_chain;
           grids[gst::kStageAns] = g;
         }
       }
@@ -1113,6 +1151,12 @@ int gst_batch_autotune(gst_batch *b, gst_stream stream, uint32_t reps, gst_tune_
   }
 
   b->stage = best;
+  if (best.ans_chain) {
+    // AnsChainKernel won as the form GST_ANS_FORM_AUTO picks for these images; later binds
+    // pick again, and the other kernel keeps its own grid.
+    b->grid_chain = grids[gst::kStageAns];
+    grids[gst::kStageAns] = b->grids[gst::kStageAns];
+  }
   memcpy(b->grids, grids, sizeof(grids));
   DropGraph(b);  // a captured graph holds the old shapes
   res.ans_groups_per_wave = best.ans_groups_per_wave;
@@ -1121,15 +1165,15 @@ int gst_batch_autotune(gst_batch *b, gst_stream stream, uint32_t reps, gst_tune_
   res.assembly_waves_per_group = best.fused_waves;
   res.ans_builds_tables = best.ans_build_tables;
   res.ans_form = AnsFormOf(best);
-  b->auto_form = false;  // the tuned form stays for later binds
+  b->auto_form = best.ans_chain != 0;  // any other tuned form stays for later binds
   res.assembly_wide = best.fused_wide;
   res.wavelet_fused = best.tile_fused;
-  res.grid_ans = grids[gst::kStageAns];
+  res.grid_ans = best.ans_chain ? b->grid_chain : grids[gst::kStageAns];
   res.grid_indices = grids[gst::kStageIndices];
   res.grid_wavelet = grids[gst::kStageWavelet];
   res.grid_assemble = grids[gst::kStageAssemble];
   for (uint32_t st = 0; st < gst::kNumStages; ++st) {
-    if (gst::StageLaunches(st, grids[st], best))
+    if (gst::StageLaunches(st, GridOf(b, st, best), best))
       res.total_ms += res.stage_ms[st];
     else
       res.stage_ms[st] = std::numeric_limits<float>::quiet_NaN();
@@ -1140,18 +1184,27 @@ int gst_batch_autotune(gst_batch *b, gst_stream stream, uint32_t reps, gst_tune_
 
 int gst_batch_decode(gst_batch *b, gst_stream stream) {
   if (!b || b->n_bound == 0) return GST_ERR_INVALID_ARGUMENT;
-  return LaunchAll(BatchArgs(b), b->grids, b->stage, static_cast<hipStream_t>(stream));
+  uint32_t grids[gst::kNumStages];
+  for (uint32_t st = 0; st < gst::kNumStages; ++st) grids[st] = GridOf(b, st, b->stage);
+  return LaunchAll(BatchArgs(b), grids, b->stage, static_cast<hipStream_t>(stream));
 }
 
 int gst_batch_capture_graph(gst_batch *b, gst_stream stream) {
   if (!b || b->n_bound == 0) return GST_ERR_INVALID_ARGUMENT;
-  if (b->exec) return GST_OK;
-  return CaptureStages(b, static_cast<hipStream_t>(stream), &b->graph, &b->exec);
+  // Both rANS kernels where a later bind may pick the other; either decodes any plan.
+  for (uint32_t chain = 0; chain < 2; ++chain) {
+    if (b->exec[chain] || (!b->auto_form && chain != b->stage.ans_chain)) continue;
+    StageConfig c = b->stage;
+    c.ans_chain = chain;
+    const int rc = CaptureStages(b, c, static_cast<hipStream_t>(stream), &b->graph[chain], &b->exec[chain]);
+    if (rc != GST_OK) return rc;
+  }
+  return GST_OK;
 }
 
 int gst_batch_launch_graph(gst_batch *b, gst_stream stream) {
-  if (!b || !b->exec || b->n_bound == 0) return GST_ERR_INVALID_ARGUMENT;
-  GST_HIP(hipGraphLaunch(b->exec, static_cast<hipStream_t>(stream)));
+  if (!b || b->n_bound == 0 || !b->exec[b->stage.ans_chain]) return GST_ERR_INVALID_ARGUMENT;
+  GST_HIP(hipGraphLaunch(b->exec[b->stage.ans_chain], static_cast<hipStream_t>(stream)));
   return GST_OK;
 }
 
@@ -1159,7 +1212,7 @@ int gst_batch_decode_timed_reps(gst_batch *b, gst_stream stream, uint32_t reps, 
   if (!b || !ms || b->n_bound == 0 || reps == 0 || reps > 4096) return GST_ERR_INVALID_ARGUMENT;
   hipStream_t s = static_cast<hipStream_t>(stream);
   uint32_t launched = 0;
-  for (uint32_t st = 0; st < gst::kNumStages; ++st) launched += gst::StageLaunches(st, b->grids[st], b->stage);
+  for (uint32_t st = 0; st < gst::kNumStages; ++st) launched += gst::StageLaunches(st, GridOf(b, st, b->stage), b->stage);
   // One event before the first decode and one after every launched stage; nothing waits
   // on the host until the last, so the decodes run back to back.
   std::vector<hipEvent_t> ev(1 + static_cast<size_t>(reps) * launched, nullptr);
@@ -1171,8 +1224,8 @@ int gst_batch_decode_timed_reps(gst_batch *b, gst_stream stream, uint32_t reps, 
   size_t k = 0;
   for (uint32_t r = 0; r < reps && e == hipSuccess; ++r) {
     for (uint32_t st = 0; st < gst::kNumStages && e == hipSuccess; ++st) {
-      if (!gst::StageLaunches(st, b->grids[st], b->stage)) continue;
-      e = gst::LaunchStage(st, a, b->grids[st], b->stage, s);
+      if (!gst::StageLaunches(st, GridOf(b, st, b->stage), b->stage)) continue;
+      e = gst::LaunchStage(st, a, GridOf(b, st, b->stage), b->stage, s);
       if (e == hipSuccess) e = hipEventRecord(ev[++k], s);
     }
   }
@@ -1181,7 +1234,7 @@ int gst_batch_decode_timed_reps(gst_batch *b, gst_stream stream, uint32_t reps, 
   k = 0;
   for (uint32_t r = 0; r < reps && e == hipSuccess; ++r) {
     for (uint32_t st = 0; st < gst::kNumStages && e == hipSuccess; ++st) {
-      if (!gst::StageLaunches(st, b->grids[st], b->stage)) continue;
+      if (!gst::StageLaunches(st, GridOf(b, st, b->stage), b->stage)) continue;
       float t = 0.f;
       e = hipEventElapsedTime(&t, ev[k], ev[k + 1]);
       sum[st] += t;
@@ -1189,7 +1242,7 @@ int gst_batch_decode_timed_reps(gst_batch *b, gst_stream stream, uint32_t reps, 
     }
   }
   for (uint32_t st = 0; st < gst::kNumStages; ++st)
-    ms[st] = gst::StageLaunches(st, b->grids[st], b->stage)
+    ms[st] = gst::StageLaunches(st, GridOf(b, st, b->stage), b->stage)
                  ? static_cast<float>(sum[st] / reps)
                  : std::numeric_limits<float>::quiet_NaN();  // nothing launched: no time to report
   for (auto x : ev)
@@ -1273,6 +1326,7 @@ int StageLaunch(uint32_t stage, const gst_header *hdr, const uint8_t *d_freqs, c
   cfg.ans_build_tables = 0;
   cfg.ans_auto = 0;
   cfg.ans_pair_short = 0;
+  cfg.ans_chain = 0;
   const uint32_t grid = gst::SinglePassGrid(stage, gst::StageUnitsOf(d, stage, AnsUnitCode(cfg)), cfg);
   GST_HIP(gst::LaunchStage(stage, a, grid, cfg, s));
   return GST_OK;

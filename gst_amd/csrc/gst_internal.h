@@ -25,7 +25,9 @@ enum Stage : uint32_t {
   kStageIndices = 2,
   kStageWavelet = 3,
   kStageAssemble = 4,
-  kNumStages = 5
+  kNumStages = 5,
+  kStageChain = 5,  // not a launch of its own: the rANS stage's work units in AnsChainKernel
+  kNumUnitKinds = 6
 };
 
 enum DevErr : uint32_t {
@@ -139,6 +141,35 @@ __host__ __device__ inline AnsUnit AnsUnitAt(const Desc &d, uint32_t code, uint3
   return r;
 }
 
+// Work units of AnsChainKernel: up to kChainGroups consecutive groups of one stream.
+constexpr uint32_t kChainGroups = 4;
+
+template <typename Desc>
+__host__ __device__ inline uint32_t ChainUnitsOf(const Desc &d) {
+  uint32_t u = 0;
+  for (uint32_t k = 0; k < 4; ++k) u += (d.groups[k] + kChainGroups - 1) / kChainGroups;
+  return u;
+}
+
+// Unit `local` of an image with these groups per stream: stream k, groups first ..
+// first + count - 1.
+struct ChainUnit {
+  uint32_t k, first, count;
+};
+
+__host__ __device__ inline ChainUnit ChainUnitAt(uint32_t g0, uint32_t g1, uint32_t g2, uint32_t g3,
+                                                 uint32_t local) {
+  const uint32_t e0 = (g0 + kChainGroups - 1) / kChainGroups, e1 = e0 + (g1 + kChainGroups - 1) / kChainGroups;
+  const uint32_t e2 = e1 + (g2 + kChainGroups - 1) / kChainGroups;
+  ChainUnit r;
+  r.k = (local >= e0 ? 1u : 0u) + (local >= e1 ? 1u : 0u) + (local >= e2 ? 1u : 0u);
+  const uint32_t start = local >= e2 ? e2 : local >= e1 ? e1 : local >= e0 ? e0 : 0u;
+  const uint32_t groups = local >= e2 ? g3 : local >= e1 ? g2 : local >= e0 ? g1 : g0;
+  r.first = kChainGroups * (local - start);
+  r.count = groups - r.first < kChainGroups ? groups - r.first : kChainGroups;
+  return r;
+}
+
 // `ans_unit_code`: groups per rANS unit, with kAnsPairShort when short remainders pair up.
 __host__ __device__ inline uint32_t StageUnitsOf(const ImageDesc &d, uint32_t stage,
                                                  uint32_t ans_unit_code) {
@@ -147,20 +178,21 @@ __host__ __device__ inline uint32_t StageUnitsOf(const ImageDesc &d, uint32_t st
     case kStageAns: return AnsUnitsOf(d, ans_unit_code);
     case kStageIndices: return d.nv / kGroupSyms;
     case kStageWavelet: return 6 * (d.nv / kTileSyms) / kWaveletTilesPerUnit;
+    case kStageChain: return ChainUnitsOf(d);
     default: return d.nv / kAssembleBlocksPerUnit;
   }
 }
 
 // Device plan for batched decodes of up to `cap` images, n of them bound: the header
-// (padded to 64 bytes), then prefix[kNumStages][cap + 1] (work units per stage,
-// exclusive prefix over the images; entries past index n hold 0xFFFFFFFF), then
+// (padded to 64 bytes), then prefix[kNumUnitKinds][cap + 1] (work units per stage and of
+// AnsChainKernel, so that either rANS kernel decodes any plan; exclusive prefix over the images; entries past index n hold 0xFFFFFFFF), then
 // ImageDesc[cap], of which the first n are used.  Every offset depends on cap alone,
 // which the kernels receive as an argument, so a kernel reads the header and the
 // prefix in one round trip; the used bytes (everything up to the n-th descriptor)
 // are one contiguous copy.
 struct PlanHeader {
   uint32_t n_images;
-  uint32_t units[kNumStages];
+  uint32_t units[kNumUnitKinds];
   uint32_t ans_unit_code;  // groups per rANS unit | kAnsPairShort
 };
 constexpr size_t kPlanHeaderBytes = 64;
@@ -171,7 +203,7 @@ __host__ __device__ inline size_t PlanPrefixOffset(uint32_t cap, uint32_t stage)
   return kPlanHeaderBytes + sizeof(uint32_t) * static_cast<size_t>(stage) * (cap + 1);
 }
 __host__ __device__ inline size_t PlanImagesOffset(uint32_t cap) {
-  return kPlanHeaderBytes + ((sizeof(uint32_t) * kNumStages * (cap + 1) + 63) & ~static_cast<size_t>(63));
+  return kPlanHeaderBytes + ((sizeof(uint32_t) * kNumUnitKinds * (cap + 1) + 63) & ~static_cast<size_t>(63));
 }
 __host__ __device__ inline size_t PlanUsedBytes(uint32_t cap, uint32_t n) {
   return PlanImagesOffset(cap) + sizeof(ImageDesc) * n;
@@ -197,10 +229,10 @@ struct StageConfig {
                                  // or 2 waves of two groups); the table stage launches nothing
   uint32_t ans_pair_short;       // 1: short stream remainders pair up in one work-group
                                  // (4 waves x 2 groups, tables built in LDS)
-  uint32_t ans_auto;             // 1: AnsAutoKernel (4 waves x 2 groups, tables built in LDS):
-                                 // ans_pair_short 1 runs the paired form, 0 the short-chain
-                                 // form (8-byte table and ring entries, one LDS round trip a
-                                 // step); the kernel takes the form from the unit code
+  uint32_t ans_auto;             // 1: AnsAutoKernel (4 waves x 2 groups, tables built in LDS),
+                                 // which takes the form (ans_pair_short) from the unit code
+  uint32_t ans_chain;            // 1, with ans_auto: AnsChainKernel on the same units instead
+                                 // (few groups: a wave per group, one LDS round trip a step)
   uint32_t wavelet_waves;        // waves per wavelet work-group (1, 2, 4); a wave takes 2 units
   uint32_t fused_waves;          // 0: separate index scan and assembly; else waves per
                                  // work-group of the fused scan + DXT1 assembly (1, 2, 4)

@@ -24,11 +24,15 @@ template <typename T>
 using GPtr = __attribute__((address_space(1))) T *;
 template <typename T>
 using CPtr = __attribute__((address_space(4))) const T *;
+template <typename T>
+using LPtr = __attribute__((address_space(3))) T *;
 #else
 template <typename T>
 using GPtr = T *;
 template <typename T>
 using CPtr = const T *;
+template <typename T>
+using LPtr = T *;
 #endif
 
 template <typename T, typename U>
@@ -74,11 +78,15 @@ __device__ __forceinline__ Located Locate(const KernelArgs &a, uint32_t stage, u
 #pragma unroll
     for (uint32_t k = 0; k < 4; ++k) cnt += Popc64(__builtin_amdgcn_ballot_w64(v[k] <= u));
     lo = cnt - 1;  // prefix[0] = 0 <= u
-    start = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(Pick4(v, lo >> 6)),
-                                                            static_cast<int>(lo & 63)));
-    if (lo + 1 < len)
-      next = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(Pick4(v, (lo + 1) >> 6)),
-                                                             static_cast<int>((lo + 1) & 63)));
+    // Four reads of a lane and scalar selects: no branches over the four registers.
+    uint32_t at[4], after[4];
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) {
+      at[k] = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v[k]), static_cast<int>(lo & 63)));
+      after[k] = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v[k]), static_cast<int>(cnt & 63)));
+    }
+    start = Pick4(at, lo >> 6);
+    next = cnt < 256 ? Pick4(after, cnt >> 6) : kPrefixPad;  // entries past the plan's are padding
   } else {
     lo = 0;
     uint32_t m = len;  // the answer lies in [lo, lo + m)
@@ -144,6 +152,18 @@ __device__ __forceinline__ DevDesc LoadDesc(const KernelArgs &a, uint32_t img) {
   d.lane_sums = Gbl<int32_t>(s.lane_sums);
   d.out = Gbl<uint8_t>(s.out);
   return d;
+}
+
+// The descriptor of image img in constant memory, the plan's or the kernel argument's, for
+// kernels that pick a stream's fields by index with scalar loads.
+__device__ __forceinline__ CPtr<ImageDesc> DescAt(const KernelArgs &a, uint32_t img) {
+  if (a.plan)
+    return (CPtr<ImageDesc>)(reinterpret_cast<uintptr_t>(a.plan) + PlanImagesOffset(a.plan_cap)) + img;
+#if defined(__HIP_DEVICE_COMPILE__)
+  return (CPtr<ImageDesc>)((CPtr<uint8_t>)__builtin_amdgcn_kernarg_segment_ptr() + offsetof(KernelArgs, single));
+#else
+  return &a.single;
+#endif
 }
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t MakeRsrc(const void *base, uint32_t bytes) {
@@ -552,77 +572,88 @@ __device__ __forceinline__ const uint8_t *Uniform(const uint8_t *p) {
 // not for its global loads in flight (a __syncthreads fence would wait for those too).
 __device__ __forceinline__ void LdsBarrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// The work of BuildTableKernel for one table, straight into the rANS kernel's LDS
-// (256 <= THREADS): thread t < 256 brings frequency f[t].  The slot -> symbol map is a
-// count, not a search.  Wave w owns slots [w S, (w + 1) S), S = 2048 / waves, lane l
-// slot w S + 64 j + l of chunk j:
-//   A. the waves clear their slots and the marks-before counters; the first four waves
-//      scan f + (f != 0) << 24, giving every symbol its cum (low 24 bits: 256 u16 sum
-//      below 2^24) and its rank among the nonzero symbols (high bits);
-//   B. every nonzero symbol x writes fc[x] = f | cum << 12, sym_of_rank[rank] = x and a
-//      start mark at slot cum[x], and each wave of symbols adds to before[w] how many
-//      of its marks fall below slot w S (a ballot per boundary, one LDS add);
-//   C. per chunk, a ballot of the marks and mbcnt give the marks up to each slot, so
-//      slot s gets symbol sym_of_rank[before + marks in the wave's slots up to s - 1].
-// Every LDS access of A and C is one word per lane at consecutive addresses.  A table
-// that does not sum to 2048 becomes the identity table.  Returns whether the table is
-// valid; ends with a work-group barrier.
-template <uint32_t THREADS>
-__device__ __forceinline__ bool BuildTableInLds(uint32_t f, uint32_t *tab, uint32_t *fc, uint8_t *sym_of_rank,
-                                                uint32_t *wsum, uint32_t *before) {
+// Inclusive prefix sum over a wave in six DPP adds (row shifts, then row broadcasts): no LDS
+// round trip, where __shfl_up is a ds_bpermute each.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t DppAdd(uint32_t v) {
+  return v + static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), CTRL, ROWS, 0xF, false));
+}
+__device__ __forceinline__ uint32_t WaveInclusiveSum(uint32_t v) {
+  v = DppAdd<0x111, 0xF>(v);  // row_shr:1
+  v = DppAdd<0x112, 0xF>(v);  // row_shr:2
+  v = DppAdd<0x114, 0xF>(v);  // row_shr:4
+  v = DppAdd<0x118, 0xF>(v);  // row_shr:8
+  v = DppAdd<0x142, 0xA>(v);  // row_bcast:15 into rows 1 and 3
+  return DppAdd<0x143, 0xC>(v);  // row_bcast:31 into rows 2 and 3
+}
+
+// The work of BuildTableKernel for one table, straight into a rANS kernel's LDS (256 <=
+// THREADS): thread t < 256 brings frequency f[t].  The slot -> symbol map is a count, not a
+// search:
+//   A. the marks are cleared (a bit a slot); the first four waves scan f + (f != 0) << 24,
+//      giving every symbol its cum (low 24 bits: 256 u16 sum below 2^24) and its rank
+//      among the nonzero symbols (high bits);
+//   B. every nonzero symbol x writes {f | x << 24, cum} at its rank and sets the mark of
+//      slot cum;
+//   C. each wave counts the marks before its 64-slot chunks (a lane per chunk and one DPP
+//      scan), and mbcnt over a chunk's marks, in scalar registers, gives each slot the
+//      rank of its symbol: one gather a slot, all of a wave's in flight together.
+// A table that does not sum to 2048 becomes the identity table.  `put(slot, {f | symbol
+// << 24, slot - cum})` stores an entry.  Returns whether the table is valid; ends with a
+// work-group barrier.  One round trip of gathers where a first version had three a chunk
+// (marks, rank to symbol, symbol to frequency), with ds_bpermute scans: 4,300 -> 2,060
+// cycles for a work-group alone on its CU.
+constexpr uint32_t kBuildScratchWords = 2 * 256 + kTableSize / 32 + 4;
+
+template <uint32_t THREADS, typename Put>
+__device__ __forceinline__ bool BuildTableInLds(uint32_t f, uint32_t *scratch, Put put) {
   constexpr uint32_t kWaves = THREADS / 64, kSlotsPerWave = kTableSize / kWaves, kChunks = kSlotsPerWave / 64;
-  static_assert(THREADS >= 256 && kWaves <= 8 && kChunks * 64 * kWaves == kTableSize, "launch shape");
+  static_assert(THREADS >= 256 && kChunks * 64 * kWaves == kTableSize, "launch shape");
+  u32x2 *const ent = reinterpret_cast<u32x2 *>(scratch);   // [256], by rank
+  uint32_t *const marks = scratch + 512;                   // a bit per slot
+  uint32_t *const wsum = scratch + 512 + kTableSize / 32;  // [4]
   const uint32_t t = threadIdx.x, lane = t & 63, wave = Uniform(t >> 6);
-  uint32_t *const mine = tab + wave * kSlotsPerWave + lane;
-#pragma unroll
-  for (uint32_t j = 0; j < kChunks; ++j) mine[64 * j] = 0;
-  if (t < kWaves) before[t] = 0;
+  if (t < kTableSize / 32) marks[t] = 0;
   const uint32_t pk = f + (static_cast<uint32_t>(f != 0) << 24);
-  uint32_t v = 0;
-  if (t < 256) {
-    v = pk;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const uint32_t n = __shfl_up(v, off);
-      if (lane >= static_cast<uint32_t>(off)) v += n;
-    }
-    if (lane == 63) wsum[wave] = v;
-  }
+  const uint32_t v = WaveInclusiveSum(pk);
+  if (lane == 63 && t < 256) wsum[wave] = v;
   LdsBarrier();
-  const bool valid = ((wsum[0] + wsum[1] + wsum[2] + wsum[3]) & 0xFFFFFFu) == kTableSize;
-  if (t < 256 && valid) {
-    uint32_t add = 0;
-    for (uint32_t w = 0; w < wave; ++w) add += wsum[w];
+  const u32x4 ws = *reinterpret_cast<const u32x4 *>(wsum);
+  const bool valid = Uniform((ws.x + ws.y + ws.z + ws.w) & 0xFFFFFFu) == kTableSize;
+  if (valid && t < 256) {
+    const uint32_t add = (wave > 0 ? ws.x : 0u) + (wave > 1 ? ws.y : 0u) + (wave > 2 ? ws.z : 0u);
     const uint32_t excl = add + v - pk, cum = excl & 0xFFFFFFu;
-    fc[t] = f | (cum << 12);
     if (f != 0) {  // the table sums to 2048, so cum + f <= 2048: the mark is inside it
-      sym_of_rank[excl >> 24] = static_cast<uint8_t>(t);
-      tab[cum] = 1;
-    }
-#pragma unroll
-    for (uint32_t w = 1; w < kWaves; ++w) {
-      const uint32_t below = static_cast<uint32_t>(__popcll(__builtin_amdgcn_ballot_w64(f != 0 && cum < w * kSlotsPerWave)));
-      if (lane == 0 && below) atomicAdd(&before[w], below);
+      ent[excl >> 24] = u32x2{f | (t << 24), cum};
+      atomicOr(&marks[cum >> 5], 1u << (cum & 31));
     }
   }
   LdsBarrier();
+  const uint32_t slot0 = wave * kSlotsPerWave + lane;
   if (valid) {
-    uint32_t base = before[wave];
+    const u32x2 m = reinterpret_cast<const u32x2 *>(marks)[lane & 31];  // lane c: chunk c's marks
+    const uint32_t n = lane < 32 ? static_cast<uint32_t>(__popc(m.x) + __popc(m.y)) : 0u;
+    // Rank of a slot's symbol: marks at slots up to it, less 1 = those of earlier chunks and
+    // of the chunk's first slot, then mbcnt (lanes below) over the marks moved down a slot.
+    const uint32_t first = WaveInclusiveSum(n) - n + (m.x & 1u) - 1u;
+    u32x2 e[kChunks];
 #pragma unroll
     for (uint32_t j = 0; j < kChunks; ++j) {
-      const uint32_t mark = mine[64 * j];
-      const uint64_t bal = __builtin_amdgcn_ballot_w64(mark != 0);
-      const uint32_t upto = base + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(bal >> 32),
-                                                             __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(bal), mark));
-      const uint32_t x = sym_of_rank[(upto - 1) & 255];
-      const uint32_t w = fc[x];
-      const uint32_t slot = wave * kSlotsPerWave + 64 * j + lane;
-      mine[64 * j] = (w & 0xFFFu) | ((slot - (w >> 12)) << 12) | (x << 24);
-      base += static_cast<uint32_t>(__popcll(bal));
+      const int c = static_cast<int>(wave * kChunks + j);
+      const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(m.x), c));
+      const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(m.y), c));
+      const uint64_t up = ((static_cast<uint64_t>(hi) << 32) | lo) >> 1;
+      const uint32_t rank = __builtin_amdgcn_mbcnt_hi(
+          static_cast<uint32_t>(up >> 32),
+          __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(up),
+                                    static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(first), c))));
+      e[j] = ent[rank & 255];
     }
+#pragma unroll
+    for (uint32_t j = 0; j < kChunks; ++j) put(slot0 + 64 * j, u32x2{e[j].x, slot0 + 64 * j - e[j].y});
   } else {
 #pragma unroll
-    for (uint32_t j = 0; j < kChunks; ++j) mine[64 * j] = kTableSize | ((wave * kSlotsPerWave + 64 * j + lane) << 12);
+    for (uint32_t j = 0; j < kChunks; ++j) put(slot0 + 64 * j, u32x2{kTableSize, slot0 + 64 * j});
   }
   LdsBarrier();
   return valid;
@@ -639,10 +670,7 @@ __device__ __forceinline__ bool BuildTableInLds(uint32_t f, uint32_t *tab, uint3
 // frequencies go out with the offsets and the states and chunks before the table is
 // built, so the LDS build overlaps their latency.
 // LDS of the rANS kernels beside their tables and rings.
-template <uint32_t WAVES>
 struct AnsLdsSmall {
-  uint32_t build_wsum[4];
-  uint32_t build_before[WAVES];
   uint32_t touch_sink[64];
 };
 
@@ -657,15 +685,12 @@ struct AnsLds {
 
 template <uint32_t WAVES, uint32_t GPW, bool kBuild, bool kPair>
 __device__ __forceinline__ void AnsDecodeUnits(const KernelArgs &a, AnsLds<WAVES, kPair> &L,
-                                               AnsLdsSmall<WAVES> &S) {
+                                               AnsLdsSmall &S) {
   static_assert(!kPair || (kBuild && WAVES % 2 == 0), "paired units build their tables in LDS");
-  static_assert(WAVES * 2 * kRingWords * 2 >= 256 * 4 + 256, "build scratch fits the rings");
+  static_assert(!kBuild || WAVES * 2 * kRingWords * 2 >= 4 * kBuildScratchWords, "build scratch fits the rings");
   auto &tab = L.tab;
   auto &ring = L.ring;
-  uint32_t *const build_fc = reinterpret_cast<uint32_t *>(&ring[0][0][0]);
-  uint8_t *const build_sym = reinterpret_cast<uint8_t *>(build_fc + 256);
-  uint32_t *const build_wsum = S.build_wsum;
-  uint32_t *const build_before = S.build_before;
+  uint32_t *const build_scratch = reinterpret_cast<uint32_t *>(&ring[0][0][0]);
   uint32_t *const touch_sink = S.touch_sink;
   constexpr uint32_t kGroupsPerUnit = WAVES * GPW;
   constexpr uint32_t kUnitCode = kGroupsPerUnit | (kPair ? kAnsPairShort : 0u);
@@ -722,10 +747,13 @@ __device__ __forceinline__ void AnsDecodeUnits(const KernelArgs &a, AnsLds<WAVES
     LdsBarrier();  // every wave is done with the previous unit's tables and rings
     bool table_ok;
     if constexpr (kBuild) {
-      table_ok = BuildTableInLds<WAVES * 64>(f, tab[0], build_fc, build_sym, build_wsum, build_before);
+      // Entries packed as in the kernel's header comment: the slot's offset is below 2^11.
+      const auto put = [](uint32_t *t) {
+        return [t](uint32_t slot, const u32x2 &e) { t[slot] = e.x | (e.y << 12); };
+      };
+      table_ok = BuildTableInLds<WAVES * 64>(f, build_scratch, put(tab[0]));
       if (kPair && second)
-        table_ok = BuildTableInLds<WAVES * 64>(f2, tab[kPair ? 1 : 0], build_fc, build_sym, build_wsum,
-                                               build_before) && table_ok;
+        table_ok = BuildTableInLds<WAVES * 64>(f2, build_scratch, put(tab[kPair ? 1 : 0])) && table_ok;
     } else {
       const uint32_t tix = Uniform(d.table_base + k);
       const GPtr<const uint32_t> src = Gbl<const uint32_t>(a.tables + static_cast<size_t>(tix) * kTableSize);
@@ -761,7 +789,7 @@ template <uint32_t WAVES, uint32_t GPW, bool kBuild, bool kPair = false>
 __global__ __launch_bounds__(WAVES * 64, kPair ? 6 : WAVES >= 4 ? 7 : 1)
 void AnsDecodeKernel(KernelArgs a) {
   __shared__ __align__(16) AnsLds<WAVES, kPair> lds;
-  __shared__ AnsLdsSmall<WAVES> small;
+  __shared__ AnsLdsSmall small;
   AnsDecodeUnits<WAVES, GPW, kBuild, kPair>(a, lds, small);
 }
 
@@ -779,12 +807,286 @@ union AnsAutoLds {
 
 __global__ __launch_bounds__(kAutoWaves * 64, 6) void AnsAutoKernel(KernelArgs a) {
   __shared__ __align__(16) AnsAutoLds lds;
-  __shared__ AnsLdsSmall<kAutoWaves> small;
+  __shared__ AnsLdsSmall small;
   const uint32_t code = a.plan ? Uniform(Gbl<const uint32_t>(&a.plan->ans_unit_code)[0]) : a.ans_unit_code;
   if (code & kAnsPairShort)
     AnsDecodeUnits<kAutoWaves, 2, true, true>(a, lds.paired, small);
   else
     AnsDecodeUnits<kAutoWaves, 2, true, false>(a, lds.single, small);
+}
+
+// ---------------------------------------------------------------------------
+// The rANS stage where latency bounds it: few groups, so that every SIMD holds at most a
+// handful of decoding waves and a step costs its dependency chain, not its issue slots.
+//
+// A wave decodes one group (32 lanes), and a step has one LDS round trip.  The lane's
+// state y is kept as it comes out of the update, before renormalisation:
+//   keep   (y >= L): next y = (y >> 11) f + off, {f, off} the table entry of slot y & 2047
+//   renorm (y <  L): x = y << 16 | w, so (x >> 11) f + off = y (32 f) + ((w >> 11) f + off)
+// with the entry of slot w & 2047: everything but y is known from the word alone.  So the
+// table holds {f | symbol << 24, off} and the ring, next to it in LDS, the renormalising
+// entry {32 f | symbol << 24, (w >> 11) f + off} of every word, made when its chunk comes
+// in (64 words' gathers in parallel, off the chain).  A step selects one of two LDS
+// addresses and one of two multiplicands, reads 8 bytes and does one v_mad_u32_u24 (which
+// takes the low 24 bits of both factors, so the symbol rides along): mad, compare, mbcnt,
+// address, select, read.
+//
+// Lane l decodes stream 31 - l and the ring is stored in reading order (descending word
+// index), so a lane's word is `q` + the renormalising lanes below it: mbcnt gives it
+// without waiting for the total.  The ring has two 256-word chunks and a copy of the
+// first behind the second: the 256 words that 8 steps can read at most are consecutive
+// from any q < 512, and addresses need no wrap.  q (a scalar byte address) moves by 8
+// times the popcount while the read is in flight; each 8 steps it is compared with the
+// chunk's end, and a crossing writes the chunk requested two crossings earlier.
+//
+// A step is bound by that chain: 123 cycles with the refills, about 52 of them the LDS read,
+// against some 280 in AnsAutoKernel (two LDS round trips, 12 dependent VALU, two scalar
+// hops).  Stage times, this kernel against AnsAutoKernel: one 512x512 image 16.9 / 33.0 us,
+// 1024x1024 images by the dozen: 8 (480 groups) 21.6 / 35.4, 34 (2,040) 28.7 / 39.8, 68
+// (4,080, four waves a SIMD) 34.5 / 44.1.  LDS holds four work-groups a CU; a second pass
+// loses the gain (4,620 groups: 43.5 / 44.5; 7,200: 55.0 / 48.8).
+constexpr uint32_t kChainWaves = kChainGroups;
+constexpr uint32_t kChainRing = 3 * kChunkWords;  // entries per wave
+
+struct AnsChainLds {
+  u32x2 tab[kTableSize];
+  u32x2 ring[kChainWaves][kChainRing];
+};
+static_assert(sizeof(AnsChainLds) == 40960, "four work-groups per CU");
+
+// The renormalising entries of lane l's four words of a chunk, in reading order, at entry
+// `at` of the ring (and again at `copy`, for the chunk the ring holds twice).
+__device__ __forceinline__ void StoreChainChunk(const u32x2 *tab, u32x2 *ring, uint32_t at, bool twice, uint32_t l,
+                                                const u32x2 &w) {
+  u32x4 o[2];
+  uint32_t word[4] = {w.x & 0xFFFFu, w.x >> 16, w.y & 0xFFFFu, w.y >> 16};
+  u32x2 e[4];
+#pragma unroll
+  for (uint32_t k = 0; k < 4; ++k) e[k] = tab[word[k] & (kTableSize - 1)];
+#pragma unroll
+  for (uint32_t k = 0; k < 4; ++k) {
+    const uint32_t f = e[k].x & 0xFFFFFFu;
+    const uint32_t lo = (f << 5) | (e[k].x & 0xFF000000u);
+    const uint32_t hi = __umul24(word[k] >> kTableLog, f) + e[k].y;
+    const uint32_t pos = 3 - k;
+    o[pos >> 1][(pos & 1) * 2] = lo;
+    o[pos >> 1][(pos & 1) * 2 + 1] = hi;
+  }
+  u32x4 *const d = reinterpret_cast<u32x4 *>(ring + at + kChunkWords - 4 - 4 * l);
+  d[0] = o[0];
+  d[1] = o[1];
+  if (twice) {
+    d[kChunkWords] = o[0];
+    d[kChunkWords + 1] = o[1];
+  }
+}
+
+// The reading half of a step: the lane's entry {multiplier | symbol << 24, addend} and the
+// state's multiplicand `mul`; moves q past the words the wave's lanes take, and (kInsert)
+// puts the previous step's symbol (bits 24-31 of `last`) into `acc`.  One block in a fixed
+// order: the address chain first, what fits behind it while the read is in flight, and
+// the wait (left to the compiler a step took 135 cycles, this way 123; a read of either
+// entry under its own exec mask, without the address select, also 135).  LDS addresses are those
+// of AnsChainLds at address 0, the kernel's only LDS object.
+template <bool kInsert>
+__device__ __forceinline__ u32x2 ChainStep(const uint32_t &y, uint32_t thr, uint32_t &q, uint32_t &mul,
+                                           uint32_t last, uint32_t &acc, uint32_t sel) {
+  u32x2 e;
+#if defined(__HIP_DEVICE_COMPILE__)
+  uint32_t slot, rank, moved;
+#define GST_CHAIN_ADDRESS                          \
+  "v_cmp_lt_u32 vcc, %[y], %[thr]\n\t"             \
+  "v_lshlrev_b32 %[slot], 3, %[y]\n\t"             \
+  "v_mbcnt_lo_u32_b32 %[rank], vcc_lo, 0\n\t"      \
+  "v_and_b32 %[slot], 0x3ff8, %[slot]\n\t"         \
+  "v_lshl_add_u32 %[rank], %[rank], 3, %[q]\n\t"   \
+  "v_cndmask_b32 %[slot], %[slot], %[rank], vcc\n\t" \
+  "ds_read_b64 %[e], %[slot]\n\t"
+#define GST_CHAIN_BEHIND                           \
+  "v_lshrrev_b32 %[mul], 11, %[y]\n\t"             \
+  "s_bcnt1_i32_b32 %[moved], vcc_lo\n\t"           \
+  "v_cndmask_b32 %[mul], %[mul], %[y], vcc\n\t"    \
+  "s_lshl_b32 %[moved], %[moved], 3\n\t"           \
+  "s_add_u32 %[q], %[q], %[moved]\n\t"             \
+  "s_waitcnt lgkmcnt(0)"
+  if constexpr (kInsert)
+    asm volatile(GST_CHAIN_ADDRESS "v_perm_b32 %[acc], %[last], %[acc], %[sel]\n\t" GST_CHAIN_BEHIND
+                 : [e] "=&v"(e), [slot] "=&v"(slot), [rank] "=&v"(rank), [mul] "=&v"(mul), [q] "+s"(q),
+                   [moved] "=&s"(moved), [acc] "+v"(acc)
+                 : [y] "v"(y), [thr] "v"(thr), [last] "v"(last), [sel] "s"(sel)
+                 : "vcc", "scc", "memory");
+  else
+    asm volatile(GST_CHAIN_ADDRESS GST_CHAIN_BEHIND
+                 : [e] "=&v"(e), [slot] "=&v"(slot), [rank] "=&v"(rank), [mul] "=&v"(mul), [q] "+s"(q),
+                   [moved] "=&s"(moved)
+                 : [y] "v"(y), [thr] "v"(thr)
+                 : "vcc", "scc", "memory");
+#undef GST_CHAIN_ADDRESS
+#undef GST_CHAIN_BEHIND
+#endif
+  return e;
+}
+
+// One group: lanes 0..31 decode streams 31..0 from state y, their words below word p
+// (chunk top first, chunks below clo read zeros), with E and O the chunks top - 2 and
+// top - 3 in flight.  Returns how many words the group consumed.
+template <bool kSum>
+__device__ __forceinline__ uint32_t DecodeGroupChain(const AnsChainLds &lds, u32x2 *ring, uint32_t ring_at,
+                                                     __amdgpu_buffer_rsrc_t rs, uint32_t lane, uint32_t y,
+                                                     uint32_t p, uint32_t clo, u32x2 pE, u32x2 pO,
+                                                     GPtr<uint8_t> outp, GPtr<int32_t> group_sum,
+                                                     GPtr<int32_t> lane_sum, GPtr<int32_t> lane_suffix) {
+  const bool active = lane < kLanesPerGroup;
+  const uint32_t j = 31 - (lane & 31);
+  const uint32_t full = active ? kStateL : 0u;
+  uint32_t thr = 0;  // a group's first step never renormalises: its states come as stored
+  asm volatile("" : "+v"(thr));
+  uint32_t top = p ? (p - 1) / kChunkWords : 0u;
+  const uint32_t q0 = ring_at + 8 * (kChunkWords - 1 - ((p - 1) & (kChunkWords - 1)));
+  uint32_t q = Uniform(q0);
+  const uint32_t end0 = ring_at + 8 * kChunkWords, end1 = ring_at + 16 * kChunkWords;
+  uint32_t limit = end0, wraps = 0;
+  int32_t sum = 0;
+  for (uint32_t sector = 0; sector < kSymsPerLane / 64; ++sector) {
+    uint32_t acc[16], last = 0, none = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < 16; ++i) acc[i] = 0;
+#pragma unroll
+    for (uint32_t blk = 0; blk < 64 / kRefillSteps; ++blk) {
+#pragma unroll
+      for (uint32_t s = 0; s < kRefillSteps; ++s) {
+        // The last step's symbol goes in while this step's read is in flight: byte `at` of
+        // the sector (the first step's has no predecessor in it).
+        const uint32_t at = 64 - kRefillSteps * blk - s;
+        const uint32_t sel = (0x03020100u & ~(0xFFu << (8 * (at & 3)))) | (7u << (8 * (at & 3)));
+        uint32_t mul;
+        u32x2 e;
+        if (at == 64)
+          e = ChainStep<false>(y, thr, q, mul, 0u, none, sel);
+        else
+          e = ChainStep<true>(y, thr, q, mul, last, acc[at >> 2], sel);
+        y = __umul24(mul, e.x) + e.y;
+        last = e.x;
+        if (at == 64) thr = full;
+        if (s == kRefillSteps - 1) {
+          // 8 steps read at most 256 words, so at most one chunk's end was crossed.  Two
+          // uniform branches, not an if/else, so that each request stays in its register.
+          const bool cross0 = q >= limit && limit == end0, cross1 = q >= limit && limit == end1;
+          if (cross0) {
+            StoreChainChunk(lds.tab, ring, 0, true, lane, pE);
+            asm volatile("" ::: "memory");
+            pE = LoadChunk(rs, top - 4, clo, lane);
+            limit = end1;
+            --top;
+          }
+          if (cross1) {
+            StoreChainChunk(lds.tab, ring, kChunkWords, false, lane, pO);
+            asm volatile("" ::: "memory");
+            pO = LoadChunk(rs, top - 4, clo, lane);
+            limit = end0;
+            --top;
+            q -= 16 * kChunkWords;
+            ++wraps;
+          }
+          WaveSync();
+        }
+      }
+    }
+    acc[0] = __builtin_amdgcn_perm(last, acc[0], 0x03020107u);
+    if (kSum) {
+      // As in DecodeHalfGroups: the sector's suffix sums from 32-symbol steps.
+      uint32_t lo = 0, hi = 0;
+#pragma unroll
+      for (uint32_t i = 0; i < 8; ++i) lo = __builtin_amdgcn_sad_u8(acc[i], 0u, lo);
+#pragma unroll
+      for (uint32_t i = 8; i < 16; ++i) hi = __builtin_amdgcn_sad_u8(acc[i], 0u, hi);
+      const int32_t r_hi = sum + static_cast<int32_t>(hi) - 32 * 128;
+      const int32_t r_lo = r_hi + static_cast<int32_t>(lo) - 32 * 128;
+      sum = r_lo;
+      if (active && lane_suffix)
+        *(GPtr<int2>)(lane_suffix + 8 * j + 6 - 2 * sector) = make_int2(r_lo, r_hi);
+    }
+    if (active) {
+      const GPtr<uint4> dst = (GPtr<uint4>)(outp + j * kSymsPerLane + (kSymsPerLane - 64) - 64 * sector);
+#pragma unroll
+      for (uint32_t i = 0; i < 4; ++i)
+        dst[i] = make_uint4(acc[4 * i], acc[4 * i + 1], acc[4 * i + 2], acc[4 * i + 3]);
+    }
+  }
+  if (kSum) {
+    // Inclusive prefix over the streams, which run down the lanes.
+    int32_t incl = sum;
+#pragma unroll
+    for (uint32_t off = 1; off < 32; off <<= 1) {
+      const int32_t n = __shfl_down(incl, off, 32);
+      if (j >= off) incl += n;
+    }
+    if (active && lane_sum) lane_sum[j] = incl;
+    if (lane == 0) *group_sum = incl;
+  }
+  q += 8 * static_cast<uint32_t>(__popc(static_cast<uint32_t>(__builtin_amdgcn_uicmp(y, full, 36 /* ULT */))));
+  return (q + 16 * kChunkWords * wraps - q0) / 8;
+}
+
+// A work-group takes four consecutive groups of one stream, a wave each; the waves past
+// the stream's last group only help with the table.
+__global__ __launch_bounds__(kChainWaves * 64, 4) void AnsChainKernel(KernelArgs a) {
+  __shared__ __align__(16) AnsChainLds lds;
+  const uint32_t lane = threadIdx.x & 63, wave = Uniform(threadIdx.x >> 6);
+  const uint32_t lane_stream = 31 - (lane & 31);
+  for (uint32_t w = blockIdx.x;; w += gridDim.x) {
+    const Located loc = Locate(a, kStageChain, w, 0);
+    if (!loc.valid) break;
+    const CPtr<ImageDesc> d = DescAt(a, loc.img);
+    const ChainUnit unit = ChainUnitAt(d->groups[0], d->groups[1], d->groups[2], d->groups[3], loc.local);
+    const uint32_t k = unit.k, g = unit.first + wave;
+    const uint32_t G = d->groups[k], slen = d->stream_len[k], nv = d->nv;
+    const __amdgpu_buffer_rsrc_t rs = MakeRsrc(d->streams[k], slen);
+    uint32_t end_v = __builtin_amdgcn_raw_buffer_load_b32(rs, static_cast<int>(4 * g), 0, 0);
+    uint32_t lo_v = __builtin_amdgcn_raw_buffer_load_b32(rs, static_cast<int>(4 * (g - 1)), 0, 0);
+    const GPtr<const uint16_t> fr = Gbl<const uint16_t>(d->freqs + 512 * k);
+    const uint32_t f = fr[threadIdx.x];
+    asm volatile("" : "+v"(end_v), "+v"(lo_v));  // one wait for both: else the second load waits for g != 0
+    const uint32_t end = Uniform(end_v), lo = g == 0 ? 4 * G : Uniform(lo_v);
+    const bool ok = ((end | lo) & 3) == 0 && end <= slen && lo >= 4 * G && lo <= end &&
+                    end - lo >= 4 * kLanesPerGroup;
+    const bool in_stream = wave < unit.count;
+    if (in_stream && !ok && lane == 0) atomicOr(a.err, kErrStreamOffsets);
+    const bool active = in_stream && ok;
+    const uint32_t x_word = __builtin_amdgcn_raw_buffer_load_b32(
+        rs, static_cast<int>(end - 4 * kLanesPerGroup + 4 * lane_stream), 0, 0);
+    const uint32_t x = active && lane < kLanesPerGroup ? x_word : 0u;
+    const uint32_t p = active ? (end - 4 * kLanesPerGroup) >> 1 : 0u;
+    const uint32_t plo = active ? lo >> 1 : 0u;
+    const uint32_t top = p ? (p - 1) / kChunkWords : 0u, clo = plo / kChunkWords;
+    const u32x2 c0 = LoadChunk(rs, top, clo, lane), c1 = LoadChunk(rs, top - 1, clo, lane);
+    const u32x2 pE = LoadChunk(rs, top - 2, clo, lane), pO = LoadChunk(rs, top - 3, clo, lane);
+
+    LdsBarrier();  // every wave is done with the previous unit's table and rings
+    const bool table_ok = BuildTableInLds<kChainWaves * 64>(
+        f, reinterpret_cast<uint32_t *>(&lds.ring[0][0]),
+        [tab = &lds.tab[0]](uint32_t slot, const u32x2 &e) { tab[slot] = e; });
+    if (!table_ok && threadIdx.x == 0) atomicOr(a.err, kErrFrequencies);
+    if (!active) continue;
+    u32x2 *const ring = lds.ring[wave];
+    StoreChainChunk(lds.tab, ring, 0, false, lane, c0);
+    StoreChainChunk(lds.tab, ring, kChunkWords, false, lane, c1);
+    WaveSync();
+    const uint32_t ring_at = sizeof(lds.tab) + wave * sizeof(lds.ring[0]);
+    const uint32_t at = k == 0 ? 0u : k == 1 ? 2 * nv : k == 2 ? 6 * nv : 6 * nv + d->palette_bytes;
+    const GPtr<uint8_t> outp = Gbl<uint8_t>(d->symbols + at) + static_cast<size_t>(g) * kGroupSyms;
+    uint32_t used;
+    if (k == 3) {
+      const GPtr<int32_t> sums = Gbl<int32_t>(d->lane_sums);
+      used = DecodeGroupChain<true>(lds, ring, ring_at, rs, lane, x, p, clo, pE, pO, outp,
+                                    Gbl<int32_t>(d->group_sums) + g, sums ? sums + g * kLanesPerGroup : nullptr,
+                                    sums ? sums + LaneSuffixBase(nv) + g * kLanesPerGroup * 8 : nullptr);
+    } else {
+      used = DecodeGroupChain<false>(lds, ring, ring_at, rs, lane, x, p, clo, pE, pO, outp, nullptr, nullptr,
+                                     nullptr);
+    }
+    if (used > p - plo && lane == 0) atomicOr(a.err, kErrStreamOffsets);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1577,7 +1879,10 @@ hipError_t LaunchStage(uint32_t stage, const KernelArgs &args, uint32_t grid,
       if (cfg.ans_auto) {
         // The form travels in the plan (or in args.ans_unit_code for a single image).
         if (!cfg.ans_build_tables || g != 2 || w != kAutoWaves) return hipErrorInvalidValue;
-        hipLaunchKernelGGL(AnsAutoKernel, dim3(grid), dim3(kAutoWaves * 64), 0, stream, args);
+        if (cfg.ans_chain)
+          hipLaunchKernelGGL(AnsChainKernel, dim3(grid), dim3(kChainWaves * 64), 0, stream, args);
+        else
+          hipLaunchKernelGGL(AnsAutoKernel, dim3(grid), dim3(kAutoWaves * 64), 0, stream, args);
         return hipGetLastError();
       }
       if (cfg.ans_pair_short) return hipErrorInvalidValue;  // paired units run in AnsAutoKernel

@@ -224,9 +224,13 @@ typedef struct gst_batch_config {
 } gst_batch_config;
 
 /* rANS work-group forms (gst_batch_config.ans_form, gst_tune_result.ans_form). */
-#define GST_ANS_FORM_AUTO 0   /* chosen at each bind: work-groups of 8 groups of one stream
-                                 while they fit the device in one pass at 6 per CU, else
-                                 PAIRED (one captured graph replays both) */
+#define GST_ANS_FORM_AUTO 0   /* chosen at each bind: a kernel with a wave per group and one
+                                 LDS round trip a step while its work-groups of 4 groups
+                                 fit the device in one pass at 4 per CU; else work-groups
+                                 of 8 groups of one stream while those fit at 6 per CU,
+                                 else PAIRED (gst_batch_launch_graph replays whichever the
+                                 bind chose; launches that a caller captured keep their
+                                 kernel, and each kernel decodes any bound plan) */
 #define GST_ANS_FORM_PAIRED 1 /* a stream's remainder of at most 4 groups shares a
                                  work-group with another stream's: fewer work-groups, at
                                  most 6 per CU */
@@ -271,9 +275,10 @@ typedef struct gst_tune_result {
   float total_ms;
   uint32_t wavelet_fused;            /* 1: wavelet + index scan + DXT1 assembly in one kernel */
   uint32_t ans_form;                 /* GST_ANS_FORM_PAIRED, _PLAIN or _AUTO (8-group units in
-                                        the kernel that also runs PAIRED) of the chosen rANS
-                                        shape when it is 4 waves x 2 groups with tables built
-                                        in LDS; else 0 */
+                                        the kernel that also runs PAIRED, or the kernel with a
+                                        wave per group, which later binds choose again) of the
+                                        chosen rANS shape when it is 4 waves x 2 groups with
+                                        tables built in LDS; else 0 */
 } gst_tune_result;
 /* No reference counterpart.  Times every launch shape of every stage on the bound
  * batch (median of `reps` launches each, 0 = 5) and keeps the fastest per stage:
