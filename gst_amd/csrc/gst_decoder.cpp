@@ -146,7 +146,7 @@ StageConfig DefaultStageConfig(bool rgb) {
   s.ans_groups_per_wave = 2;
   s.wavelet_waves = 1;
   s.fused_waves = rgb ? 0 : 4;
-  s.tile_fused = rgb ? 0 : 1;
+  s.tile_fused = 1;
   s.ans_build_tables = 1;
   s.ans_auto = 1;  // GST_ANS_FORM_AUTO: the caller sets ans_pair_short from AutoPairs
   s.ans_pair_short = 0;
@@ -893,7 +893,7 @@ int gst_batch_create(const gst_batch_config *cfg, gst_batch **out) {
                              ? 0
                              : (cfg->assembly_waves_per_group ? cfg->assembly_waves_per_group : 4);
   b->stage.fused_wide = cfg->assembly_wide ? 1 : 0;
-  b->stage.tile_fused = (cfg->rgb_output || cfg->separate_index_scan || cfg->separate_wavelet) ? 0 : 1;
+  b->stage.tile_fused = (cfg->separate_index_scan || cfg->separate_wavelet) ? 0 : 1;
   b->stage.rgb = cfg->rgb_output ? 1 : 0;
   const uint32_t cus = static_cast<uint32_t>(G().cu_count > 0 ? G().cu_count : 256);
   b->grids[gst::kStageTables] = 4 * cfg->capacity_images;
@@ -1040,9 +1040,9 @@ int gst_batch_autotune(gst_batch *b, gst_stream stream, uint32_t reps, gst_tune_
   res.stage_ms[gst::kStageAns] = best_ans;
   if (best.ans_build_tables) grids[gst::kStageTables] = 0;
 
-  // Wavelet inside the DXT1 assembly (grid), timed before anything overwrites the
+  // Wavelet inside the assembly (grid), timed before anything overwrites the
   // rANS stage's partial sums; the separate shapes follow.
-  const bool try_tile_fused = !best.rgb && !b->cfg.separate_index_scan && !b->cfg.separate_wavelet;
+  const bool try_tile_fused = !b->cfg.separate_index_scan && !b->cfg.separate_wavelet;
   float tile_ms = 1e30f;
   uint32_t tile_grid = 0;
   if (try_tile_fused) {

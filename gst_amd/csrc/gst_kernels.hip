@@ -1637,7 +1637,59 @@ __device__ __forceinline__ uint32_t Rgb565Pair(uint32_t y1, uint32_t y2, uint32_
   return Bits(r << static_cast<s16x2>(11)) | Bits(g << static_cast<s16x2>(5)) | Bits(b);
 }
 
-// Stages 4 and 5 in one kernel: inverse wavelet, index scan and DXT1 assembly of two
+// The four colours of a block (codec/assemble.cl:83-130) as three words, one a channel: byte
+// i of rgb[c] is channel c of colour i.  Both endpoints go through the 16-bit halves of a
+// register (|r|, |b| <= 288 and |g| <= 319 before the shifts, so every 16-bit result is the
+// int32 one); the two between are thirds in C's truncating division: for |s| < 2^15,
+// s * 21846 >> 16 is the floor of s / 3, off from it by under a third of a step, and 1 less
+// than the truncation when s is negative.
+__device__ __forceinline__ uint32_t Third(int32_t s) {
+  return static_cast<uint32_t>((__mul24(s, 21846) >> 16) + static_cast<int32_t>(static_cast<uint32_t>(s) >> 31));
+}
+
+__device__ __forceinline__ uint32_t FourColours(s16x2 ends) {
+  const uint32_t e = Bits(ends);
+  const int32_t a = static_cast<int16_t>(e & 0xFFFFu), b = static_cast<int32_t>(e) >> 16;
+  const uint32_t between = __builtin_amdgcn_perm(Third(a + 2 * b), Third(2 * a + b), 0x0C0C0400u);
+  return __builtin_amdgcn_perm(between, e, 0x05040200u);
+}
+
+__device__ __forceinline__ void BlockColours(uint32_t y1, uint32_t y2, uint32_t co1, uint32_t co2, uint32_t cg1,
+                                             uint32_t cg2, uint32_t k, uint32_t (&rgb)[3]) {
+  const s16x2 y = SBytePair(y1, y2, k), co = SBytePair(co1, co2, k);
+  uint32_t cgw = Bits(SBytePair(cg1, cg2, k));
+  asm volatile("" : "+v"(cgw));  // as in Rgb565Pair
+  const s16x2 cg = AsPair(cgw);
+  const s16x2 t = y - TruncDiv2(cg);
+  const s16x2 g = cg + t;
+  const s16x2 b = TruncDiv2(t - co);
+  const s16x2 r = b + co;
+  rgb[0] = FourColours((r << static_cast<s16x2>(3)) | (r >> static_cast<s16x2>(2)));
+  rgb[1] = FourColours((g << static_cast<s16x2>(2)) | (g >> static_cast<s16x2>(4)));
+  rgb[2] = FourColours((b << static_cast<s16x2>(3)) | (b >> static_cast<s16x2>(2)));
+}
+
+// One texel row of a block, 4 texels of RGB8 in three words: the row's four 2-bit indices
+// become the byte selectors of v_perm, which picks four texels of a channel at once.
+__device__ __forceinline__ void BlockRow(const uint32_t (&rgb)[3], uint32_t word, uint32_t row, uint32_t *out) {
+  const uint32_t idx = (word >> (8 * row)) & 0xFFu, pairs = idx | (idx << 6);
+  const uint32_t sel = (pairs | (pairs << 12)) & 0x03030303u;
+  const uint32_t r = __builtin_amdgcn_perm(0u, rgb[0], sel);
+  const uint32_t g = __builtin_amdgcn_perm(0u, rgb[1], sel);
+  const uint32_t b = __builtin_amdgcn_perm(0u, rgb[2], sel);
+  // r0 g0 b0 r1 | g1 b1 r2 g2 | b2 r3 g3 b3: selector codes 0-3 are bytes of the second
+  // operand, 4-7 of the first.
+  const uint32_t rg01 = __builtin_amdgcn_perm(g, r, 0x05010400u);  // r0 g0 r1 g1
+  const uint32_t rg23 = __builtin_amdgcn_perm(g, r, 0x07030602u);  // r2 g2 r3 g3
+  out[0] = __builtin_amdgcn_perm(b, rg01, 0x02040100u);
+  out[1] = __builtin_amdgcn_perm(__builtin_amdgcn_perm(b, rg01, 0x0C0C0503u), rg23, 0x01000504u);
+  out[2] = __builtin_amdgcn_perm(b, rg23, 0x07030206u);
+}
+
+// 16 bytes to an address that is a multiple of 4 (RGB8 output has no wider guarantee).
+typedef uint32_t u32x4Words __attribute__((ext_vector_type(4), aligned(4)));
+
+// Stages 4 and 5 in one kernel: inverse wavelet, index scan and assembly of two
 // tile positions per work-group, so the int8 planes never leave LDS (the planes
 // buffer's write and read, 12 bytes a block, are the traffic this saves).
 //
@@ -1655,7 +1707,15 @@ __device__ __forceinline__ uint32_t Rgb565Pair(uint32_t y1, uint32_t y2, uint32_
 // per-row reduction) plus the sum before the row within its group.
 constexpr uint32_t kTileFusedWaves = 3;
 
+// kRgb writes RGB8 instead of DXT1 blocks: the same planes, indices and palette words, a
+// lane's four blocks being 48 bytes of four texel rows each.  Bound by its writes (48 bytes
+// a block of 55): 32 2048x2048 textures in 115.8 us (4.0 TB/s), where the index scan, the
+// wavelet and AssembleRgbKernel took 17.3 + 38.3 + 370.1 us, the last one a texel's byte
+// at a time in the vector unit; six mixed textures (5.2 Mtexel) 14.4 us against 4.9 + 6.9
+// + 23.8.
+//
 // At most 96 VGPRs: 5 waves per SIMD, about what the 25 KiB of LDS allows.
+template <bool kRgb>
 __global__ __launch_bounds__(kTileFusedWaves * 64, 5) void WaveletAssembleKernel(KernelArgs a) {
   __shared__ uint32_t lds[kTileFusedWaves][2][kTileDim * kLdsStride];
   constexpr uint32_t kWaveLdsBytes = sizeof(lds[0]);
@@ -1781,15 +1841,33 @@ __global__ __launch_bounds__(kTileFusedWaves * 64, 5) void WaveletAssembleKernel
       for (uint32_t p = 0; p < 6; ++p)
         pw[p] = *reinterpret_cast<const uint32_t *>(tiles + (p >> 1) * kWaveLdsBytes +
                                                     ((p & 1) * 2 + P) * kTileSyms + y * kTileDim + xb);
-      uint32_t o[8];
+      if constexpr (kRgb) {
+        uint32_t rgb[4][3];
 #pragma unroll
-      for (uint32_t k = 0; k < 4; ++k) {
-        o[2 * k] = Rgb565Pair(pw[0], pw[1], pw[2], pw[4], pw[3], pw[5], k);
-        o[2 * k + 1] = word[i][k];
+        for (uint32_t k = 0; k < 4; ++k) BlockColours(pw[0], pw[1], pw[2], pw[4], pw[3], pw[5], k, rgb[k]);
+        const uint32_t by = (P ? ty1 : ty0) * kTileDim + y, x4 = (P ? tx1 : tx0) * kTileDim + xb;
+        GPtr<uint8_t> row = d.out + 3 * (static_cast<size_t>(d.width) * 4 * by + 4 * x4);
+#pragma unroll
+        for (uint32_t t = 0; t < 4; ++t) {
+          uint32_t o[12];
+#pragma unroll
+          for (uint32_t k = 0; k < 4; ++k) BlockRow(rgb[k], word[i][k], t, o + 3 * k);
+          const GPtr<u32x4Words> dst = (GPtr<u32x4Words>)row;
+#pragma unroll
+          for (uint32_t k = 0; k < 3; ++k) dst[k] = u32x4Words{o[4 * k], o[4 * k + 1], o[4 * k + 2], o[4 * k + 3]};
+          row += 3 * static_cast<size_t>(d.width);
+        }
+      } else {
+        uint32_t o[8];
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) {
+          o[2 * k] = Rgb565Pair(pw[0], pw[1], pw[2], pw[4], pw[3], pw[5], k);
+          o[2 * k + 1] = word[i][k];
+        }
+        const GPtr<uint4> dst = (GPtr<uint4>)(d.out + 8 * static_cast<size_t>(blk[i]));
+        dst[0] = make_uint4(o[0], o[1], o[2], o[3]);
+        dst[1] = make_uint4(o[4], o[5], o[6], o[7]);
       }
-      const GPtr<uint4> dst = (GPtr<uint4>)(d.out + 8 * static_cast<size_t>(blk[i]));
-      dst[0] = make_uint4(o[0], o[1], o[2], o[3]);
-      dst[1] = make_uint4(o[4], o[5], o[6], o[7]);
     }
     if (bad) atomicOr(a.err, kErrPaletteIndex);
     LdsBarrier();  // the next unit's transposes reuse the tiles' space
@@ -1919,8 +1997,10 @@ hipError_t LaunchStage(uint32_t stage, const KernelArgs &args, uint32_t grid,
       return hipGetLastError();
     case kStageAssemble:
       if (cfg.tile_fused) {
-        if (cfg.rgb) return hipErrorInvalidValue;  // the fused kernel writes DXT1 only
-        hipLaunchKernelGGL(WaveletAssembleKernel, dim3(grid), dim3(kTileFusedWaves * 64), 0, stream, args);
+        if (cfg.rgb)
+          hipLaunchKernelGGL(WaveletAssembleKernel<true>, dim3(grid), dim3(kTileFusedWaves * 64), 0, stream, args);
+        else
+          hipLaunchKernelGGL(WaveletAssembleKernel<false>, dim3(grid), dim3(kTileFusedWaves * 64), 0, stream, args);
       } else if (cfg.rgb) {
         if (cfg.fused_waves) return hipErrorInvalidValue;  // the fused scan writes DXT1 only
         hipLaunchKernelGGL(AssembleRgbKernel, dim3(grid), dim3(256), 0, stream, args);
