@@ -145,7 +145,6 @@ int gst_ans_decode(const gst_ans_decoder *d, const uint32_t *states, uint32_t nu
   hipError_t e = hipMallocAsync(reinterpret_cast<void **>(&d_data), total, d->stream);
   if (e == hipSuccess) e = hipMallocAsync(reinterpret_cast<void **>(&d_out), out_bytes, d->stream);
   if (e == hipSuccess) e = hipMemcpyAsync(d_data, packed.data(), total, hipMemcpyHostToDevice, d->stream);
-  if (e == hipSuccess) e = hipMemsetAsync(d_out, 0, out_bytes, d->stream);
   if (e == hipSuccess) e = hipMemsetAsync(d->d_err, 0, sizeof(uint32_t), d->stream);
   if (e == hipSuccess)
     e = gst::LaunchAnsGroups(d->d_tables, d_data, static_cast<uint32_t>(total), n_data, lanes, d_out, d->d_err,

@@ -927,23 +927,25 @@ __device__ __forceinline__ u32x2 ChainStep(const uint32_t &y, uint32_t thr, uint
   return e;
 }
 
-// One group: lanes 0..31 decode streams 31..0 from state y, their words below word p
-// (chunk top first, chunks below clo read zeros), with E and O the chunks top - 2 and
-// top - 3 in flight.  Returns how many words the group consumed.
+// One group of n <= 32 streams: lanes 0 .. n - 1 decode streams n - 1 .. 0 from state y,
+// their words below word p (chunk top first, chunks below clo read zeros), with E and O
+// the chunks top - 2 and top - 3 in flight.  Leaves the state before its last
+// renormalisation in y and the ring address of the next word in q; returns how many words
+// the group consumed before that renormalisation.
 template <bool kSum>
 __device__ __forceinline__ uint32_t DecodeGroupChain(const AnsChainLds &lds, u32x2 *ring, uint32_t ring_at,
-                                                     __amdgpu_buffer_rsrc_t rs, uint32_t lane, uint32_t y,
-                                                     uint32_t p, uint32_t clo, u32x2 pE, u32x2 pO,
-                                                     GPtr<uint8_t> outp, GPtr<int32_t> group_sum,
+                                                     __amdgpu_buffer_rsrc_t rs, uint32_t lane, uint32_t n,
+                                                     uint32_t &y, uint32_t &q, uint32_t p, uint32_t clo, u32x2 pE,
+                                                     u32x2 pO, GPtr<uint8_t> outp, GPtr<int32_t> group_sum,
                                                      GPtr<int32_t> lane_sum, GPtr<int32_t> lane_suffix) {
-  const bool active = lane < kLanesPerGroup;
-  const uint32_t j = 31 - (lane & 31);
+  const bool active = lane < n;
+  const uint32_t j = active ? n - 1 - lane : 0u;
   const uint32_t full = active ? kStateL : 0u;
   uint32_t thr = 0;  // a group's first step never renormalises: its states come as stored
   asm volatile("" : "+v"(thr));
   uint32_t top = p ? (p - 1) / kChunkWords : 0u;
   const uint32_t q0 = ring_at + 8 * (kChunkWords - 1 - ((p - 1) & (kChunkWords - 1)));
-  uint32_t q = Uniform(q0);
+  q = Uniform(q0);
   const uint32_t end0 = ring_at + 8 * kChunkWords, end1 = ring_at + 16 * kChunkWords;
   uint32_t limit = end0, wraps = 0;
   int32_t sum = 0;
@@ -1014,17 +1016,16 @@ __device__ __forceinline__ uint32_t DecodeGroupChain(const AnsChainLds &lds, u32
     }
   }
   if (kSum) {
-    // Inclusive prefix over the streams, which run down the lanes.
+    // Inclusive prefix over the 32 streams, which run down the lanes.
     int32_t incl = sum;
 #pragma unroll
     for (uint32_t off = 1; off < 32; off <<= 1) {
-      const int32_t n = __shfl_down(incl, off, 32);
-      if (j >= off) incl += n;
+      const int32_t n_below = __shfl_down(incl, off, 32);
+      if (j >= off) incl += n_below;
     }
     if (active && lane_sum) lane_sum[j] = incl;
     if (lane == 0) *group_sum = incl;
   }
-  q += 8 * static_cast<uint32_t>(__popc(static_cast<uint32_t>(__builtin_amdgcn_uicmp(y, full, 36 /* ULT */))));
   return (q + 16 * kChunkWords * wraps - q0) / 8;
 }
 
@@ -1075,16 +1076,17 @@ __global__ __launch_bounds__(kChainWaves * 64, 4) void AnsChainKernel(KernelArgs
     const uint32_t ring_at = sizeof(lds.tab) + wave * sizeof(lds.ring[0]);
     const uint32_t at = k == 0 ? 0u : k == 1 ? 2 * nv : k == 2 ? 6 * nv : 6 * nv + d->palette_bytes;
     const GPtr<uint8_t> outp = Gbl<uint8_t>(d->symbols + at) + static_cast<size_t>(g) * kGroupSyms;
-    uint32_t used;
+    uint32_t y = x, q, used;
     if (k == 3) {
       const GPtr<int32_t> sums = Gbl<int32_t>(d->lane_sums);
-      used = DecodeGroupChain<true>(lds, ring, ring_at, rs, lane, x, p, clo, pE, pO, outp,
+      used = DecodeGroupChain<true>(lds, ring, ring_at, rs, lane, kLanesPerGroup, y, q, p, clo, pE, pO, outp,
                                     Gbl<int32_t>(d->group_sums) + g, sums ? sums + g * kLanesPerGroup : nullptr,
                                     sums ? sums + LaneSuffixBase(nv) + g * kLanesPerGroup * 8 : nullptr);
     } else {
-      used = DecodeGroupChain<false>(lds, ring, ring_at, rs, lane, x, p, clo, pE, pO, outp, nullptr, nullptr,
-                                     nullptr);
+      used = DecodeGroupChain<false>(lds, ring, ring_at, rs, lane, kLanesPerGroup, y, q, p, clo, pE, pO, outp,
+                                     nullptr, nullptr, nullptr);
     }
+    used += Popc64(__builtin_amdgcn_ballot_w64(lane < kLanesPerGroup && y < kStateL));  // the last renormalisation's
     if (used > p - plo && lane == 0) atomicOr(a.err, kErrStreamOffsets);
   }
 }
@@ -1097,55 +1099,62 @@ __global__ __launch_bounds__(kChainWaves * 64, 4) void AnsChainKernel(KernelArgs
 // step as the texture path: slot = x & 2047, x = (x >> 11) f + slot - cum, and lanes
 // with x < 2^15 take the next words in lane order.
 //
-// One wave per group; lanes >= n sit out of the ballot.  The table and the group's
-// last 8192 words (a group of 32 streams x 256 steps reads at most that many) are
-// copied to LDS first, so the serial chain reads only LDS; every global read is
-// range-checked through a buffer resource.  Stream j of group g leaves its 256
-// symbols at out[(g n + j) 256 ..], the last decoded first, 4 bytes per store.  A
-// malformed end offset, or a group that does not end in the encoder's initial state
-// 2^15, raises GST_DEVERR_STREAM_OFFSETS.
-constexpr uint32_t kGroupWindow = kLanesPerGroup * kSymsPerLane;  // 8192 words
-
-__global__ __launch_bounds__(64) void AnsGroupsKernel(const uint32_t *table, const uint8_t *data,
-                                                      uint32_t data_len, uint32_t n, uint8_t *out,
-                                                      uint32_t *err) {
-  __shared__ uint32_t tab[kTableSize];
-  __shared__ uint16_t words[kGroupWindow];
-  const uint32_t lane = threadIdx.x, g = blockIdx.x;
-  const GPtr<const uint32_t> t = Gbl<const uint32_t>(table);
-  for (uint32_t i = lane; i < kTableSize; i += 64) tab[i] = t[i];
+// A wave per group, four to a work-group, decoding as AnsChainKernel does from the given
+// table; lanes >= n never renormalise.  Words come from anywhere below the group's states
+// (a pointer that runs below the data reads zeros); every global read is range-checked
+// through a buffer resource.  Stream j of group g leaves its 256 symbols at
+// out[(g n + j) 256 ..], the last decoded first.  A malformed end offset, or a group that
+// does not end in the encoder's initial state 2^15, raises GST_DEVERR_STREAM_OFFSETS; the
+// output of a group with a malformed end offset is zeros.
+//
+// 24 groups of 32 streams: 16.3 us, where a wave per group with two LDS round trips a step
+// and the words copied to LDS two bytes a lane took 87 us.
+__global__ __launch_bounds__(kChainWaves * 64, 4) void AnsGroupsKernel(const uint32_t *table, const uint8_t *data,
+                                                                       uint32_t data_len, uint32_t groups,
+                                                                       uint32_t n, uint8_t *out, uint32_t *err) {
+  __shared__ __align__(16) AnsChainLds lds;
+  const uint32_t lane = threadIdx.x & 63, wave = Uniform(threadIdx.x >> 6);
+  const uint32_t g = blockIdx.x * kChainWaves + wave;
   const __amdgpu_buffer_rsrc_t rs = MakeRsrc(data, data_len);
-  const uint32_t end = __builtin_amdgcn_raw_buffer_load_b32(rs, static_cast<int>(4 * g), 0, 0);
-  const bool ok = (end & 3) == 0 && end <= data_len && end >= 4 * n;
-  const uint32_t p0 = ok ? (end - 4 * n) / 2 : 0u;
-  const uint32_t wbase = p0 > kGroupWindow ? p0 - kGroupWindow : 0u;
-  for (uint32_t i = lane; i < kGroupWindow; i += 64) {
-    const uint32_t w = wbase + i;
-    words[i] = w < p0 ? static_cast<uint16_t>(__builtin_amdgcn_raw_buffer_load_b16(rs, static_cast<int>(2 * w), 0, 0))
-                      : static_cast<uint16_t>(0);
+  const uint32_t end = Uniform(__builtin_amdgcn_raw_buffer_load_b32(rs, static_cast<int>(4 * g), 0, 0));
+  // The packed table, 8 entries a thread.
+  const GPtr<const uint4> t = Gbl<const uint4>(table);
+  const uint4 t0 = t[2 * threadIdx.x], t1 = t[2 * threadIdx.x + 1];
+  const bool in = g < groups;
+  const bool ok = in && (end & 3) == 0 && end <= data_len && end >= 4 * n;
+  const uint32_t p = ok ? (end - 4 * n) / 2 : 0u;
+  const uint32_t top = p ? (p - 1) / kChunkWords : 0u;
+  const uint32_t x = __builtin_amdgcn_raw_buffer_load_b32(
+      rs, static_cast<int>(ok && lane < n ? end - 4 * (lane + 1) : 0u), 0, 0);  // stream n - 1 - lane
+  const u32x2 c0 = LoadChunk(rs, top, 0, lane), c1 = LoadChunk(rs, top - 1, 0, lane);
+  const u32x2 pE = LoadChunk(rs, top - 2, 0, lane), pO = LoadChunk(rs, top - 3, 0, lane);
+  const uint32_t packed[8] = {t0.x, t0.y, t0.z, t0.w, t1.x, t1.y, t1.z, t1.w};
+#pragma unroll
+  for (uint32_t i = 0; i < 8; ++i)
+    lds.tab[8 * threadIdx.x + i] = u32x2{packed[i] & 0xFF000FFFu, (packed[i] >> 12) & (kTableSize - 1)};
+  LdsBarrier();
+  if (!in) return;
+  GPtr<uint8_t> dst = Gbl<uint8_t>(out) + static_cast<size_t>(g) * n * kSymsPerLane;
+  if (!ok) {
+    for (uint32_t i = 4 * lane; i < n * kSymsPerLane; i += 256) *(GPtr<uint32_t>)(dst + i) = 0;
+    if (lane == 0) atomicOr(err, kErrStreamOffsets);
+    return;
   }
-  const bool active = ok && lane < n;
-  uint32_t x = __builtin_amdgcn_raw_buffer_load_b32(rs, static_cast<int>(active ? end - 4 * n + 4 * lane : 0u), 0, 0);
-  x = active ? x : 0u;
-  __syncthreads();
-  uint32_t p = p0, acc = 0;
-  const GPtr<uint32_t> dst = Gbl<uint32_t>(reinterpret_cast<uint32_t *>(out + (static_cast<size_t>(g) * n + lane) *
-                                                                                 kSymsPerLane));
-  for (uint32_t i = 0; i < kSymsPerLane; ++i) {
-    const uint32_t e = tab[x & (kTableSize - 1)];
-    x = __umul24(x >> kTableLog, e & 0xFFFu) + __builtin_amdgcn_ubfe(e, 12, 11);
-    const bool need = active && x < kStateL;
-    const uint64_t m = __builtin_amdgcn_ballot_w64(need);
-    const uint32_t total = static_cast<uint32_t>(__popcll(m));
-    const uint32_t rank = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(m >> 32),
-                                                    __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), 0u));
-    if (need) x = (x << 16) | words[(p - total + rank - wbase) & (kGroupWindow - 1)];
-    p -= total;
-    acc = (acc << 8) | (e >> 24);
-    if ((i & 3) == 3 && active) dst[(kSymsPerLane - 1 - i) / 4] = acc;
-  }
-  const bool bad = (lane == 0 && !ok) || (active && x != kStateL);
-  if (__builtin_amdgcn_ballot_w64(bad) != 0 && lane == 0) atomicOr(err, kErrStreamOffsets);
+  u32x2 *const ring = lds.ring[wave];
+  StoreChainChunk(lds.tab, ring, 0, false, lane, c0);
+  StoreChainChunk(lds.tab, ring, kChunkWords, false, lane, c1);
+  WaveSync();
+  const bool active = lane < n;
+  uint32_t y = active ? x : 0u, q, mul, unused = 0;
+  DecodeGroupChain<false>(lds, ring, sizeof(lds.tab) + wave * sizeof(lds.ring[0]), rs, lane, n, y, q, p, 0, pE, pO,
+                          dst, nullptr, nullptr, nullptr);
+  // The final state is 2^15: y itself, or y = 0 renormalised with the word 2^15, which its
+  // ring entry tells from every other word (slot 0, 16 above it: an rANS step is one to one).
+  const u32x2 e = ChainStep<false>(y, active ? kStateL : 0u, q, mul, 0u, unused, 0u);
+  const uint32_t f = lds.tab[0].x & 0xFFFFFFu;
+  const bool last = y >= kStateL ? y == kStateL
+                                 : y == 0 && e.x == ((f << 5) | (lds.tab[0].x & 0xFF000000u)) && e.y == 16 * f;
+  if (__builtin_amdgcn_ballot_w64(active && !last) != 0 && lane == 0) atomicOr(err, kErrStreamOffsets);
 }
 
 // ---------------------------------------------------------------------------
@@ -2146,7 +2155,8 @@ hipError_t LaunchAnsGroups(const uint32_t *table, const uint8_t *data, uint32_t 
                            uint32_t n, uint8_t *out, uint32_t *err, hipStream_t stream) {
   if (groups == 0) return hipSuccess;
   if (n == 0 || n > kLanesPerGroup) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(AnsGroupsKernel, dim3(groups), dim3(64), 0, stream, table, data, data_len, n, out, err);
+  hipLaunchKernelGGL(AnsGroupsKernel, dim3((groups + kChainWaves - 1) / kChainWaves), dim3(kChainWaves * 64), 0,
+                     stream, table, data, data_len, groups, n, out, err);
   return hipGetLastError();
 }
 

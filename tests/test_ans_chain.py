@@ -1,6 +1,7 @@
 """The rANS kernel with a wave per group (the default for images and batches of few groups)
 on streams at the edges of its ring: no renormalisation word at all, 16 words a step, and 22
-a step (one more than a chunk every 12 steps), for group counts of every remainder."""
+a step (one more than a chunk every 12 steps), for group counts of every remainder; and the
+stand-alone groups, which decode the same way."""
 import struct
 
 import numpy as np
@@ -12,9 +13,8 @@ from oracle import gst_oracle as go
 pytestmark = pytest.mark.gpu
 
 
-def _stream(norm, syms):
-    """One .gtc stream: u32 end offsets, then per group its words (padded in front to 4
-    bytes) and 32 final states.  `syms`: groups x 32 streams x 256."""
+def _encode(norm, syms):
+    """rANS over groups x streams x 256 symbols: (words of each group, final states)."""
     f, cum = norm[syms], (np.cumsum(norm) - norm)[syms]
     x = np.full(syms.shape[:2], 1 << 15, np.int64)
     words = [[] for _ in syms]
@@ -24,29 +24,36 @@ def _stream(norm, syms):
             words[g].append(x[g][over[g]] & 0xFFFF)
         x = np.where(over, x >> 16, x)
         x = (x // f[:, :, i] << 11) + x % f[:, :, i] + cum[:, :, i]
+    return [np.concatenate(w) if w else np.zeros(0, np.int64) for w in words], x
+
+
+def _stream(norm, syms):
+    """One .gtc stream: u32 end offsets, then per group its words (padded in front to 4
+    bytes) and 32 final states."""
+    words, x = _encode(norm, syms)
     parts = []
     for g, w in enumerate(words):
-        w = np.concatenate(w) if w else np.zeros(0, np.int64)
         parts.append(np.concatenate([np.zeros(len(w) % 2, np.int64), w]).astype("<u2").tobytes() +
                      x[g].astype("<u4").tobytes())
     ends = 4 * len(parts) + np.cumsum([len(p) for p in parts])
     return ends.astype("<u4").tobytes() + b"".join(parts)
 
 
+def _symbols(kind, rng, shape):
+    if kind == "constant":
+        norm = np.zeros(256, np.int64)
+        norm[77] = 2048
+        return norm, np.full(shape, 77)
+    if kind == "uniform":
+        return np.full(256, 8, np.int64), rng.integers(0, 256, shape)
+    return np.array([1793] + [1] * 255, np.int64), rng.integers(1, 256, shape)  # rare: 11 bits a symbol
+
+
 def _texture(width, height, palette_groups, kind, seed):
     rng = np.random.default_rng(seed)
     groups = width * height // 131072
 
-    def draw(n):
-        if kind == "constant":
-            norm = np.zeros(256, np.int64)
-            norm[77] = 2048
-            return norm, np.full((n, 32, 256), 77)
-        if kind == "uniform":
-            return np.full(256, 8, np.int64), rng.integers(0, 256, (n, 32, 256))
-        return (np.array([1793] + [1] * 255, np.int64),
-                rng.integers(1, 256, (n, 32, 256)))  # rare: every symbol costs 11 bits
-    streams = [draw(2 * groups), draw(4 * groups), draw(palette_groups)]
+    streams = [_symbols(kind, rng, (n, 32, 256)) for n in (2 * groups, 4 * groups, palette_groups)]
     if kind == "constant":
         norm = np.zeros(256, np.int64)
         norm[128] = 2048
@@ -86,3 +93,17 @@ def test_ring_edges_match_oracle(device, kind):
             assert b.error_bits(device.stream) == 0
         finally:
             b.close()
+
+
+@pytest.mark.parametrize("kind", ["uniform", "rare"])
+@pytest.mark.parametrize("groups,streams", [(1, 1), (3, 2), (4, 31), (5, 32), (9, 24)])
+def test_stand_alone_groups(device, kind, groups, streams):
+    norm, syms = _symbols(kind, np.random.default_rng(groups), (groups, streams, 256))
+    words, x = _encode(norm, syms)
+    data = [w.astype("<u2").tobytes() for w in words]
+    d = gst_amd.AnsDecoder(norm.tolist(), streams)
+    try:
+        expected = [s.astype(np.uint8).tobytes() for s in syms.reshape(-1, 256)]
+        assert d.decode(x.reshape(-1).tolist(), data) == expected
+    finally:
+        d.close()
