@@ -128,6 +128,7 @@ void FillDesc(const gst_header &h, const uint8_t *freqs, const uint8_t *streams,
   }
   d->table_base = table_base;
   d->rgb = rgb ? 1 : 0;
+  d->tile_mul = gst::TileMul(d->bx / gst::kTileDim);
   d->freqs = freqs;
   d->symbols = scratch + c.symbols;
   d->planes = reinterpret_cast<int8_t *>(scratch + c.planes);

@@ -47,6 +47,7 @@ struct ImageDesc {
   uint32_t stream_len[4];
   uint32_t table_base;   // index of the image's first of 4 tables
   uint32_t rgb;          // 1: RGB8 output
+  uint32_t tile_mul;     // TileRowOf's multiplier for bx / 32 tiles a row
   const uint8_t *freqs;  // 4 x 256 little-endian u16
   const uint8_t *streams[4];
   uint8_t *symbols;
@@ -56,6 +57,16 @@ struct ImageDesc {
   int32_t *lane_sums;    // index-stream partial sums (layout at LaneSuffixBase), or null
   uint8_t *out;
 };
+
+// t / tiles_x for a tile t < 2^14 of an image of tiles_x < 2^14 tiles a row: the high word of
+// t times floor(2^32 / tiles_x) + 1, which exceeds 2^32 / tiles_x by at most 1, an error below
+// t / 2^32 < 1 / tiles_x in the quotient.  0 stands for one tile a row.
+inline uint32_t TileMul(uint32_t tiles_x) {
+  return tiles_x == 1 ? 0u : static_cast<uint32_t>((1ull << 32) / tiles_x) + 1;
+}
+__host__ __device__ inline uint32_t TileRowOf(uint32_t t, uint32_t tile_mul) {
+  return tile_mul == 0 ? t : static_cast<uint32_t>((static_cast<uint64_t>(t) * tile_mul) >> 32);
+}
 
 // Partial sums of (diff - 128) over the index stream that the rANS stage leaves in
 // lane_sums, so a palette index can start at any 32-block boundary: int32 entries

@@ -55,6 +55,25 @@ struct Located {
   bool valid;  // false: u is past the stage's last unit
 };
 
+// Locate among the up to 256 prefix entries a wave holds, entry lane + 64 k in v[k]
+// (padding past the plan's).
+constexpr uint32_t kPrefixInRegs = 256;
+__device__ __forceinline__ Located LocateIn(const uint32_t (&v)[4], uint32_t u) {
+  uint32_t cnt = 0;
+#pragma unroll
+  for (uint32_t k = 0; k < 4; ++k) cnt += Popc64(__builtin_amdgcn_ballot_w64(v[k] <= u));
+  const uint32_t lo = cnt - 1;  // prefix[0] = 0 <= u
+  // Reads of a lane and scalar selects: no branches over the four registers.
+  uint32_t at[4], after[4];
+#pragma unroll
+  for (uint32_t k = 0; k < 4; ++k) {
+    at[k] = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v[k]), static_cast<int>(lo & 63)));
+    after[k] = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v[k]), static_cast<int>(cnt & 63)));
+  }
+  const uint32_t next = cnt < kPrefixInRegs ? Pick4(after, cnt >> 6) : kPrefixPad;
+  return {lo, u - Pick4(at, lo >> 6), next != kPrefixPad};
+}
+
 // Work unit u of `stage` as (image, unit within the image).  Called by a whole wave
 // with u uniform.  The image is the last index i with prefix[i] <= u, found by
 // counting over a ballot instead of a dependent binary search: for plans of up to 255
@@ -70,23 +89,11 @@ __device__ __forceinline__ Located Locate(const KernelArgs &a, uint32_t stage, u
       Gbl<const uint32_t>(reinterpret_cast<const uint8_t *>(a.plan) + PlanPrefixOffset(a.plan_cap, stage));
   const uint32_t lane = __lane_id();
   uint32_t lo, start, next = kPrefixPad;
-  if (len <= 256) {
+  if (len <= kPrefixInRegs) {
     uint32_t v[4];
 #pragma unroll
     for (uint32_t k = 0; k < 4; ++k) v[k] = lane + 64 * k < len ? pre[lane + 64 * k] : kPrefixPad;
-    uint32_t cnt = 0;
-#pragma unroll
-    for (uint32_t k = 0; k < 4; ++k) cnt += Popc64(__builtin_amdgcn_ballot_w64(v[k] <= u));
-    lo = cnt - 1;  // prefix[0] = 0 <= u
-    // Four reads of a lane and scalar selects: no branches over the four registers.
-    uint32_t at[4], after[4];
-#pragma unroll
-    for (uint32_t k = 0; k < 4; ++k) {
-      at[k] = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v[k]), static_cast<int>(lo & 63)));
-      after[k] = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v[k]), static_cast<int>(cnt & 63)));
-    }
-    start = Pick4(at, lo >> 6);
-    next = cnt < 256 ? Pick4(after, cnt >> 6) : kPrefixPad;  // entries past the plan's are padding
+    return LocateIn(v, u);
   } else {
     lo = 0;
     uint32_t m = len;  // the answer lies in [lo, lo + m)
@@ -171,11 +178,23 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t MakeRsrc(const void *base, uin
                                            kBufferRsrcWord3);
 }
 
-template <typename T>
-__device__ __forceinline__ T WaveSumWidth32(T v) {
-#pragma unroll
-  for (int off = 16; off > 0; off >>= 1) v += __shfl_xor(v, off, 32);
-  return v;
+// Inclusive prefix sum over a wave in six DPP adds (row shifts, then row broadcasts): no LDS
+// round trip, where __shfl_up is a ds_bpermute each.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t DppAdd(uint32_t v) {
+  return v + static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), CTRL, ROWS, 0xF, false));
+}
+__device__ __forceinline__ uint32_t WaveInclusiveSum(uint32_t v) {
+  v = DppAdd<0x111, 0xF>(v);  // row_shr:1
+  v = DppAdd<0x112, 0xF>(v);  // row_shr:2
+  v = DppAdd<0x114, 0xF>(v);  // row_shr:4
+  v = DppAdd<0x118, 0xF>(v);  // row_shr:8
+  v = DppAdd<0x142, 0xA>(v);  // row_bcast:15 into rows 1 and 3
+  return DppAdd<0x143, 0xC>(v);  // row_bcast:31 into rows 2 and 3
+}
+
+__device__ __forceinline__ uint32_t WaveTotal(uint32_t v) {
+  return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(WaveInclusiveSum(v)), 63));
 }
 
 // ---------------------------------------------------------------------------
@@ -571,21 +590,6 @@ __device__ __forceinline__ const uint8_t *Uniform(const uint8_t *p) {
 // Work-group barrier that orders LDS only: waits for the wave's own LDS operations,
 // not for its global loads in flight (a __syncthreads fence would wait for those too).
 __device__ __forceinline__ void LdsBarrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
-// Inclusive prefix sum over a wave in six DPP adds (row shifts, then row broadcasts): no LDS
-// round trip, where __shfl_up is a ds_bpermute each.
-template <int CTRL, int ROWS>
-__device__ __forceinline__ uint32_t DppAdd(uint32_t v) {
-  return v + static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), CTRL, ROWS, 0xF, false));
-}
-__device__ __forceinline__ uint32_t WaveInclusiveSum(uint32_t v) {
-  v = DppAdd<0x111, 0xF>(v);  // row_shr:1
-  v = DppAdd<0x112, 0xF>(v);  // row_shr:2
-  v = DppAdd<0x114, 0xF>(v);  // row_shr:4
-  v = DppAdd<0x118, 0xF>(v);  // row_shr:8
-  v = DppAdd<0x142, 0xA>(v);  // row_bcast:15 into rows 1 and 3
-  return DppAdd<0x143, 0xC>(v);  // row_bcast:31 into rows 2 and 3
-}
 
 // The work of BuildTableKernel for one table, straight into a rANS kernel's LDS (256 <=
 // THREADS): thread t < 256 brings frequency f[t].  The slot -> symbol map is a count, not a
@@ -1487,7 +1491,8 @@ __device__ __forceinline__ int32_t WaveSum64(int32_t v) {
 
 // Sum of (diff - 128) over the blocks of b's rANS group that come before block b
 // (b a multiple of 32): the lane's inclusive prefix less the lane's suffix from b.
-__device__ __forceinline__ int32_t GroupLocalPrefix(const DevDesc &d, uint32_t b) {
+template <typename Desc>
+__device__ __forceinline__ int32_t GroupLocalPrefix(const Desc &d, uint32_t b) {
   const uint32_t lane_ix = b / kSymsPerLane;  // group * 32 + lane
   const uint32_t k = (b % kSymsPerLane) / kRowBlocks;
   return d.lane_sums[lane_ix] - d.lane_sums[LaneSuffixBase(d.nv) + lane_ix * 8 + k];
@@ -1716,6 +1721,38 @@ typedef uint32_t u32x4Words __attribute__((ext_vector_type(4), aligned(4)));
 // per-row reduction) plus the sum before the row within its group.
 constexpr uint32_t kTileFusedWaves = 3;
 
+// Tile positions t0 and t0 + 1 of an image: what the fused kernel needs of its descriptor,
+// the first position's tile row and column, and the index-stream groups its rows touch,
+// g_min .. g_min + g_span.
+struct TilePair {
+  uint32_t nv, bx, tiles_x, palette_bytes;
+  uint32_t t0, ty0, tx0, g_min, g_span;
+  GPtr<uint8_t> symbols;
+  GPtr<int32_t> group_sums;
+  GPtr<int32_t> lane_sums;
+  GPtr<uint8_t> out;
+};
+
+__device__ __forceinline__ TilePair PairAt(CPtr<ImageDesc> d, uint32_t t0) {
+  TilePair p;
+  p.nv = d->nv;
+  p.bx = d->bx;
+  p.tiles_x = p.bx / kTileDim;
+  p.palette_bytes = d->palette_bytes;
+  p.t0 = t0;
+  p.ty0 = TileRowOf(t0, d->tile_mul);
+  p.tx0 = t0 - p.ty0 * p.tiles_x;
+  const bool wraps = p.tx0 + 1 == p.tiles_x;
+  const uint32_t ty1 = wraps ? p.ty0 + 1 : p.ty0, tx1 = wraps ? 0 : p.tx0 + 1;
+  p.g_min = (p.ty0 * kTileDim * p.bx + p.tx0 * kTileDim) / kGroupSyms;
+  p.g_span = ((ty1 * kTileDim + kTileDim - 1) * p.bx + tx1 * kTileDim) / kGroupSyms - p.g_min;
+  p.symbols = Gbl<uint8_t>(d->symbols);
+  p.group_sums = Gbl<int32_t>(d->group_sums);
+  p.lane_sums = Gbl<int32_t>(d->lane_sums);
+  p.out = Gbl<uint8_t>(d->out);
+  return p;
+}
+
 // kRgb writes RGB8 instead of DXT1 blocks: the same planes, indices and palette words, a
 // lane's four blocks being 48 bytes of four texel rows each.  Bound by its writes (48 bytes
 // a block of 55): 32 2048x2048 textures in 115.8 us (4.0 TB/s), where the index scan, the
@@ -1723,50 +1760,76 @@ constexpr uint32_t kTileFusedWaves = 3;
 // at a time in the vector unit; six mixed textures (5.2 Mtexel) 14.4 us against 4.9 + 6.9
 // + 23.8.
 //
-// At most 96 VGPRs: 5 waves per SIMD, about what the 25 KiB of LDS allows.
+// A unit starts with three dependent trips to memory (plan, descriptor, rows and sums), two
+// thirds of the transform's own time.  So the plan's prefix is in LDS, the next unit's
+// descriptor and loads go out while this one is assembled, where the transform's registers
+// are free, and all sums over lanes are DPP: the batch of 128 textures 55.1 -> 53.0 us, 24
+// textures 15.6 -> 14.4, one unit alone 15,700 -> 12,400 cycles.
+//
+// At most 96 VGPRs: 5 waves per SIMD, about what the 26 KiB of LDS allows.
 template <bool kRgb>
 __global__ __launch_bounds__(kTileFusedWaves * 64, 5) void WaveletAssembleKernel(KernelArgs a) {
   __shared__ uint32_t lds[kTileFusedWaves][2][kTileDim * kLdsStride];
+  __shared__ uint32_t prefix[kPrefixInRegs];
   constexpr uint32_t kWaveLdsBytes = sizeof(lds[0]);
   const uint32_t lane = threadIdx.x & 63, half = lane >> 5, r = lane & 31;
   const uint32_t wave = Uniform(threadIdx.x >> 6);
   uint32_t *const L = lds[wave][half];
+  // The plan's prefix once per work-group, so that finding a unit costs no round trip to
+  // memory; requested together with the unit count.
+  const bool in_lds = a.plan != nullptr && a.plan_cap + 1 <= kPrefixInRegs;
+  if (in_lds) {
+    const GPtr<const uint32_t> pre =
+        Gbl<const uint32_t>(reinterpret_cast<const uint8_t *>(a.plan) + PlanPrefixOffset(a.plan_cap, kStageAssemble));
+    for (uint32_t i = threadIdx.x; i < kPrefixInRegs; i += kTileFusedWaves * 64)
+      prefix[i] = i <= a.plan_cap ? pre[i] : kPrefixPad;
+  }
   // Work units are pairs of assembly units (every image has an even number of them).
-  const uint32_t pairs = (a.plan ? Uniform(Gbl<const uint32_t>(&a.plan->units[kStageAssemble])[0])
+  const uint32_t pairs = (a.plan ? ((CPtr<PlanHeader>)(reinterpret_cast<uintptr_t>(a.plan)))->units[kStageAssemble]
                                  : StageUnitsOf(a.single, kStageAssemble, 1)) / 2;
   const XcdSpan span = XcdBalanced(blockIdx.x, gridDim.x, pairs);
+  if (in_lds) LdsBarrier();
+  TilePair cur = {}, nxt = {};
+  uint4 a0, a1, b0, b1;
+  int32_t gs = 0, gb = 0;
+  // The unit's descriptor, and its loads that do not depend on anything else: the rows of
+  // plane 2 wave + half of both tiles (adjacent in the tile-linear symbols), the group
+  // totals from g_min on and those before it.
+  const auto request = [&](uint32_t u) {
+    Located loc;
+    if (in_lds) {
+      const uint32_t v[4] = {prefix[lane], prefix[lane + 64], prefix[lane + 128], prefix[lane + 192]};
+      loc = LocateIn(v, 2 * u);
+    } else {
+      loc = Locate(a, kStageAssemble, 2 * u, 1);
+    }
+    nxt = PairAt(DescAt(a, loc.img), loc.local);
+    const GPtr<const uint8_t> src = nxt.symbols + static_cast<size_t>(2 * wave + half) * nxt.nv +
+                                    static_cast<size_t>(nxt.t0) * kTileSyms + r * kTileDim;
+    a0 = ((GPtr<const uint4>)src)[0], a1 = ((GPtr<const uint4>)src)[1];
+    b0 = ((GPtr<const uint4>)(src + kTileSyms))[0], b1 = ((GPtr<const uint4>)(src + kTileSyms))[1];
+    if (nxt.g_span < 64) {
+      gs = lane <= nxt.g_span ? nxt.group_sums[nxt.g_min + lane] : 0;
+      gb = lane < nxt.g_min ? nxt.group_sums[lane] : 0;
+    }
+  };
+  if (span.first < span.end) request(span.first);
   for (uint32_t u = span.first; u < span.end; u += span.stride) {
-    const Located loc = Locate(a, kStageAssemble, 2 * u, 1);
-    if (!loc.valid) break;
-    const DevDesc d = LoadDesc(a, loc.img);
-    const uint32_t nv = d.nv, bx = d.bx, tiles_x = bx / kTileDim;
-    const uint32_t t0 = loc.local, t1 = t0 + 1;
-    // Rows of plane 2 wave + half, tiles t0 and t1 (adjacent in the tile-linear symbols).
-    const GPtr<const uint8_t> src = d.symbols + static_cast<size_t>(2 * wave + half) * nv +
-                                    static_cast<size_t>(t0) * kTileSyms + r * kTileDim;
-    const uint4 a0 = ((GPtr<const uint4>)src)[0], a1 = ((GPtr<const uint4>)src)[1];
-    const uint4 b0 = ((GPtr<const uint4>)(src + kTileSyms))[0], b1 = ((GPtr<const uint4>)(src + kTileSyms))[1];
-
-    // Totals of the groups before each of the (at most 64) groups the rows touch:
-    // lane i holds the sum over groups < g_min + i.
-    const uint32_t ty0 = t0 / tiles_x, tx0 = t0 - ty0 * tiles_x;
-    const uint32_t ty1 = t1 / tiles_x, tx1 = t1 - ty1 * tiles_x;
-    const uint32_t g_min = (ty0 * kTileDim * bx + tx0 * kTileDim) / kGroupSyms;
-    const uint32_t g_max = ((ty1 * kTileDim + kTileDim - 1) * bx + tx1 * kTileDim) / kGroupSyms;
-    const bool few_groups = g_max - g_min < 64;
+    cur = nxt;
+    const uint32_t nv = cur.nv, bx = cur.bx;
+    const uint32_t ty0 = cur.ty0, tx0 = cur.tx0;
+    const bool wraps = tx0 + 1 == cur.tiles_x;
+    const uint32_t ty1 = wraps ? ty0 + 1 : ty0, tx1 = wraps ? 0 : tx0 + 1;
+    const uint32_t g_min = cur.g_min;
+    const bool few_groups = cur.g_span < 64;
+    // Totals of the groups before each of the (at most 64) groups the rows touch: lane i
+    // holds the sum over groups < g_min + i.
     int32_t gpre = 0;
     if (few_groups) {
-      int32_t before = 0;
-      for (uint32_t i = lane; i < g_min; i += 64) before += d.group_sums[i];
-      before = WaveSum64(before);
-      const int32_t gs = lane <= g_max - g_min ? d.group_sums[g_min + lane] : 0;
-      int32_t incl = gs;
-#pragma unroll
-      for (uint32_t off = 1; off < 64; off <<= 1) {
-        const int32_t n = __shfl_up(incl, off);
-        if (lane >= off) incl += n;
-      }
-      gpre = before + incl - gs;
+      int32_t before = gb;
+      for (uint32_t i = lane + 64; i < g_min; i += 64) before += cur.group_sums[i];
+      before = static_cast<int32_t>(WaveTotal(static_cast<uint32_t>(before)));
+      gpre = before + static_cast<int32_t>(WaveInclusiveSum(static_cast<uint32_t>(gs))) - gs;
     }
 
     uint32_t oa[8], ob[8];
@@ -1779,10 +1842,13 @@ __global__ __launch_bounds__(kTileFusedWaves * 64, 5) void WaveletAssembleKernel
     db[0] = make_uint4(ob[0], ob[1], ob[2], ob[3]);
     db[1] = make_uint4(ob[4], ob[5], ob[6], ob[7]);
     LdsBarrier();
+    // The next unit's loads are in flight while this one is assembled (the registers of the
+    // transform are free now).
+    if (u + span.stride < span.end) request(u + span.stride);
 
-    const GPtr<const uint8_t> diffs = d.symbols + SymbolOffset(d, 3);
-    const GPtr<const uint32_t> pal = (GPtr<const uint32_t>)(d.symbols + SymbolOffset(d, 2));
-    const uint32_t words = d.palette_bytes / 4;
+    const GPtr<const uint8_t> diffs = cur.symbols + 6 * nv + cur.palette_bytes;
+    const GPtr<const uint32_t> pal = (GPtr<const uint32_t>)(cur.symbols + 6 * nv);
+    const uint32_t words = cur.palette_bytes / 4;
     const uint8_t *const tiles = reinterpret_cast<const uint8_t *>(&lds[0][0][0]);
     bool bad = false;
     // 64 tile rows (2 positions x 32) in row groups of 8: lane l takes blocks
@@ -1792,6 +1858,7 @@ __global__ __launch_bounds__(kTileFusedWaves * 64, 5) void WaveletAssembleKernel
     constexpr uint32_t kGroupsOfRows = 2 * kTileDim / 8;
     constexpr uint32_t kSteps = (kGroupsOfRows + kTileFusedWaves - 1) / kTileFusedWaves;  // 3
     const uint32_t sub = lane >> 3, xb = 4 * (lane & 7);
+    const int32_t from1 = (lane & 7) >= 1 ? -1 : 0, from2 = (lane & 7) >= 2 ? -1 : 0;
     uint32_t blk[kSteps], dw[kSteps];
     int32_t base[kSteps];
 #pragma unroll
@@ -1809,11 +1876,11 @@ __global__ __launch_bounds__(kTileFusedWaves * 64, 5) void WaveletAssembleKernel
         before = __shfl(gpre, static_cast<int>(g - g_min));
       } else {
         before = 0;
-        for (uint32_t k = xb / 4; k < g; k += 8) before += d.group_sums[k];
+        for (uint32_t k = xb / 4; k < g; k += 8) before += cur.group_sums[k];
 #pragma unroll
         for (int off = 4; off > 0; off >>= 1) before += __shfl_xor(before, off, 8);
       }
-      base[i] = before + GroupLocalPrefix(d, row0);
+      base[i] = before + GroupLocalPrefix(cur, row0);
     }
     uint32_t word[kSteps][4];
 #pragma unroll
@@ -1825,12 +1892,11 @@ __global__ __launch_bounds__(kTileFusedWaves * 64, 5) void WaveletAssembleKernel
         acc += static_cast<int32_t>((dw[i] >> (8 * k)) & 0xFFu) - 128;
         run[k] = acc;
       }
+      // Inclusive sum over 8 lanes: row shifts, with a lane's reach past its 8 masked off.
       int32_t incl = acc;
-#pragma unroll
-      for (uint32_t off = 1; off < 8; off <<= 1) {
-        const int32_t n = __shfl_up(incl, off, 8);
-        if ((lane & 7) >= off) incl += n;
-      }
+      incl += __builtin_amdgcn_update_dpp(0, incl, 0x111, 0xF, 0xF, true) & from1;
+      incl += __builtin_amdgcn_update_dpp(0, incl, 0x112, 0xF, 0xF, true) & from2;
+      incl += __builtin_amdgcn_update_dpp(0, incl, 0x114, 0xF, 0xA, true);  // into lanes 4-7 of each 8
       const int32_t start = base[i] + incl - acc;
 #pragma unroll
       for (uint32_t k = 0; k < 4; ++k) {
@@ -1855,7 +1921,7 @@ __global__ __launch_bounds__(kTileFusedWaves * 64, 5) void WaveletAssembleKernel
 #pragma unroll
         for (uint32_t k = 0; k < 4; ++k) BlockColours(pw[0], pw[1], pw[2], pw[4], pw[3], pw[5], k, rgb[k]);
         const uint32_t by = (P ? ty1 : ty0) * kTileDim + y, x4 = (P ? tx1 : tx0) * kTileDim + xb;
-        GPtr<uint8_t> row = d.out + 3 * (static_cast<size_t>(d.width) * 4 * by + 4 * x4);
+        GPtr<uint8_t> row = cur.out + 3 * (static_cast<size_t>(4 * cur.bx) * 4 * by + 4 * x4);
 #pragma unroll
         for (uint32_t t = 0; t < 4; ++t) {
           uint32_t o[12];
@@ -1864,7 +1930,7 @@ __global__ __launch_bounds__(kTileFusedWaves * 64, 5) void WaveletAssembleKernel
           const GPtr<u32x4Words> dst = (GPtr<u32x4Words>)row;
 #pragma unroll
           for (uint32_t k = 0; k < 3; ++k) dst[k] = u32x4Words{o[4 * k], o[4 * k + 1], o[4 * k + 2], o[4 * k + 3]};
-          row += 3 * static_cast<size_t>(d.width);
+          row += 3 * static_cast<size_t>(4 * cur.bx);
         }
       } else {
         uint32_t o[8];
@@ -1873,7 +1939,7 @@ __global__ __launch_bounds__(kTileFusedWaves * 64, 5) void WaveletAssembleKernel
           o[2 * k] = Rgb565Pair(pw[0], pw[1], pw[2], pw[4], pw[3], pw[5], k);
           o[2 * k + 1] = word[i][k];
         }
-        const GPtr<uint4> dst = (GPtr<uint4>)(d.out + 8 * static_cast<size_t>(blk[i]));
+        const GPtr<uint4> dst = (GPtr<uint4>)(cur.out + 8 * static_cast<size_t>(blk[i]));
         dst[0] = make_uint4(o[0], o[1], o[2], o[3]);
         dst[1] = make_uint4(o[4], o[5], o[6], o[7]);
       }
