@@ -1338,15 +1338,11 @@ __device__ __forceinline__ bool WaveletTile(const KernelArgs &a, uint32_t u, uin
   return true;
 }
 
-// Row r of two tiles (a: 32 symbols of the first, b: of the second) through the five
-// levels, with this half-wave's transpose tile L; returns the rows' int8 results,
-// 32 bytes each.
-__device__ __forceinline__ void TransformRowPair(const uint4 &a0, const uint4 &a1, const uint4 &b0,
-                                                 const uint4 &b1, uint32_t *L, uint32_t r, uint32_t (&oa)[8],
-                                                 uint32_t (&ob)[8]) {
+// Row r of two tiles (a: 32 symbols of the first, b: of the second) as 16-bit pairs.
+__device__ __forceinline__ void UnpackRowPair(const uint4 &a0, const uint4 &a1, const uint4 &b0, const uint4 &b1,
+                                              s16x2 (&v)[kTileDim]) {
   const uint32_t wa[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
   const uint32_t wb[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
-  s16x2 v[kTileDim];
 #pragma unroll
   for (int i = 0; i < static_cast<int>(kTileDim); ++i) {
     // Byte i&3 of the first tile's word to bits 0-7, of the second's to bits
@@ -1355,6 +1351,15 @@ __device__ __forceinline__ void TransformRowPair(const uint4 &a0, const uint4 &a
     const uint32_t sel = 0x0C000C00u | q | ((4u + q) << 16);
     v[i] = AsPair(__builtin_amdgcn_perm(wb[i >> 2], wa[i >> 2], sel)) - static_cast<s16x2>(128);
   }
+}
+
+// The pair's rows through the five levels, with this half-wave's transpose tile L;
+// returns the rows' int8 results, 32 bytes each.
+__device__ __forceinline__ void TransformRowPair(const uint4 &a0, const uint4 &a1, const uint4 &b0,
+                                                 const uint4 &b1, uint32_t *L, uint32_t r, uint32_t (&oa)[8],
+                                                 uint32_t (&ob)[8]) {
+  s16x2 v[kTileDim];
+  UnpackRowPair(a0, a1, b0, b1, v);
   WaveletLevel<2>(v, L, static_cast<int>(r));
   WaveletLevel<4>(v, L, static_cast<int>(r));
   WaveletLevel<8>(v, L, static_cast<int>(r));
@@ -1368,6 +1373,30 @@ __device__ __forceinline__ void TransformRowPair(const uint4 &a0, const uint4 &a
     oa[w] = __builtin_amdgcn_perm(t23, t01, 0x05040100u);
     ob[w] = __builtin_amdgcn_perm(t23, t01, 0x07060302u);
   }
+}
+
+// The same, with the results left in L instead: the pair of row y, column x at L[33 y + x],
+// each value wrapped to a signed byte as the reference's int8 planes hold it.  The column
+// pass of the last level writes them there, so the rows are not read back.
+__device__ __forceinline__ void TransformToLds(const uint4 &a0, const uint4 &a1, const uint4 &b0, const uint4 &b1,
+                                               uint32_t *L, uint32_t r) {
+  s16x2 v[kTileDim];
+  UnpackRowPair(a0, a1, b0, b1, v);
+  WaveletLevel<2>(v, L, static_cast<int>(r));
+  WaveletLevel<4>(v, L, static_cast<int>(r));
+  WaveletLevel<8>(v, L, static_cast<int>(r));
+  WaveletLevel<16>(v, L, static_cast<int>(r));
+  Inverse1D<kTileDim>(v);
+#pragma unroll
+  for (uint32_t c = 0; c < kTileDim; ++c) L[r * kLdsStride + c] = Bits(v[c]);
+  WaveSync();
+#pragma unroll
+  for (uint32_t c = 0; c < kTileDim; ++c) v[c] = AsPair(L[c * kLdsStride + r]);
+  WaveSync();
+  Inverse1D<kTileDim>(v);
+#pragma unroll
+  for (uint32_t c = 0; c < kTileDim; ++c)
+    L[c * kLdsStride + r] = Bits((v[c] << static_cast<s16x2>(8)) >> static_cast<s16x2>(8));
 }
 
 template <uint32_t WAVES>
@@ -1626,29 +1655,24 @@ __global__ __launch_bounds__(WAVES * 64) void AssembleFusedWideKernel(KernelArgs
   }
 }
 
-// Byte k of a and of b, sign-extended into the low and high 16-bit halves.
-__device__ __forceinline__ s16x2 SBytePair(uint32_t a, uint32_t b, uint32_t k) {
-  // Selector codes 0-3 take bytes of the second operand, 4-7 of the first, 0x0c a zero:
-  // a's byte to bits 8-15, b's to bits 24-31, then an arithmetic shift of each half.
-  const uint32_t sel = 0x0C | (k << 8) | (0x0Cu << 16) | ((4u + k) << 24);
-  return AsPair(__builtin_amdgcn_perm(b, a, sel)) >> static_cast<s16x2>(8);
-}
-
 // Rgb565 of both endpoints of a block at once, endpoint 1 in the low and endpoint 2 in
 // the high half: the same truncating divisions and the same low 16 bits of the shifts
-// (|y|, |co|, |cg| <= 128, so every intermediate fits 16 bits).  Arguments: the four
-// blocks' plane words (y1, y2, co1, co2, cg1, cg2) and the block's byte k.
-__device__ __forceinline__ uint32_t Rgb565Pair(uint32_t y1, uint32_t y2, uint32_t co1, uint32_t co2,
-                                               uint32_t cg1, uint32_t cg2, uint32_t k) {
-  const s16x2 y = SBytePair(y1, y2, k), co = SBytePair(co1, co2, k);
-  uint32_t cgw = Bits(SBytePair(cg1, cg2, k));
-  asm volatile("" : "+v"(cgw));  // else cg / 2 is split into two 16-bit halves and re-packed
-  const s16x2 cg = AsPair(cgw);
-  const s16x2 t = y - TruncDiv2(cg);
-  const s16x2 g = cg + t;
-  const s16x2 b = TruncDiv2(t - co);
-  const s16x2 r = b + co;
-  return Bits(r << static_cast<s16x2>(11)) | Bits(g << static_cast<s16x2>(5)) | Bits(b);
+// (|y|, |co|, |cg| <= 128, so every intermediate fits 16 bits).
+struct EndPair {
+  s16x2 r, g, b;
+};
+__device__ __forceinline__ EndPair EndpointPair(uint32_t y, uint32_t co, uint32_t cg) {
+  asm volatile("" : "+v"(cg));  // else cg / 2 is split into two 16-bit halves and re-packed
+  const s16x2 t = AsPair(y) - TruncDiv2(AsPair(cg));
+  EndPair e;
+  e.g = AsPair(cg) + t;
+  e.b = TruncDiv2(t - AsPair(co));
+  e.r = e.b + AsPair(co);
+  return e;
+}
+__device__ __forceinline__ uint32_t Rgb565Pair(uint32_t y, uint32_t co, uint32_t cg) {
+  const EndPair e = EndpointPair(y, co, cg);
+  return Bits(e.r << static_cast<s16x2>(11)) | Bits(e.g << static_cast<s16x2>(5)) | Bits(e.b);
 }
 
 // The four colours of a block (codec/assemble.cl:83-130) as three words, one a channel: byte
@@ -1668,19 +1692,11 @@ __device__ __forceinline__ uint32_t FourColours(s16x2 ends) {
   return __builtin_amdgcn_perm(between, e, 0x05040200u);
 }
 
-__device__ __forceinline__ void BlockColours(uint32_t y1, uint32_t y2, uint32_t co1, uint32_t co2, uint32_t cg1,
-                                             uint32_t cg2, uint32_t k, uint32_t (&rgb)[3]) {
-  const s16x2 y = SBytePair(y1, y2, k), co = SBytePair(co1, co2, k);
-  uint32_t cgw = Bits(SBytePair(cg1, cg2, k));
-  asm volatile("" : "+v"(cgw));  // as in Rgb565Pair
-  const s16x2 cg = AsPair(cgw);
-  const s16x2 t = y - TruncDiv2(cg);
-  const s16x2 g = cg + t;
-  const s16x2 b = TruncDiv2(t - co);
-  const s16x2 r = b + co;
-  rgb[0] = FourColours((r << static_cast<s16x2>(3)) | (r >> static_cast<s16x2>(2)));
-  rgb[1] = FourColours((g << static_cast<s16x2>(2)) | (g >> static_cast<s16x2>(4)));
-  rgb[2] = FourColours((b << static_cast<s16x2>(3)) | (b >> static_cast<s16x2>(2)));
+__device__ __forceinline__ void BlockColours(uint32_t y, uint32_t co, uint32_t cg, uint32_t (&rgb)[3]) {
+  const EndPair e = EndpointPair(y, co, cg);
+  rgb[0] = FourColours((e.r << static_cast<s16x2>(3)) | (e.r >> static_cast<s16x2>(2)));
+  rgb[1] = FourColours((e.g << static_cast<s16x2>(2)) | (e.g >> static_cast<s16x2>(4)));
+  rgb[2] = FourColours((e.b << static_cast<s16x2>(3)) | (e.b >> static_cast<s16x2>(2)));
 }
 
 // One texel row of a block, 4 texels of RGB8 in three words: the row's four 2-bit indices
@@ -1709,16 +1725,16 @@ typedef uint32_t u32x4Words __attribute__((ext_vector_type(4), aligned(4)));
 //
 // A work unit is two consecutive assembly units of one image, i.e. tile positions
 // t0 and t0 + 1 of the per-plane raster tile order (every plane has a multiple of 8
-// tiles, so pairs never straddle images).  Wave w transforms planes 2w and 2w + 1,
-// one per half-wave, with t0 in the low and t0 + 1 in the high 16 bits, exactly as
-// InvWaveletKernel does, and leaves the int8 rows of its four tiles in its own
-// transpose space (1 KiB a tile).  After a work-group barrier each half-wave
-// assembles tile rows: lane x of row y of position P is block (32 ty + y, 32 tx + x)
-// of that position; its six plane values are LDS bytes, its palette index is the
-// row's base plus a 32-lane scan of the diffs, and its 8 bytes join the row's 256
-// contiguous output bytes.  A row's base is the earlier groups' totals (one 64-lane
-// scan of the group sums of the groups the unit's rows touch, when at most 64; else a
-// per-row reduction) plus the sum before the row within its group.
+// tiles, so pairs never straddle images).  Wave 0 transforms the Y planes, wave 1 the Co
+// and wave 2 the Cg planes, endpoint 1's in the low and endpoint 2's in the high 16 bits,
+// position t0 in the lower and t0 + 1 in the upper half-wave, with the arithmetic of
+// InvWaveletKernel, and leaves the values in its transpose space.  A block's three words
+// there are then what the endpoint conversion takes for both endpoints at once, with
+// nothing packed or unpacked in between.  After a work-group barrier the waves assemble
+// the tile rows: a lane takes four blocks, whose palette indices are the row's base plus
+// a scan of the diffs over 8 lanes.  A row's base is the earlier groups' totals (one
+// 64-lane scan of the group sums of the groups the unit's rows touch, when at most 64;
+// else a per-row reduction) plus the sum before the row within its group.
 constexpr uint32_t kTileFusedWaves = 3;
 
 // Tile positions t0 and t0 + 1 of an image: what the fused kernel needs of its descriptor,
@@ -1764,14 +1780,17 @@ __device__ __forceinline__ TilePair PairAt(CPtr<ImageDesc> d, uint32_t t0) {
 // thirds of the transform's own time.  So the plan's prefix is in LDS, the next unit's
 // descriptor and loads go out while this one is assembled, where the transform's registers
 // are free, and all sums over lanes are DPP: the batch of 128 textures 55.1 -> 53.0 us, 24
-// textures 15.6 -> 14.4, one unit alone 15,700 -> 12,400 cycles.
+// textures 15.6 -> 14.4.  From there on the vector unit bounds it (22.1 M instructions, 42
+// of the 53 us at 4.5 waves a SIMD): pairs of planes that the conversion takes as they lie,
+// no read back of the last level's rows, addresses with a scalar base, signed dot products
+// for the running indices and the palette's range check in the buffer: 20.8 M, 49.6 us (24
+// textures 13.4, one 512x512 image 7.6 -> 7.0, 4096x4096 11.4 -> 10.3).
 //
 // At most 96 VGPRs: 5 waves per SIMD, about what the 26 KiB of LDS allows.
 template <bool kRgb>
 __global__ __launch_bounds__(kTileFusedWaves * 64, 5) void WaveletAssembleKernel(KernelArgs a) {
   __shared__ uint32_t lds[kTileFusedWaves][2][kTileDim * kLdsStride];
   __shared__ uint32_t prefix[kPrefixInRegs];
-  constexpr uint32_t kWaveLdsBytes = sizeof(lds[0]);
   const uint32_t lane = threadIdx.x & 63, half = lane >> 5, r = lane & 31;
   const uint32_t wave = Uniform(threadIdx.x >> 6);
   uint32_t *const L = lds[wave][half];
@@ -1789,12 +1808,13 @@ __global__ __launch_bounds__(kTileFusedWaves * 64, 5) void WaveletAssembleKernel
                                  : StageUnitsOf(a.single, kStageAssemble, 1)) / 2;
   const XcdSpan span = XcdBalanced(blockIdx.x, gridDim.x, pairs);
   if (in_lds) LdsBarrier();
-  TilePair cur = {}, nxt = {};
+  uint32_t img = 0, t0 = 0;  // of the unit requested last
   uint4 a0, a1, b0, b1;
   int32_t gs = 0, gb = 0;
-  // The unit's descriptor, and its loads that do not depend on anything else: the rows of
-  // plane 2 wave + half of both tiles (adjacent in the tile-linear symbols), the group
-  // totals from g_min on and those before it.
+  // The unit's descriptor, and its loads that do not depend on anything else: row r of the
+  // wave's two planes (Y1, Y2; Co1, Co2; Cg1, Cg2) for the half's position, the group totals
+  // from g_min on and those before it.
+  const uint32_t plane1 = wave == 0 ? 0u : wave + 1, planes_apart = wave == 0 ? 1u : 2u;
   const auto request = [&](uint32_t u) {
     Located loc;
     if (in_lds) {
@@ -1803,11 +1823,14 @@ __global__ __launch_bounds__(kTileFusedWaves * 64, 5) void WaveletAssembleKernel
     } else {
       loc = Locate(a, kStageAssemble, 2 * u, 1);
     }
-    nxt = PairAt(DescAt(a, loc.img), loc.local);
-    const GPtr<const uint8_t> src = nxt.symbols + static_cast<size_t>(2 * wave + half) * nxt.nv +
-                                    static_cast<size_t>(nxt.t0) * kTileSyms + r * kTileDim;
-    a0 = ((GPtr<const uint4>)src)[0], a1 = ((GPtr<const uint4>)src)[1];
-    b0 = ((GPtr<const uint4>)(src + kTileSyms))[0], b1 = ((GPtr<const uint4>)(src + kTileSyms))[1];
+    img = Uniform(loc.img);
+    t0 = Uniform(loc.local);
+    const TilePair nxt = PairAt(DescAt(a, img), t0);
+    const GPtr<const uint8_t> src = nxt.symbols + static_cast<size_t>(plane1) * nxt.nv + nxt.t0 * kTileSyms;
+    const GPtr<const uint8_t> src2 = src + static_cast<size_t>(planes_apart) * nxt.nv;
+    const uint32_t at = half * kTileSyms + r * kTileDim;
+    a0 = ((GPtr<const uint4>)(src + at))[0], a1 = ((GPtr<const uint4>)(src + at))[1];
+    b0 = ((GPtr<const uint4>)(src2 + at))[0], b1 = ((GPtr<const uint4>)(src2 + at))[1];
     if (nxt.g_span < 64) {
       gs = lane <= nxt.g_span ? nxt.group_sums[nxt.g_min + lane] : 0;
       gb = lane < nxt.g_min ? nxt.group_sums[lane] : 0;
@@ -1815,7 +1838,9 @@ __global__ __launch_bounds__(kTileFusedWaves * 64, 5) void WaveletAssembleKernel
   };
   if (span.first < span.end) request(span.first);
   for (uint32_t u = span.first; u < span.end; u += span.stride) {
-    cur = nxt;
+    // Read again from the scalar cache rather than carried: two units' descriptors would not
+    // fit the scalar registers.
+    const TilePair cur = PairAt(DescAt(a, Uniform(img)), Uniform(t0));
     const uint32_t nv = cur.nv, bx = cur.bx;
     const uint32_t ty0 = cur.ty0, tx0 = cur.tx0;
     const bool wraps = tx0 + 1 == cur.tiles_x;
@@ -1832,44 +1857,40 @@ __global__ __launch_bounds__(kTileFusedWaves * 64, 5) void WaveletAssembleKernel
       gpre = before + static_cast<int32_t>(WaveInclusiveSum(static_cast<uint32_t>(gs))) - gs;
     }
 
-    uint32_t oa[8], ob[8];
-    TransformRowPair(a0, a1, b0, b1, L, r, oa, ob);
-    // Tile (2 half + P) of this wave's space: row r at byte 32 r.
-    uint4 *const da = reinterpret_cast<uint4 *>(&lds[wave][0][0] + (2 * half + 0) * (kTileSyms / 4) + r * 8);
-    uint4 *const db = reinterpret_cast<uint4 *>(&lds[wave][0][0] + (2 * half + 1) * (kTileSyms / 4) + r * 8);
-    da[0] = make_uint4(oa[0], oa[1], oa[2], oa[3]);
-    da[1] = make_uint4(oa[4], oa[5], oa[6], oa[7]);
-    db[0] = make_uint4(ob[0], ob[1], ob[2], ob[3]);
-    db[1] = make_uint4(ob[4], ob[5], ob[6], ob[7]);
+    TransformToLds(a0, a1, b0, b1, L, r);
     LdsBarrier();
     // The next unit's loads are in flight while this one is assembled (the registers of the
     // transform are free now).
     if (u + span.stride < span.end) request(u + span.stride);
 
-    const GPtr<const uint8_t> diffs = cur.symbols + 6 * nv + cur.palette_bytes;
-    const GPtr<const uint32_t> pal = (GPtr<const uint32_t>)(cur.symbols + 6 * nv);
+    const GPtr<const uint8_t> diffs = cur.symbols + 6 * static_cast<size_t>(nv) + cur.palette_bytes;
+    const GPtr<const uint8_t> lane_sums = (GPtr<const uint8_t>)cur.lane_sums;
+    const GPtr<const uint8_t> suffixes = lane_sums + 4 * static_cast<size_t>(LaneSuffixBase(nv));
+    const __amdgpu_buffer_rsrc_t pal =
+        MakeRsrc(reinterpret_cast<const void *>((uintptr_t)(cur.symbols + 6 * static_cast<size_t>(nv))), cur.palette_bytes);
     const uint32_t words = cur.palette_bytes / 4;
-    const uint8_t *const tiles = reinterpret_cast<const uint8_t *>(&lds[0][0][0]);
-    bool bad = false;
+    uint32_t worst = 0;  // the largest palette index
     // 64 tile rows (2 positions x 32) in row groups of 8: lane l takes blocks
     // 4 (l % 8) .. +3 of row l / 8 of its group, and wave w groups w, w + 3, w + 6
     // (< 8).  Each phase runs over all of a wave's groups, so their loads are in
-    // flight together: diffs and row bases, then palette words, then the stores.
+    // flight together: diffs and row bases, then palette words, then the stores.  What
+    // depends on the group alone is scalar, so that a load takes its address from a
+    // scalar base and one 32-bit offset.
     constexpr uint32_t kGroupsOfRows = 2 * kTileDim / 8;
     constexpr uint32_t kSteps = (kGroupsOfRows + kTileFusedWaves - 1) / kTileFusedWaves;  // 3
     const uint32_t sub = lane >> 3, xb = 4 * (lane & 7);
     const int32_t from1 = (lane & 7) >= 1 ? -1 : 0, from2 = (lane & 7) >= 2 ? -1 : 0;
-    uint32_t blk[kSteps], dw[kSteps];
+    const uint32_t row_off = sub * bx, blk_off = row_off + xb;
+    uint32_t group0[kSteps], dw[kSteps];  // first block of the row group; the lane's four diffs
     int32_t base[kSteps];
 #pragma unroll
     for (uint32_t i = 0; i < kSteps; ++i) {
       const uint32_t grp0 = wave + kTileFusedWaves * i;
-      const uint32_t q = 8 * (grp0 < kGroupsOfRows ? grp0 : wave) + sub;  // a spare step repeats group `wave`
-      const uint32_t P = q / kTileDim, y = q % kTileDim;
-      const uint32_t ty = P ? ty1 : ty0, tx = P ? tx1 : tx0;
-      const uint32_t row0 = (ty * kTileDim + y) * bx + tx * kTileDim;
-      blk[i] = row0 + xb;
-      dw[i] = *(GPtr<const uint32_t>)(diffs + blk[i]);
+      const uint32_t grp = grp0 < kGroupsOfRows ? grp0 : wave;  // a spare step repeats group `wave`
+      const uint32_t P = grp / 4, ty = P ? ty1 : ty0, tx = P ? tx1 : tx0;
+      group0[i] = (ty * kTileDim + 8 * (grp & 3)) * bx + tx * kTileDim;
+      dw[i] = *(GPtr<const uint32_t>)(diffs + group0[i] + blk_off) ^ 0x80808080u;  // signed bytes: diff - 128
+      const uint32_t row0 = group0[i] + row_off;
       const uint32_t g = row0 / kGroupSyms;
       int32_t before;
       if (few_groups) {
@@ -1880,70 +1901,72 @@ __global__ __launch_bounds__(kTileFusedWaves * 64, 5) void WaveletAssembleKernel
 #pragma unroll
         for (int off = 4; off > 0; off >>= 1) before += __shfl_xor(before, off, 8);
       }
-      base[i] = before + GroupLocalPrefix(cur, row0);
+      // GroupLocalPrefix: entries row0 / 256 and row0 / 32 (row0 is a multiple of 32).
+      base[i] = before + *(GPtr<const int32_t>)(lane_sums + row0 / kSymsPerLane * 4) -
+                *(GPtr<const int32_t>)(suffixes + row0 / kRowBlocks * 4);
     }
     uint32_t word[kSteps][4];
 #pragma unroll
     for (uint32_t i = 0; i < kSteps; ++i) {
-      int32_t run[4];
-      int32_t acc = 0;
-#pragma unroll
-      for (uint32_t k = 0; k < 4; ++k) {
-        acc += static_cast<int32_t>((dw[i] >> (8 * k)) & 0xFFu) - 128;
-        run[k] = acc;
-      }
       // Inclusive sum over 8 lanes: row shifts, with a lane's reach past its 8 masked off.
-      int32_t incl = acc;
+      const int32_t total = __builtin_amdgcn_sdot4(static_cast<int>(dw[i]), 0x01010101, 0, false);
+      int32_t incl = total;
       incl += __builtin_amdgcn_update_dpp(0, incl, 0x111, 0xF, 0xF, true) & from1;
       incl += __builtin_amdgcn_update_dpp(0, incl, 0x112, 0xF, 0xF, true) & from2;
       incl += __builtin_amdgcn_update_dpp(0, incl, 0x114, 0xF, 0xA, true);  // into lanes 4-7 of each 8
-      const int32_t start = base[i] + incl - acc;
+      const int32_t start = base[i] + incl - total;
 #pragma unroll
       for (uint32_t k = 0; k < 4; ++k) {
-        const uint32_t pi = static_cast<uint32_t>(start + run[k]);
-        word[i][k] = 0;
-        if (pi < words) word[i][k] = pal[pi]; else bad = true;
+        // The sum of the first k + 1 diffs on top of `start`.
+        const uint32_t pi = static_cast<uint32_t>(
+            __builtin_amdgcn_sdot4(static_cast<int>(dw[i]), static_cast<int>(0x01010101u >> (24 - 8 * k)), start, false));
+        worst = max(worst, pi);
+        // An index outside the palette reads a zero word through the buffer's range check.
+        word[i][k] = __builtin_amdgcn_raw_buffer_load_b32(pal, static_cast<int>(min(pi, words) * 4), 0, 0);
       }
     }
 #pragma unroll
     for (uint32_t i = 0; i < kSteps; ++i) {
       const uint32_t grp = wave + kTileFusedWaves * i;
       if (grp >= kGroupsOfRows) continue;
-      const uint32_t q = 8 * grp + sub;
-      const uint32_t P = q / kTileDim, y = q % kTileDim;
-      uint32_t pw[6];
+      const uint32_t P = grp / 4;
+      const uint32_t at = (8 * (grp & 3) + sub) * kLdsStride + xb;
+      uint32_t pw[3][4];
 #pragma unroll
-      for (uint32_t p = 0; p < 6; ++p)
-        pw[p] = *reinterpret_cast<const uint32_t *>(tiles + (p >> 1) * kWaveLdsBytes +
-                                                    ((p & 1) * 2 + P) * kTileSyms + y * kTileDim + xb);
+      for (uint32_t p = 0; p < 3; ++p)
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) pw[p][k] = lds[p][P][at + k];
       if constexpr (kRgb) {
         uint32_t rgb[4][3];
 #pragma unroll
-        for (uint32_t k = 0; k < 4; ++k) BlockColours(pw[0], pw[1], pw[2], pw[4], pw[3], pw[5], k, rgb[k]);
-        const uint32_t by = (P ? ty1 : ty0) * kTileDim + y, x4 = (P ? tx1 : tx0) * kTileDim + xb;
-        GPtr<uint8_t> row = cur.out + 3 * (static_cast<size_t>(4 * cur.bx) * 4 * by + 4 * x4);
+        for (uint32_t k = 0; k < 4; ++k) BlockColours(pw[0][k], pw[1][k], pw[2][k], rgb[k]);
+        // Byte 48 of a block, 12 of it a texel row; a texel row of the image is 12 bx bytes.
+        const uint32_t tx = P ? tx1 : tx0, ty = P ? ty1 : ty0;
+        GPtr<uint8_t> row = cur.out + 48 * static_cast<size_t>(ty * kTileDim + 8 * (grp & 3)) * bx + 12 * tx * kTileDim;
+        const uint32_t off = 48 * row_off + 12 * xb;
 #pragma unroll
         for (uint32_t t = 0; t < 4; ++t) {
           uint32_t o[12];
 #pragma unroll
           for (uint32_t k = 0; k < 4; ++k) BlockRow(rgb[k], word[i][k], t, o + 3 * k);
-          const GPtr<u32x4Words> dst = (GPtr<u32x4Words>)row;
+          const GPtr<u32x4Words> dst = (GPtr<u32x4Words>)(row + off);
 #pragma unroll
           for (uint32_t k = 0; k < 3; ++k) dst[k] = u32x4Words{o[4 * k], o[4 * k + 1], o[4 * k + 2], o[4 * k + 3]};
-          row += 3 * static_cast<size_t>(4 * cur.bx);
+          row += 12 * static_cast<size_t>(bx);
         }
       } else {
         uint32_t o[8];
 #pragma unroll
         for (uint32_t k = 0; k < 4; ++k) {
-          o[2 * k] = Rgb565Pair(pw[0], pw[1], pw[2], pw[4], pw[3], pw[5], k);
+          o[2 * k] = Rgb565Pair(pw[0][k], pw[1][k], pw[2][k]);
           o[2 * k + 1] = word[i][k];
         }
-        const GPtr<uint4> dst = (GPtr<uint4>)(cur.out + 8 * static_cast<size_t>(blk[i]));
+        const GPtr<uint4> dst = (GPtr<uint4>)(cur.out + 8 * static_cast<size_t>(group0[i]) + 8 * blk_off);
         dst[0] = make_uint4(o[0], o[1], o[2], o[3]);
         dst[1] = make_uint4(o[4], o[5], o[6], o[7]);
       }
     }
+    const bool bad = worst >= words;
     if (bad) atomicOr(a.err, kErrPaletteIndex);
     LdsBarrier();  // the next unit's transposes reuse the tiles' space
   }
