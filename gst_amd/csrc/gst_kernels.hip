@@ -1284,8 +1284,9 @@ constexpr int kLdsStride = kTileDim + 1;
 
 // One level on the half-wave's tile pair; lanes r >= LEN sit out (their rows and
 // columns are outside this level's square).  Each half-wave owns its LDS tile, so
-// wave-level ordering is all the transposes need.
-template <int LEN>
+// wave-level ordering is all the transposes need.  The level's result is left in L, row y
+// at L[33 y], and with kReadBack in the rows again.
+template <int LEN, bool kReadBack = true>
 __device__ __forceinline__ void WaveletLevel(s16x2 (&v)[kTileDim], uint32_t *L, int r) {
   if (r < LEN) {
     Inverse1D<LEN>(v);
@@ -1304,9 +1305,78 @@ __device__ __forceinline__ void WaveletLevel(s16x2 (&v)[kTileDim], uint32_t *L, 
     for (int c = 0; c < LEN; ++c) L[c * kLdsStride + r] = Bits(v[c]);
   }
   WaveSync();
-  if (r < LEN) {
+  if (kReadBack) {
+    if (r < LEN) {
 #pragma unroll
-    for (int c = 0; c < LEN; ++c) v[c] = AsPair(L[r * kLdsStride + c]);
+      for (int c = 0; c < LEN; ++c) v[c] = AsPair(L[r * kLdsStride + c]);
+    }
+    WaveSync();
+  }
+}
+
+// One pass of level LEN = 8 or 16 in L, by all 32 lanes of the half-wave: 32 / LEN lanes a
+// line, each the outputs of N = LEN * LEN / 64 consecutive k.  `step` is the distance of a
+// line's elements, `line` its start, `part` the lane's place in it.  The mirrored ends
+// are other addresses for the first and last part: the neighbour before is lo and hi 0 of
+// the line itself, the one after the last is the last again (its even output, recomputed
+// from hi[k - 1] and hi[k]).
+template <int LEN>
+__device__ __forceinline__ void SplitPass(uint32_t *L, uint32_t line, uint32_t step, uint32_t part) {
+  constexpr int MID = LEN / 2, N = LEN * LEN / 64;
+  constexpr uint32_t kParts = MID / N;
+  const uint32_t *const own = L + line + part * N * step;
+  const uint32_t *const prev = part == 0 ? own : own - step;
+  const bool end = part == kParts - 1;
+  const uint32_t *const next = own + (end ? N - 1 : N) * step;
+  s16x2 lo[N + 1], hi[N + 2];  // hi[j + 1] is hi of the lane's j-th k
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    lo[j] = AsPair(own[j * step]);
+    hi[j + 1] = AsPair(own[(MID + j) * step]);
+  }
+  hi[0] = AsPair(prev[MID * step]);
+  lo[N] = AsPair(next[0]);
+  hi[N + 1] = AsPair(next[MID * step]);
+  WaveSync();
+  s16x2 even[N + 1];
+#pragma unroll
+  for (int j = 0; j < N; ++j) even[j] = lo[j] - TruncDiv4(hi[j] + hi[j + 1] + static_cast<s16x2>(2));
+  const s16x2 before = end ? hi[N - 1] : hi[N];
+  even[N] = lo[N] - TruncDiv4(before + hi[N + 1] + static_cast<s16x2>(2));
+  uint32_t *const out = L + line + 2 * part * N * step;
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    out[2 * j * step] = Bits(even[j]);
+    out[(2 * j + 1) * step] = Bits(hi[j + 1] + TruncDiv2(even[j] + even[j + 1]));
+  }
+  WaveSync();
+}
+
+template <int LEN>
+__device__ __forceinline__ void SplitLevel(uint32_t *L, uint32_t r) {
+  constexpr uint32_t kParts = 32 / LEN;
+  const uint32_t i = r / kParts, part = r % kParts;
+  SplitPass<LEN>(L, i * kLdsStride, 1, part);
+  SplitPass<LEN>(L, i, kLdsStride, part);
+}
+
+// Levels 2 to 16.  They touch the tile's first 16 rows and columns only, so a lane a row
+// would leave half the lanes idle at level 16 and three quarters at level 8: those two run
+// from L, with 2 and 4 lanes a line (140 fewer vector instructions a wave of some 1,090).
+__device__ __forceinline__ void CoarseLevels(s16x2 (&v)[kTileDim], uint32_t *L, uint32_t r) {
+  if (r < 16) {
+#pragma unroll
+    for (uint32_t c = 0; c < 16; ++c) L[r * kLdsStride + c] = Bits(v[c]);
+  }
+  WaveletLevel<2>(v, L, static_cast<int>(r));
+  WaveletLevel<4, false>(v, L, static_cast<int>(r));
+  uint32_t lane = r;
+  asm volatile("" : "+v"(lane));  // addresses made here, not kept in registers between units
+  SplitLevel<8>(L, lane);
+  SplitLevel<16>(L, lane);
+  if (r < 16) {
+#pragma unroll
+    for (uint32_t c = 0; c < 16; ++c) v[c] = AsPair(L[r * kLdsStride + c]);
   }
   WaveSync();
 }
@@ -1360,10 +1430,7 @@ __device__ __forceinline__ void TransformRowPair(const uint4 &a0, const uint4 &a
                                                  uint32_t (&ob)[8]) {
   s16x2 v[kTileDim];
   UnpackRowPair(a0, a1, b0, b1, v);
-  WaveletLevel<2>(v, L, static_cast<int>(r));
-  WaveletLevel<4>(v, L, static_cast<int>(r));
-  WaveletLevel<8>(v, L, static_cast<int>(r));
-  WaveletLevel<16>(v, L, static_cast<int>(r));
+  CoarseLevels(v, L, r);
   WaveletLevel<32>(v, L, static_cast<int>(r));
 #pragma unroll
   for (int w = 0; w < 8; ++w) {
@@ -1382,10 +1449,7 @@ __device__ __forceinline__ void TransformToLds(const uint4 &a0, const uint4 &a1,
                                                uint32_t *L, uint32_t r) {
   s16x2 v[kTileDim];
   UnpackRowPair(a0, a1, b0, b1, v);
-  WaveletLevel<2>(v, L, static_cast<int>(r));
-  WaveletLevel<4>(v, L, static_cast<int>(r));
-  WaveletLevel<8>(v, L, static_cast<int>(r));
-  WaveletLevel<16>(v, L, static_cast<int>(r));
+  CoarseLevels(v, L, r);
   Inverse1D<kTileDim>(v);
 #pragma unroll
   for (uint32_t c = 0; c < kTileDim; ++c) L[r * kLdsStride + c] = Bits(v[c]);
