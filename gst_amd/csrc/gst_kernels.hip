@@ -436,9 +436,7 @@ __device__ __forceinline__ void DecodeHalfGroups(const uint32_t *tab, uint16_t *
       case 2: __builtin_amdgcn_s_setprio(1); break;
       default: __builtin_amdgcn_s_setprio(0); break;
     }
-    uint32_t acc[16];
-#pragma unroll
-    for (uint32_t i = 0; i < 16; ++i) acc[i] = 0;
+    uint32_t acc[16], first = 0;
 #pragma unroll
     for (uint32_t blk = 0; blk < 64 / kRefillSteps; ++blk) {
 #pragma unroll
@@ -464,13 +462,20 @@ __device__ __forceinline__ void DecodeHalfGroups(const uint32_t *tab, uint16_t *
           const uint32_t xn = (x << 16) | ring_half[widx & (kRingWords - 1)];
           x = need ? xn : x;
         }
-        // Step 8*blk + s lands at byte 63 - 8*blk - s of the sector.  The symbol (byte
-        // 3 of fs) goes in with v_perm: selector codes 4-7 take bytes of the first
-        // operand, 0-3 bytes of the second.
+        // Step 8*blk + s lands at byte 63 - 8*blk - s of the sector, the last decoded first.
+        // The symbol (byte 3 of fs) goes in with v_perm: selector codes 4-7 take bytes of
+        // the first operand, 0-3 bytes of the second, 0x0c is zero; the first two of a word
+        // go in together.
         const uint32_t pos = 63 - kRefillSteps * blk - s;
-        const uint32_t sel = (0x03020100u & ~(0xFFu << (8 * (pos & 3)))) | (7u << (8 * (pos & 3)));
-        acc[pos >> 2] = __builtin_amdgcn_perm(fs, acc[pos >> 2], sel);
-        asm volatile("" : "+v"(acc[pos >> 2]));  // insert now: keeps 64 symbols out of VGPRs
+        if ((pos & 3) == 3) {
+          first = fs;
+        } else {
+          if ((pos & 3) == 2)
+            acc[pos >> 2] = __builtin_amdgcn_perm(first, fs, 0x07030C0Cu);
+          else
+            acc[pos >> 2] = __builtin_amdgcn_perm(fs, acc[pos >> 2], (pos & 3) == 1 ? 0x0302070Cu : 0x03020107u);
+          asm volatile("" : "+v"(acc[pos >> 2]));  // insert now: keeps 64 symbols out of VGPRs
+        }
       }
       // Ring refill at the 8-step boundary: the pointer moved at most 256 words, so it
       // crossed at most one chunk boundary, and the next 8 steps read only chunks
