@@ -15,9 +15,11 @@ Device buffers and streams are passed as integer addresses / handles (for exampl
 raises GstError on a non-zero status.  The library must be built
 (gst_amd/build.py); importing without it raises, there is no fallback path.
 """
+import array
 import ctypes
 import math
 import os
+import struct
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libgst_amd.so")
@@ -212,6 +214,18 @@ def _events(init):
     return len(init), ctypes.cast(arr, _P)
 
 
+_PyBytes = ctypes.pythonapi.PyBytes_FromStringAndSize
+_PyBytes.argtypes = [_P, ctypes.c_ssize_t]
+_PyBytes.restype = ctypes.py_object
+
+
+def _new_bytes(n):
+    """A bytes object of n bytes that nobody else holds yet, to be filled by one call of
+    the library (ctypes passes its address) before anybody does: no buffer to clear and
+    copy from."""
+    return _PyBytes(None, n)
+
+
 # ---- codec/decoder.h mirror -------------------------------------------------------
 
 def InitializeDecoder(device=0):
@@ -228,10 +242,11 @@ def ParseHeader(data):
 
 def DecompressDXT(data):
     """Host .gtc bytes -> host DXT1 blocks (bytes)."""
+    data = bytes(data)
     hdr = ParseHeader(data)
-    out = ctypes.create_string_buffer(hdr.dxt_bytes)
-    _check(lib().gst_decompress_dxt(bytes(data), len(data), out, len(out)), "DecompressDXT")
-    return out.raw
+    out = _new_bytes(hdr.dxt_bytes)
+    _check(lib().gst_decompress_dxt(data, len(data), out, len(out)), "DecompressDXT")
+    return out
 
 
 def _load(fn, name, hdrs, stream, d_cmp, d_out, init, want_event):
@@ -467,14 +482,19 @@ class AnsDecoder:
         holding len(states) / len(data) streams).  Returns one bytes object of 256
         symbols per state."""
         blobs = [bytes(data)] if isinstance(data, (bytes, bytearray)) else [bytes(d) for d in data]
-        st, ns = _u32_array(states)
-        bufs = [ctypes.create_string_buffer(b, max(1, len(b))) for b in blobs]
-        ptrs = (_P * len(bufs))(*[ctypes.cast(b, _P) for b in bufs])
-        lens = (_SZ * len(bufs))(*[len(b) for b in blobs])
-        out = ctypes.create_string_buffer(ns * ANS_SYMBOLS_PER_STREAM)
-        _check(lib().gst_ans_decode(self._h, st, ns, ptrs, lens, len(bufs), out), "gst_ans_decode")
-        raw = out.raw
-        return [raw[i * ANS_SYMBOLS_PER_STREAM:(i + 1) * ANS_SYMBOLS_PER_STREAM] for i in range(ns)]
+        states = states if isinstance(states, (list, tuple)) else list(states)
+        try:
+            values = array.array("I", states)
+            ns = len(values)
+            st = (_U32 * max(1, ns)).from_buffer(values if ns else array.array("I", [0]))
+        except (TypeError, OverflowError):  # values array.array does not take as they are
+            st, ns = _u32_array(states)
+        ptrs = (ctypes.c_char_p * len(blobs))(*blobs)
+        lens = (_SZ * len(blobs))(*map(len, blobs))
+        raw = _new_bytes(ns * ANS_SYMBOLS_PER_STREAM)
+        _check(lib().gst_ans_decode(self._h, st, ns, ctypes.cast(ptrs, ctypes.POINTER(_P)), lens, len(blobs), raw),
+               "gst_ans_decode")
+        return list(struct.unpack("%ds" % ANS_SYMBOLS_PER_STREAM * ns, raw))
 
     def close(self):
         if self._h:

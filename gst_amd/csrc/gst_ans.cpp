@@ -2,7 +2,7 @@
 // of the reference's ans::ocl::OpenCLDecoder (ans/ans_ocl.h:26-72, ans/ans_ocl.cpp).
 // The table is built by the texture path's BuildTableKernel (one of its four slots)
 // and the groups are decoded by AnsGroupsKernel; this file holds the host side:
-// frequency normalisation, the data packing and the blocking copies.
+// frequency normalisation, the data packing and the blocking call.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -54,6 +54,7 @@ int BuildTable(gst_ans_decoder *d, const uint32_t *F, uint32_t n) {
 }
 
 size_t RoundUp4(size_t x) { return (x + 3) & ~static_cast<size_t>(3); }
+size_t RoundUp256(size_t x) { return (x + 255) & ~static_cast<size_t>(255); }
 
 }  // namespace
 
@@ -129,33 +130,38 @@ int gst_ans_decode(const gst_ans_decoder *d, const uint32_t *states, uint32_t nu
     total += RoundUp4(data_lens[i]) + 4 * static_cast<size_t>(lanes);
   }
   if (total > 0xFFFFFFF0u) return GST_ERR_INVALID_ARGUMENT;
-  std::vector<uint8_t> packed(total, 0);
+  const size_t out_bytes = static_cast<size_t>(num_streams) * GST_ANS_SYMBOLS_PER_STREAM;
+  const size_t out_at = RoundUp256(total), status_at = out_at + RoundUp256(out_bytes);
+  const size_t all = status_at + 4 * static_cast<size_t>(n_data);
+  // The kernel reads the packed data and writes the symbols and status words in pinned
+  // memory itself: one launch and one wait a call.
+  gst::PinnedBuffer buf;
+  hipError_t e = gst::TakePinned(all, &buf);
+  if (e != hipSuccess) return HipFail(e);
+  std::lock_guard<std::mutex> lock(d->mu);
+  uint8_t *const packed = buf.host;
   size_t at = 4 * static_cast<size_t>(n_data);
   for (uint32_t i = 0; i < n_data; ++i) {
-    const size_t end = at + RoundUp4(data_lens[i]) + 4 * static_cast<size_t>(lanes);
-    if (data_lens[i]) std::memcpy(&packed[end - 4 * lanes - data_lens[i]], data[i], data_lens[i]);
-    std::memcpy(&packed[end - 4 * lanes], states + static_cast<size_t>(i) * lanes, 4 * lanes);
-    const uint32_t end32 = static_cast<uint32_t>(end);
-    std::memcpy(&packed[4 * i], &end32, 4);
-    at = end;
+    const size_t pad = RoundUp4(data_lens[i]) - data_lens[i];
+    std::memset(packed + at, 0, pad);
+    if (data_lens[i]) std::memcpy(packed + at + pad, data[i], data_lens[i]);
+    at += pad + data_lens[i];
+    std::memcpy(packed + at, states + static_cast<size_t>(i) * lanes, 4 * lanes);
+    at += 4 * static_cast<size_t>(lanes);
+    const uint32_t end32 = static_cast<uint32_t>(at);
+    std::memcpy(packed + 4 * static_cast<size_t>(i), &end32, 4);
   }
-  const size_t out_bytes = static_cast<size_t>(num_streams) * GST_ANS_SYMBOLS_PER_STREAM;
-  std::lock_guard<std::mutex> lock(d->mu);
-  uint8_t *d_data = nullptr, *d_out = nullptr;
-  hipError_t e = hipMallocAsync(reinterpret_cast<void **>(&d_data), total, d->stream);
-  if (e == hipSuccess) e = hipMallocAsync(reinterpret_cast<void **>(&d_out), out_bytes, d->stream);
-  if (e == hipSuccess) e = hipMemcpyAsync(d_data, packed.data(), total, hipMemcpyHostToDevice, d->stream);
-  if (e == hipSuccess) e = hipMemsetAsync(d->d_err, 0, sizeof(uint32_t), d->stream);
-  if (e == hipSuccess)
-    e = gst::LaunchAnsGroups(d->d_tables, d_data, static_cast<uint32_t>(total), n_data, lanes, d_out, d->d_err,
-                             d->stream);
-  uint32_t err = 0;
-  if (e == hipSuccess) e = hipMemcpyAsync(out, d_out, out_bytes, hipMemcpyDeviceToHost, d->stream);
-  if (e == hipSuccess) e = hipMemcpyAsync(&err, d->d_err, sizeof(err), hipMemcpyDeviceToHost, d->stream);
-  if (d_data) (void)hipFreeAsync(d_data, d->stream);
-  if (d_out) (void)hipFreeAsync(d_out, d->stream);
+  e = gst::LaunchAnsGroups(d->d_tables, buf.dev, static_cast<uint32_t>(total), n_data, lanes,
+                           buf.dev + out_at, reinterpret_cast<uint32_t *>(buf.dev + status_at), d->stream);
   const hipError_t s = hipStreamSynchronize(d->stream);
   if (e == hipSuccess) e = s;
+  uint32_t err = 0;
+  if (e == hipSuccess) {
+    std::memcpy(out, packed + out_at, out_bytes);
+    const uint32_t *const status = reinterpret_cast<const uint32_t *>(packed + status_at);
+    for (uint32_t i = 0; i < n_data; ++i) err |= status[i];
+  }
+  gst::GivePinned(buf);
   if (e != hipSuccess) return HipFail(e);
   return err ? GST_ERR_CORRUPT_STREAM : GST_OK;
 }

@@ -243,7 +243,9 @@ class PinnedRing {
         // Coherent: the device reads a slot itself and must never see a stale cached copy.
         GST_HIP(hipHostMalloc(&sl.host, kSlotBytes, hipHostMallocCoherent));
         GST_HIP(hipHostGetDevicePointer(&sl.dev, sl.host, 0));
-        GST_HIP(hipEventCreateWithFlags(&sl.ev, hipEventDisableTiming));
+        // The event only tells when the slot was read: nothing on the host looks at what the
+        // device wrote, and a system-scope fence would hold the decode's first kernel 2 us.
+        GST_HIP(hipEventCreateWithFlags(&sl.ev, hipEventDisableTiming | hipEventDisableSystemFence));
         sl.used = false;
         slots_.push_back(sl);
       }
@@ -330,14 +332,109 @@ int LaunchAll(const KernelArgs &a, const uint32_t grids[gst::kNumStages], const 
   return GST_OK;
 }
 
-// Scratch for one decode call: the preallocation when it has room, otherwise
-// stream-ordered device memory released on the stream after the last kernel.
+// Device scratch that belongs to one stream, in whose order its users follow each other.
+struct KeptScratch {
+  uint8_t *ptr = nullptr;
+  size_t bytes = 0;
+  int device = 0;
+  bool busy = false;  // a call is enqueuing on it
+};
+
+constexpr size_t kKeptScratchBytes = size_t{256} << 20;
+
+// At least n bytes, the old memory given back behind the stream's work.
+hipError_t GrowScratch(KeptScratch *k, size_t n, hipStream_t s) {
+  if (n <= k->bytes) return hipSuccess;
+  hipError_t e = k->ptr ? hipFreeAsync(k->ptr, s) : hipSuccess;
+  k->ptr = nullptr;
+  k->bytes = 0;
+  size_t want = size_t{1} << 20;
+  while (want < n) want *= 2;
+  void *p = nullptr;
+  if (e == hipSuccess) e = hipMallocAsync(&p, want, s);
+  if (e != hipSuccess) return e;
+  k->ptr = static_cast<uint8_t *>(p);
+  k->bytes = want;
+  return hipSuccess;
+}
+
+// Scratch kept for the default stream's calls.  hipFreeAsync waits for the work before it
+// (measured; hipMallocAsync does not), so allocating per call makes every call wait for
+// the one before: 3 us a pass of a 512x512 image, and 60-80 us where passes are waited
+// for, as the memory goes back to the system in between.  The default stream's work is
+// one sequence for the whole process and it is never destroyed, so what a call leaves may
+// be used by the next one at once.  A stream that its owner may destroy does not have
+// that: its handle can come back as another stream while its work still runs.  Calls on
+// such streams allocate and free as before.  A slot is one call's while it enqueues, so
+// threads that share the stream take different ones.
+class DefaultStreamScratch {
+ public:
+  static DefaultStreamScratch &Get() {
+    static DefaultStreamScratch *p = new DefaultStreamScratch;  // never destroyed: the runtime may be gone by then
+    return *p;
+  }
+  // Null if the caller has to allocate.
+  KeptScratch *Take(size_t n) {
+    int dev = 0;
+    if (n > kKeptScratchBytes || hipGetDevice(&dev) != hipSuccess) return nullptr;
+    KeptScratch *pick = nullptr;
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      size_t mine = 0;
+      for (KeptScratch *k : slots_) {
+        if (k->device != dev) continue;
+        ++mine;
+        if (!k->busy && (!pick || (pick->bytes < n && k->bytes > pick->bytes))) pick = k;
+      }
+      if (!pick && mine < kSlots) {
+        pick = new KeptScratch;
+        pick->device = dev;
+        slots_.push_back(pick);
+      }
+      if (!pick) return nullptr;
+      pick->busy = true;
+    }
+    if (GrowScratch(pick, n, nullptr) == hipSuccess) return pick;
+    (void)hipGetLastError();
+    Give(pick);
+    return nullptr;
+  }
+  // After the call's last kernel was enqueued.
+  void Give(KeptScratch *k) {
+    std::lock_guard<std::mutex> lk(mu_);
+    k->busy = false;
+  }
+  void Trim() {
+    std::lock_guard<std::mutex> lk(mu_);
+    for (size_t i = 0; i < slots_.size();) {
+      KeptScratch *k = slots_[i];
+      if (k->busy) {
+        ++i;
+        continue;
+      }
+      if (k->ptr) (void)hipFree(k->ptr);  // waits for the device
+      delete k;
+      slots_.erase(slots_.begin() + i);
+    }
+    (void)hipGetLastError();
+  }
+
+ private:
+  static constexpr size_t kSlots = 2;  // a device
+  std::mutex mu_;
+  std::vector<KeptScratch *> slots_;
+};
+
+// Scratch for one decode call: the preallocation when it has room, otherwise what the
+// caller keeps for this stream (`own`) or the default stream's, otherwise stream-ordered
+// device memory released on the stream after the last kernel.
 struct Scratch {
   uint8_t *ptr = nullptr;
   bool async = false;
+  KeptScratch *slot = nullptr;  // the default stream's
 };
 
-int TakeScratch(size_t bytes, hipStream_t s, Scratch *out) {
+int TakeScratch(size_t bytes, hipStream_t s, KeptScratch *own, Scratch *out) {
   Globals &g = G();
   {
     std::lock_guard<std::mutex> lk(g.mu);
@@ -351,11 +448,27 @@ int TakeScratch(size_t bytes, hipStream_t s, Scratch *out) {
       }
     }
   }
+  if (own && bytes <= kKeptScratchBytes) {
+    GST_HIP(GrowScratch(own, bytes, s));
+    out->ptr = own->ptr;
+    return GST_OK;
+  }
+  if (!s && (out->slot = DefaultStreamScratch::Get().Take(bytes)) != nullptr) {
+    out->ptr = out->slot->ptr;
+    return GST_OK;
+  }
   void *p = nullptr;
   GST_HIP(hipMallocAsync(&p, bytes, s));
   out->ptr = static_cast<uint8_t *>(p);
   out->async = true;
   return GST_OK;
+}
+
+// After the call's last kernel; keeps the first error of the call and of this.
+int GiveScratch(const Scratch &sc, hipStream_t s, int rc) {
+  if (sc.slot) DefaultStreamScratch::Get().Give(sc.slot);
+  const hipError_t e = sc.async ? hipFreeAsync(sc.ptr, s) : hipSuccess;
+  return rc == GST_OK && e != hipSuccess ? HipFail(e) : rc;
 }
 
 // Scratch of one decode call: [tables 4n x 8 KiB][status 4n u32][plan blob if n > 1]
@@ -386,7 +499,8 @@ CallLayout LayoutCall(const gst_header *hdrs, uint32_t n) {
 
 // n images from a staging buffer in the reference layout (codec/decoder.cpp:98-428).
 int DecodeStaging(const gst_header *hdrs, uint32_t n, hipStream_t s, const void *d_cmp, void *d_out,
-                  bool rgb, uint32_t num_init, const gst_event *init, gst_event *done) {
+                  bool rgb, uint32_t num_init, const gst_event *init, gst_event *done,
+                  KeptScratch *own = nullptr) {
   if (!hdrs || n == 0 || !d_cmp || !d_out || (num_init && !init)) return GST_ERR_INVALID_ARGUMENT;
   int rc = EnsureInit();
   if (rc != GST_OK) return rc;
@@ -403,7 +517,7 @@ int DecodeStaging(const gst_header *hdrs, uint32_t n, hipStream_t s, const void 
   const uint8_t *streams = base + offsets_bytes + 2048ull * n;
   const CallLayout L = LayoutCall(hdrs, n);
   Scratch sc;
-  if ((rc = TakeScratch(L.total, s, &sc)) != GST_OK) return rc;
+  if ((rc = TakeScratch(L.total, s, own, &sc)) != GST_OK) return rc;
 
   StageConfig cfg = DefaultStageConfig(rgb);
   std::vector<ImageDesc> descs(n);
@@ -441,10 +555,7 @@ int DecodeStaging(const gst_header *hdrs, uint32_t n, hipStream_t s, const void 
       rc = LaunchAll(a, grids, cfg, s);
     }
   }
-  if (sc.async) {
-    const hipError_t e = hipFreeAsync(sc.ptr, s);
-    if (rc == GST_OK && e != hipSuccess) rc = HipFail(e);
-  }
+  rc = GiveScratch(sc, s, rc);
   if (rc != GST_OK) return rc;
   if (done) {
     hipEvent_t ev;
@@ -455,9 +566,182 @@ int DecodeStaging(const gst_header *hdrs, uint32_t n, hipStream_t s, const void 
   return GST_OK;
 }
 
+class PinnedPool {
+ public:
+  static PinnedPool &Get() {
+    static PinnedPool *p = new PinnedPool;  // as the scratch pool
+    return *p;
+  }
+  hipError_t Take(size_t n, gst::PinnedBuffer *out) {
+    gst::PinnedBuffer old;
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      for (size_t i = 0; i < idle_.size(); ++i) {
+        if (idle_[i].cap < n) continue;
+        *out = idle_[i];
+        idle_.erase(idle_.begin() + i);
+        return hipSuccess;
+      }
+      if (idle_.size() == kKept) {  // all too small: the larger one takes a place
+        old = idle_.front();
+        idle_.erase(idle_.begin());
+      }
+    }
+    if (old.host) (void)hipHostFree(old.host);
+    size_t cap = size_t{1} << 18;
+    while (cap < n && cap < kKeptBytes) cap *= 2;
+    cap = std::max(cap, n);
+    void *h = nullptr, *d = nullptr;
+    hipError_t e = hipHostMalloc(&h, cap, hipHostMallocCoherent);
+    if (e == hipSuccess && (e = hipHostGetDevicePointer(&d, h, 0)) != hipSuccess) (void)hipHostFree(h);
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      return e;
+    }
+    *out = {static_cast<uint8_t *>(h), static_cast<uint8_t *>(d), cap};
+    return hipSuccess;
+  }
+  void Give(const gst::PinnedBuffer &b) {
+    if (b.cap <= kKeptBytes) {
+      std::lock_guard<std::mutex> lk(mu_);
+      if (idle_.size() < kKept) {
+        idle_.push_back(b);
+        return;
+      }
+    }
+    (void)hipHostFree(b.host);
+  }
+  void Trim() {
+    std::vector<gst::PinnedBuffer> all;
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      all.swap(idle_);
+    }
+    for (const gst::PinnedBuffer &b : all) (void)hipHostFree(b.host);
+  }
+
+ private:
+  static constexpr size_t kKept = 4, kKeptBytes = size_t{64} << 20;
+  std::mutex mu_;
+  std::vector<gst::PinnedBuffer> idle_;
+};
+
+// What a host-to-host decode needs beside pinned memory: a stream of its own with scratch
+// for it, a pinned word for the error bits and the staging buffer on the device.  Creating them all
+// took most of a call's time (a 1024x1024 file 163 us in the library, of which the GPU's
+// part is 35; with them kept 72).  At most kKept stay for later calls, each with one call
+// at a time; gst_free_decompressor gives them back.
+class HostCalls {
+ public:
+  struct Call {
+    int device = 0;
+    hipStream_t stream = nullptr;
+    uint8_t *d_cmp = nullptr;
+    size_t cmp_cap = 0;
+    KeptScratch scratch;
+    uint32_t *bits = nullptr, *bits_dev = nullptr;  // pinned error bits
+  };
+
+  static HostCalls &Get() {
+    static HostCalls *p = new HostCalls;  // as the scratch pool
+    return *p;
+  }
+
+  // Null if something could not be allocated.
+  Call *Take(size_t staging) {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return Fail(nullptr);
+    Call *c = nullptr;
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      for (size_t i = 0; i < idle_.size() && !c; ++i) {
+        if (idle_[i]->device != dev) continue;
+        c = idle_[i];
+        idle_.erase(idle_.begin() + i);
+      }
+    }
+    if (!c) {
+      c = new Call;
+      c->device = dev;
+      void *b = nullptr, *bd = nullptr;
+      if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) return Fail(c);
+      if (hipHostMalloc(&b, sizeof(uint32_t), hipHostMallocCoherent) != hipSuccess) return Fail(c);
+      c->bits = static_cast<uint32_t *>(b);
+      if (hipHostGetDevicePointer(&bd, b, 0) != hipSuccess) return Fail(c);
+      c->bits_dev = static_cast<uint32_t *>(bd);
+    }
+    if (staging > c->cmp_cap) {
+      if (c->d_cmp) (void)hipFree(c->d_cmp);
+      c->d_cmp = nullptr;
+      c->cmp_cap = 0;
+      void *d = nullptr;
+      const size_t cap = Rounded(staging);
+      if (hipMalloc(&d, cap) != hipSuccess) return Fail(c);
+      c->d_cmp = static_cast<uint8_t *>(d);
+      c->cmp_cap = cap;
+    }
+    return c;
+  }
+
+  // The call's stream is idle.  keep: nothing went wrong on it.
+  void Give(Call *c, bool keep) {
+    if (keep && c->cmp_cap <= kKeptBytes && c->scratch.bytes <= kKeptBytes * 4) {
+      std::lock_guard<std::mutex> lk(mu_);
+      if (idle_.size() < kKept) {
+        idle_.push_back(c);
+        return;
+      }
+    }
+    Destroy(c);
+  }
+
+  void Trim() {
+    std::vector<Call *> all;
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      all.swap(idle_);
+    }
+    for (Call *c : all) Destroy(c);
+  }
+
+ private:
+  static constexpr size_t kKept = 4, kKeptBytes = size_t{16} << 20;
+  static size_t Rounded(size_t n) {
+    size_t r = size_t{1} << 18;
+    while (r < n && r < kKeptBytes) r *= 2;
+    return std::max(r, n);
+  }
+  static Call *Fail(Call *c) {
+    (void)hipGetLastError();
+    if (c) Destroy(c);
+    return nullptr;
+  }
+  static void Destroy(Call *c) {
+    if (c->bits) (void)hipHostFree(c->bits);
+    if (c->scratch.ptr) (void)hipFree(c->scratch.ptr);
+    if (c->d_cmp) (void)hipFree(c->d_cmp);
+    if (c->stream) {
+      Globals &g = G();
+      std::lock_guard<std::mutex> lk(g.mu);
+      auto it = g.err_words.find(c->stream);
+      if (it != g.err_words.end()) {
+        (void)hipFree(it->second);
+        g.err_words.erase(it);
+      }
+      (void)hipStreamDestroy(c->stream);
+    }
+    delete c;
+  }
+  std::mutex mu_;
+  std::vector<Call *> idle_;
+};
+
 }  // namespace
 
 int gst::EnsureDecoderInit() { return EnsureInit(); }
+
+hipError_t gst::TakePinned(size_t bytes, PinnedBuffer *out) { return PinnedPool::Get().Take(bytes, out); }
+void gst::GivePinned(const PinnedBuffer &b) { PinnedPool::Get().Give(b); }
 
 // ---------------------------------------------------------------------------
 // C ABI
@@ -522,6 +806,9 @@ int gst_preallocate_decompressor(size_t bytes) {
 }
 
 int gst_free_decompressor(void) {
+  DefaultStreamScratch::Get().Trim();
+  HostCalls::Get().Trim();
+  PinnedPool::Get().Trim();
   Globals &g = G();
   std::lock_guard<std::mutex> lk(g.mu);
   if (g.pre_base) {
@@ -712,39 +999,43 @@ int gst_decompress_dxt(const uint8_t *file, size_t len, uint8_t *out, size_t out
   if (out_len < dxt) return GST_ERR_INVALID_ARGUMENT;
   if ((rc = EnsureInit()) != GST_OK) return rc;
   // codec/decoder.cpp:430-476: offsets block of 512 B, then the file minus its header.
-  const size_t body = sizeof(gst_header) + 2048 + StreamBytes(h) - sizeof(gst_header);
-  std::vector<uint8_t> staging(512 + body, 0);
+  const size_t staging = 512 + 2048 + StreamBytes(h);
+  HostCalls::Call *c = HostCalls::Get().Take(staging);
+  if (!c) return GST_ERR_OUT_OF_MEMORY;
+  const size_t out_at = AlignUp(staging, kAlign);
+  gst::PinnedBuffer pin;  // [staging][blocks]
+  hipError_t e = gst::TakePinned(out_at + dxt, &pin);
+  if (e != hipSuccess) {
+    HostCalls::Get().Give(c, true);
+    return HipFail(e);
+  }
   const uint8_t *const files[1] = {file};
   const size_t lens[1] = {len};
-  if ((rc = gst_pack_staging(files, lens, 1, staging.data(), staging.size())) != GST_OK) return rc;
-  hipStream_t s = nullptr;
-  GST_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
-  void *d_cmp = nullptr, *d_out = nullptr;
-  hipError_t e = hipMalloc(&d_cmp, staging.size());
-  if (e == hipSuccess) e = hipMalloc(&d_out, dxt);
-  if (e == hipSuccess) e = hipMemcpyAsync(d_cmp, staging.data(), staging.size(), hipMemcpyHostToDevice, s);
-  if (e == hipSuccess) {
-    rc = DecodeStaging(&h, 1, s, d_cmp, d_out, false, 0, nullptr, nullptr);
-    if (rc == GST_OK) e = hipMemcpyAsync(out, d_out, dxt, hipMemcpyDeviceToHost, s);
-    if (rc == GST_OK && e == hipSuccess) e = hipStreamSynchronize(s);
+  rc = gst_pack_staging(files, lens, 1, pin.host, staging);
+  uint32_t *const err = rc == GST_OK ? ErrWord(c->stream) : nullptr;
+  if (rc == GST_OK && !err) rc = GST_ERR_HIP;
+  // The file goes up by one gather launch, the blocks come back by the decode's own stores
+  // into pinned memory and the error bits by a kernel: no DMA copy, whose fixed cost is
+  // about 10 us each.
+  if (rc == GST_OK) {
+    gst::GatherArgs ga;
+    ga.n = 1;
+    ga.job[0] = {pin.dev, c->d_cmp, staging};
+    e = gst::LaunchGather(ga, c->stream);
   }
-  uint32_t bits = 0;
-  if (e == hipSuccess && rc == GST_OK) rc = gst_read_error_bits(s, &bits);
-  if (d_cmp) (void)hipFree(d_cmp);
-  if (d_out) (void)hipFree(d_out);
-  {
-    Globals &g = G();
-    std::lock_guard<std::mutex> lk(g.mu);
-    auto it = g.err_words.find(s);
-    if (it != g.err_words.end()) {
-      (void)hipFree(it->second);
-      g.err_words.erase(it);
-    }
+  if (rc == GST_OK && e == hipSuccess)
+    rc = DecodeStaging(&h, 1, c->stream, c->d_cmp, pin.dev + out_at, false, 0, nullptr, nullptr,
+                      &c->scratch);
+  if (rc == GST_OK && e == hipSuccess) e = gst::LaunchExportBits(err, c->bits_dev, c->stream);
+  const hipError_t sync = hipStreamSynchronize(c->stream);
+  if (e == hipSuccess) e = sync;
+  if (rc == GST_OK && e == hipSuccess) {
+    memcpy(out, pin.host + out_at, dxt);
+    rc = *c->bits ? GST_ERR_CORRUPT_STREAM : GST_OK;
   }
-  (void)hipStreamDestroy(s);
-  if (e != hipSuccess) return HipFail(e);
-  if (rc != GST_OK) return rc;
-  return bits ? GST_ERR_CORRUPT_STREAM : GST_OK;
+  gst::GivePinned(pin);
+  HostCalls::Get().Give(c, e == hipSuccess && (rc == GST_OK || rc == GST_ERR_CORRUPT_STREAM));
+  return e != hipSuccess ? HipFail(e) : rc;
 }
 
 }  // extern "C"
@@ -923,7 +1214,8 @@ int gst_batch_create(const gst_batch_config *cfg, gst_batch **out) {
   if (e == hipSuccess) e = hipMemset(b->dmem, 0, b->scratch_off);
   if (e == hipSuccess) e = hipHostMalloc(&b->h_blob, b->blob_bytes, hipHostMallocCoherent);
   if (e == hipSuccess) e = hipHostGetDevicePointer(&b->h_blob_dev, b->h_blob, 0);
-  if (e == hipSuccess) e = hipEventCreateWithFlags(&b->blob_ev, hipEventDisableTiming);
+  // As in PinnedRing: the event only tells when the blob was read.
+  if (e == hipSuccess) e = hipEventCreateWithFlags(&b->blob_ev, hipEventDisableTiming | hipEventDisableSystemFence);
   if (e != hipSuccess) {
     gst_batch_destroy(b);
     return HipFail(e);

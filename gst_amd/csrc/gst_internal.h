@@ -286,8 +286,13 @@ hipError_t LaunchStage(uint32_t stage, const KernelArgs &args, uint32_t grid,
 
 // Stand-alone rANS groups (`groups` end offsets at the head of `data`, n = 1..32
 // interleaved streams each) against one packed table; out gets groups * n * 256 bytes.
+// `status` gets a word a group: 0, or 1 for a malformed end offset or final state.
 hipError_t LaunchAnsGroups(const uint32_t *table, const uint8_t *data, uint32_t data_len, uint32_t groups,
-                           uint32_t n, uint8_t *out, uint32_t *err, hipStream_t stream);
+                           uint32_t n, uint8_t *out, uint32_t *status, hipStream_t stream);
+
+// Moves a stream's error bits to pinned host memory and clears them, in stream order and
+// without a DMA copy's fixed cost.
+hipError_t LaunchExportBits(uint32_t *bits, uint32_t *host, hipStream_t stream);
 
 // Device-side comparison of decoded outputs with expected bytes: the server checks
 // every completion this way under load.  Job i sets flags[job.flag] to 1 when its
@@ -332,5 +337,16 @@ uint8_t *NoAllocScratch(int device);
 
 // The decoder library's one-time device set-up (gst_initialize_decoder(0) on first use).
 int EnsureDecoderInit();
+
+// Coherent pinned host memory that host-to-host calls pass their data through.  A few
+// buffers are kept for later calls, each with one call at a time (gst_free_decompressor
+// gives them back); allocating one takes some hundred microseconds.
+struct PinnedBuffer {
+  uint8_t *host = nullptr;
+  uint8_t *dev = nullptr;  // its address for device code
+  size_t cap = 0;
+};
+hipError_t TakePinned(size_t bytes, PinnedBuffer *out);
+void GivePinned(const PinnedBuffer &b);  // nothing reads or writes it any more
 
 }  // namespace gst

@@ -1112,15 +1112,16 @@ __global__ __launch_bounds__(kChainWaves * 64, 4) void AnsChainKernel(KernelArgs
 // table; lanes >= n never renormalise.  Words come from anywhere below the group's states
 // (a pointer that runs below the data reads zeros); every global read is range-checked
 // through a buffer resource.  Stream j of group g leaves its 256 symbols at
-// out[(g n + j) 256 ..], the last decoded first.  A malformed end offset, or a group that
-// does not end in the encoder's initial state 2^15, raises GST_DEVERR_STREAM_OFFSETS; the
-// output of a group with a malformed end offset is zeros.
+// out[(g n + j) 256 ..], the last decoded first.  status[g] is 1 for a malformed end
+// offset or a group that does not end in the encoder's initial state 2^15, else 0; the
+// output of a group with a malformed end offset is zeros.  data, out and status may be
+// pinned host memory: every chunk is read once, two chunks ahead.
 //
 // 24 groups of 32 streams: 16.3 us, where a wave per group with two LDS round trips a step
 // and the words copied to LDS two bytes a lane took 87 us.
 __global__ __launch_bounds__(kChainWaves * 64, 4) void AnsGroupsKernel(const uint32_t *table, const uint8_t *data,
                                                                        uint32_t data_len, uint32_t groups,
-                                                                       uint32_t n, uint8_t *out, uint32_t *err) {
+                                                                       uint32_t n, uint8_t *out, uint32_t *status) {
   __shared__ __align__(16) AnsChainLds lds;
   const uint32_t lane = threadIdx.x & 63, wave = Uniform(threadIdx.x >> 6);
   const uint32_t g = blockIdx.x * kChainWaves + wave;
@@ -1146,7 +1147,7 @@ __global__ __launch_bounds__(kChainWaves * 64, 4) void AnsGroupsKernel(const uin
   GPtr<uint8_t> dst = Gbl<uint8_t>(out) + static_cast<size_t>(g) * n * kSymsPerLane;
   if (!ok) {
     for (uint32_t i = 4 * lane; i < n * kSymsPerLane; i += 256) *(GPtr<uint32_t>)(dst + i) = 0;
-    if (lane == 0) atomicOr(err, kErrStreamOffsets);
+    if (lane == 0) Gbl<uint32_t>(status)[g] = 1;
     return;
   }
   u32x2 *const ring = lds.ring[wave];
@@ -1163,7 +1164,8 @@ __global__ __launch_bounds__(kChainWaves * 64, 4) void AnsGroupsKernel(const uin
   const uint32_t f = lds.tab[0].x & 0xFFFFFFu;
   const bool last = y >= kStateL ? y == kStateL
                                  : y == 0 && e.x == ((f << 5) | (lds.tab[0].x & 0xFF000000u)) && e.y == 16 * f;
-  if (__builtin_amdgcn_ballot_w64(active && !last) != 0 && lane == 0) atomicOr(err, kErrStreamOffsets);
+  const uint64_t wrong = __builtin_amdgcn_ballot_w64(active && !last);
+  if (lane == 0) Gbl<uint32_t>(status)[g] = wrong != 0 ? 1u : 0u;
 }
 
 // ---------------------------------------------------------------------------
@@ -2309,12 +2311,23 @@ uint8_t *NoAllocScratch(int device) {
   return g_scratch_ptr[device];
 }
 
+__global__ __launch_bounds__(64) void ExportBitsKernel(uint32_t *bits, uint32_t *host) {
+  if (threadIdx.x != 0) return;
+  Gbl<uint32_t>(host)[0] = Gbl<uint32_t>(bits)[0];
+  Gbl<uint32_t>(bits)[0] = 0;
+}
+
+hipError_t LaunchExportBits(uint32_t *bits, uint32_t *host, hipStream_t stream) {
+  hipLaunchKernelGGL(ExportBitsKernel, dim3(1), dim3(64), 0, stream, bits, host);
+  return hipGetLastError();
+}
+
 hipError_t LaunchAnsGroups(const uint32_t *table, const uint8_t *data, uint32_t data_len, uint32_t groups,
-                           uint32_t n, uint8_t *out, uint32_t *err, hipStream_t stream) {
+                           uint32_t n, uint8_t *out, uint32_t *status, hipStream_t stream) {
   if (groups == 0) return hipSuccess;
   if (n == 0 || n > kLanesPerGroup) return hipErrorInvalidValue;
   hipLaunchKernelGGL(AnsGroupsKernel, dim3((groups + kChainWaves - 1) / kChainWaves), dim3(kChainWaves * 64), 0,
-                     stream, table, data, data_len, groups, n, out, err);
+                     stream, table, data, data_len, groups, n, out, status);
   return hipGetLastError();
 }
 

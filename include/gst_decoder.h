@@ -121,7 +121,11 @@ size_t gst_required_scratch_mem(const gst_header *hdr);
  * codec/decoder.cpp:478-485).  With a preallocation, decodes carve their scratch
  * from it in call order until FreeDecompressor (as the reference's bump allocator);
  * without one (or when it is used up) each decode takes stream-ordered scratch
- * that is released on its stream after the last kernel. */
+ * that is released on its stream after the last kernel, except on the default stream,
+ * where up to 2 pieces of at most 256 MiB a device are kept for the next calls.
+ * gst_free_decompressor also gives back these and what host-to-host calls keep: up to 4
+ * streams with at most 16 MiB of staging and 64 MiB of scratch each, and up to 4 pinned
+ * buffers of at most 64 MiB. */
 int gst_preallocate_decompressor(size_t bytes);
 int gst_free_decompressor(void);
 
