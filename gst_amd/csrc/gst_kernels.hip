@@ -895,8 +895,10 @@ __device__ __forceinline__ void StoreChainChunk(const u32x2 *tab, u32x2 *ring, u
 // puts the previous step's symbol (bits 24-31 of `last`) into `acc`.  One block in a fixed
 // order: the address chain first, what fits behind it while the read is in flight, and
 // the wait (left to the compiler a step took 135 cycles, this way 123; a read of either
-// entry under its own exec mask, without the address select, also 135).  LDS addresses are those
-// of AnsChainLds at address 0, the kernel's only LDS object.
+// entry under its own exec mask, without the address select, also 135).  Two instructions
+// stand between the compare and the first vector read of its vcc_lo, the wait states that
+// this chip asks for and that nothing checks inside the block.  LDS addresses are those of
+// AnsChainLds at address 0, the kernel's only LDS object.
 template <bool kInsert>
 __device__ __forceinline__ u32x2 ChainStep(const uint32_t &y, uint32_t thr, uint32_t &q, uint32_t &mul,
                                            uint32_t last, uint32_t &acc, uint32_t sel) {
@@ -906,8 +908,8 @@ __device__ __forceinline__ u32x2 ChainStep(const uint32_t &y, uint32_t thr, uint
 #define GST_CHAIN_ADDRESS                          \
   "v_cmp_lt_u32 vcc, %[y], %[thr]\n\t"             \
   "v_lshlrev_b32 %[slot], 3, %[y]\n\t"             \
-  "v_mbcnt_lo_u32_b32 %[rank], vcc_lo, 0\n\t"      \
   "v_and_b32 %[slot], 0x3ff8, %[slot]\n\t"         \
+  "v_mbcnt_lo_u32_b32 %[rank], vcc_lo, 0\n\t"      \
   "v_lshl_add_u32 %[rank], %[rank], 3, %[q]\n\t"   \
   "v_cndmask_b32 %[slot], %[slot], %[rank], vcc\n\t" \
   "ds_read_b64 %[e], %[slot]\n\t"
