@@ -267,7 +267,7 @@ __global__ __launch_bounds__(256) void BuildTableKernel(KernelArgs a) {
 // with that stream's table resident in LDS in the 4-byte packed form BuildTableKernel
 // writes (one random LDS read per step: random table reads are where the LDS bank
 // conflicts come from; 8 KiB per table, so a 4-wave work-group with its rings takes
-// 16 KiB).  The state update is one v_mad_u32_u24 after two bit-field extracts.  With
+// 18.5 KiB).  The state update is one v_mad_u32_u24 after two bit-field extracts.  With
 // GPW = 2 a wave carries two 32-stream groups, one per half-wave; each lane holds
 // one stream's state.  The reference's local-memory renormalisation mask
 // (atomic_or / popcount / atomic_and between barriers) becomes one ballot: a lane
@@ -279,10 +279,10 @@ __global__ __launch_bounds__(256) void BuildTableKernel(KernelArgs a) {
 // serial chain of a step only touches LDS.  Chunk c covers stream words
 // [256c, 256c + 256) and lives at ring slot c & 1.  With `top` the chunk holding the
 // half's pointer - 1, chunks top and top-1 are resident and chunks top-2 and top-3
-// are in flight in registers.  A step moves the pointer by at most 32 words, so 8
-// steps read only chunks top and top-1; every 8 steps, if the pointer has dropped
-// below 256*top, chunk top-2 is written over top's slot, top-3 moves up and top-4 is
-// requested, which then has at least 16 steps to arrive.  Stream loads go through a
+// are in flight in registers.  A step moves the pointer by at most 32 words, so 4
+// steps read only chunks top and top-1; every 4 steps, if the pointer has dropped
+// below 256*top, chunk top-2 is written over top's slot and top-4 is requested, which
+// then has at least 16 steps to arrive.  Stream loads go through a
 // buffer resource bounded by the stream length (corrupt offsets read zeros, never
 // fault); a pointer that ends below the group's first byte raises kErrStreamOffsets.
 // Each lane packs 64 symbols into 16 registers and writes them as one 64-byte sector,
@@ -290,6 +290,17 @@ __global__ __launch_bounds__(256) void BuildTableKernel(KernelArgs a) {
 // Index-stream groups also emit
 // the sum of (symbol - 128) per group and per lane, the totals the index scan
 // starts from.
+//
+// VALU issue bounds it where every SIMD holds several waves: 128 images (11,040 groups, five
+// or six waves a SIMD) spend 314 cycles a step and wave, 58 a wave's own VALU, after a
+// prologue of 11,000 cycles (20,000 when the streams come from HBM).
+
+// readfirstlane returns a signed int: every use converts through uint32_t so no
+// 64-bit widening can sign-extend a value with bit 31 set.
+__device__ __forceinline__ uint32_t Uniform(uint32_t v) {
+  return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v)));
+}
+
 // LDS written by some lanes of a wave and read by others: the wave's LDS operations
 // complete in order, so only the compiler needs a fence.
 __device__ __forceinline__ void WaveSync() {
@@ -301,6 +312,12 @@ __device__ __forceinline__ void WaveSync() {
 constexpr uint32_t kChunkWords = 256;
 constexpr uint32_t kRingWords = 2 * kChunkWords;
 constexpr uint32_t kRefillSteps = kChunkWords / kLanesPerGroup;  // 8
+// The ring is checked every 4 steps, which read at most 128 words; below its first chunk
+// stands a copy of the last 128 words of its second, so that they are consecutive downwards
+// from any pointer and addresses need no wrap.
+constexpr uint32_t kCheckSteps = 4;
+constexpr uint32_t kRingBelow = kCheckSteps * kLanesPerGroup;
+constexpr uint32_t kRingAlloc = kRingBelow + kRingWords;
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
@@ -317,8 +334,88 @@ __device__ __forceinline__ u32x2 LoadChunk(__amdgpu_buffer_rsrc_t rs, uint32_t c
   return __builtin_amdgcn_raw_buffer_load_b64(rs, static_cast<int>((c * kChunkWords + 4 * l) * 2), 0, 0);
 }
 
-__device__ __forceinline__ void StoreChunk(uint16_t *ring, uint32_t c, uint32_t l, const u32x2 &a) {
-  *reinterpret_cast<u32x2 *>(ring + ((c * kChunkWords + 4 * l) & (kRingWords - 1))) = a;
+// (Odd chunks also leave their last 128 words below the ring: the upper lanes there, the
+// others once more where they are.)
+__device__ __forceinline__ void StoreChunk(uint16_t *ring, bool odd, uint32_t l, const u32x2 &a) {
+  *reinterpret_cast<u32x2 *>(ring + kRingBelow + (odd ? kChunkWords : 0u) + 4 * l) = a;
+  if (odd)
+    *reinterpret_cast<u32x2 *>(ring + 4 * l + (4 * l >= kChunkWords - kRingBelow ? kRingBelow - kChunkWords
+                                                                               : kRingBelow + kChunkWords)) = a;
+}
+
+// A local object's LDS address as the instructions take it.
+template <typename T>
+__device__ __forceinline__ uint32_t LdsAddress(T *p) {
+  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) void *)p));
+}
+
+// One step of a wave's two groups: the table read at slot x & 2047, the update, the
+// pointers, and the next word for the lanes below their threshold.  Symbols are bits 24-31
+// of the entry it returns; while the table read is in flight the step puts earlier ones
+// into `acc`: the last two at once (kIns 1, `first` the earlier) or the last one (kIns 2).
+//
+// pA and pB are the halves' pointers as LDS word addresses.  An upper lane's word is at
+// pB' plus its rank in its half, that is rank - tlo + pB', and pA' = pA - tlo, so the two
+// halves' addresses are rank + pA' and rank + pA' + (pB' - pA): one v_mad with the half `h`.
+//
+// Written out because the loop is bound by issue (six waves a SIMD hide the latencies): the
+// compare writes the lane mask, so the renormalisation is one v_lshl_or under it, and lanes
+// that keep their state need no select.  12.75 VALU and 6 SALU a step, where the compiler's
+// form, with selects, a wrap per lane and a masked add, had 15.6 and 5: the stage of 128
+// images 64.8 -> 62.4 us with inputs from HBM (25.8 -> 21.0 M VALU).
+template <int kIns>
+__device__ __forceinline__ uint32_t AnsStep(uint32_t &x, uint32_t thr, uint32_t tab_at, uint32_t h, uint64_t lanes,
+                                            uint32_t &pA, uint32_t &pB, uint32_t first, uint32_t last, uint32_t &acc,
+                                            uint32_t sel) {
+  uint32_t fs;
+#if defined(__HIP_DEVICE_COMPILE__)
+  uint32_t t, r, a, b;
+#define GST_ANS_TABLE                               \
+  "v_and_b32 %[t], 0x7ff, %[x]\n\t"                 \
+  "v_lshl_add_u32 %[t], %[t], 2, %[tab]\n\t"        \
+  "ds_read_b32 %[fs], %[t]\n\t"                     \
+  "v_lshrrev_b32 %[x], 11, %[x]\n\t"
+#define GST_ANS_UPDATE                              \
+  "s_waitcnt lgkmcnt(0)\n\t"                        \
+  "v_and_b32 %[t], 0xfff, %[fs]\n\t"                \
+  "v_bfe_u32 %[r], %[fs], 12, 11\n\t"               \
+  "v_mad_u32_u24 %[x], %[x], %[t], %[r]\n\t"        \
+  "v_cmpx_lt_u32 vcc, %[x], %[thr]\n\t"             \
+  "s_bcnt1_i32_b32 %[a], vcc_lo\n\t"                \
+  "s_bcnt1_i32_b32 %[b], vcc_hi\n\t"                \
+  "v_mbcnt_lo_u32_b32 %[t], vcc_lo, 0\n\t"           \
+  "s_sub_u32 %[pB], %[pB], %[b]\n\t"                \
+  "s_sub_u32 %[b], %[pB], %[pA]\n\t"                \
+  "v_mbcnt_hi_u32_b32 %[t], vcc_hi, %[t]\n\t"       \
+  "s_sub_u32 %[pA], %[pA], %[a]\n\t"                \
+  "v_mad_i32_i24 %[t], %[h], %[b], %[t]\n\t"        \
+  "v_add_lshl_u32 %[t], %[t], %[pA], 1\n\t"         \
+  "ds_read_u16 %[t], %[t]\n\t"                      \
+  "s_waitcnt lgkmcnt(0)\n\t"                        \
+  "v_lshl_or_b32 %[x], %[x], 16, %[t]\n\t"          \
+  "s_mov_b64 exec, %[lanes]"
+#define GST_ANS_OUT                                                                                           \
+  [x] "+v"(x), [fs] "=&v"(fs), [t] "=&v"(t), [r] "=&v"(r), [a] "=&s"(a), [b] "=&s"(b), [pA] "+s"(pA), [pB] "+s"(pB)
+#define GST_ANS_IN                                                                                             \
+  [thr] "v"(thr), [tab] "s"(tab_at), [h] "v"(h), [lanes] "s"(lanes)
+  if constexpr (kIns == 0)
+    asm volatile(GST_ANS_TABLE GST_ANS_UPDATE : GST_ANS_OUT : GST_ANS_IN : "vcc", "scc", "memory");
+  else if constexpr (kIns == 1)
+    asm volatile(GST_ANS_TABLE "v_perm_b32 %[acc], %[first], %[last], %[sel]\n\t" GST_ANS_UPDATE
+                 : GST_ANS_OUT, [acc] "=&v"(acc)
+                 : GST_ANS_IN, [first] "v"(first), [last] "v"(last), [sel] "s"(sel)
+                 : "vcc", "scc", "memory");
+  else
+    asm volatile(GST_ANS_TABLE "v_perm_b32 %[acc], %[last], %[acc], %[sel]\n\t" GST_ANS_UPDATE
+                 : GST_ANS_OUT, [acc] "+v"(acc)
+                 : GST_ANS_IN, [last] "v"(last), [sel] "s"(sel)
+                 : "vcc", "scc", "memory");
+#undef GST_ANS_TABLE
+#undef GST_ANS_UPDATE
+#undef GST_ANS_OUT
+#undef GST_ANS_IN
+#endif
+  return fs;
 }
 
 // The first two chunks of each half's ring (top and top-1, top = the chunk holding
@@ -377,25 +474,31 @@ __device__ __forceinline__ void TouchStreamTail(__amdgpu_buffer_rsrc_t rs, uint3
 }
 
 template <bool kSum, uint32_t GPW>
-__device__ __forceinline__ void DecodeHalfGroups(const uint32_t *tab, uint16_t *ring_wave, uint16_t *ring_half,
-                                                 uint32_t *sink, __amdgpu_buffer_rsrc_t rs, AnsRing ring,
-                                                 uint32_t lane,
-                                                 bool active, uint32_t x, uint32_t pA, uint32_t pB,
+__device__ __forceinline__ void DecodeHalfGroups(const uint32_t *tab, uint16_t *ring_wave, uint32_t *sink,
+                                                 __amdgpu_buffer_rsrc_t rs, AnsRing ring, uint32_t lane, bool active, uint32_t x, uint32_t pA, uint32_t pB,
                                                  uint32_t loA, uint32_t loB, GPtr<uint8_t> outp,
                                                  GPtr<int32_t> group_sum, GPtr<int32_t> lane_sum,
                                                  GPtr<int32_t> lane_suffix, uint32_t *err) {
   const uint32_t j = lane & 31;
-  uint32_t upper = lane < 32 ? 0u : 0xFFFFFFFFu;
-  asm volatile("" : "+v"(upper));  // keep the half-wave mask an opaque VGPR (one v_and below)
   // Renormalisation threshold per lane: L for a lane with a stream, 0 (never) for one
-  // without, so the compare's mask is already the renormalising lanes and neither the
-  // ballot nor the select needs a scalar AND with the active lanes.
+  // without, so the compare's mask is already the renormalising lanes.
   uint32_t thr = active ? kStateL : 0u;
   asm volatile("" : "+v"(thr));
   uint16_t *const ringA = ring_wave;
-  uint16_t *const ringB = ring_wave + kRingWords;
+  uint16_t *const ringB = ring_wave + kRingAlloc;
+  const uint32_t tab_at = Uniform(LdsAddress(tab));
+  // Word addresses of the two rings' first chunks, and from here on the pointers and the
+  // start of the chunk each is in.
+  const uint32_t slotA = Uniform(LdsAddress(ringA)) / 2 + kRingBelow, slotB = slotA + kRingAlloc;
+  const uint32_t mostA = pA - loA, mostB = pB - loB;
   uint32_t topA = ring.topA, topB = ring.topB;
-  const uint32_t startA = pA, startB = pB;  // a pointer above its start has wrapped below 0
+  uint32_t limA = slotA + (topA & 1u) * kChunkWords, limB = slotB + (topB & 1u) * kChunkWords;
+  const uint32_t startA = pA, startB = pB;
+  pA += limA - topA * kChunkWords;
+  pB += limB - topB * kChunkWords;
+  uint32_t h = lane >> 5;
+  asm volatile("" : "+v"(h));
+  const uint64_t lanes = __builtin_amdgcn_read_exec();
   // Chunks top-2 and top-3 go in flight in two fixed registers by chunk parity (even
   // chunks in pXE, odd in pXO): a load lands in the register its chunk is later
   // stored from, so no register moves sit between in-flight loads.  The wait before a
@@ -411,11 +514,11 @@ __device__ __forceinline__ void DecodeHalfGroups(const uint32_t *tab, uint16_t *
     pBO = LoadChunk(rs, (topB & 1u) ? topB - 2 : topB - 3, cloB, lane);
   }
   TouchStreamTail(rs, lane < 32 ? topA : topB, 2u * (lane < 32 ? loA : loB), j, sink);
-  StoreChunk(ringA, topA, lane, ring.rA0);
-  StoreChunk(ringA, topA - 1, lane, ring.rA1);
+  StoreChunk(ringA, (topA & 1u) != 0, lane, ring.rA0);
+  StoreChunk(ringA, (topA & 1u) == 0, lane, ring.rA1);
   if (GPW == 2) {
-    StoreChunk(ringB, topB, lane, ring.rB0);
-    StoreChunk(ringB, topB - 1, lane, ring.rB1);
+    StoreChunk(ringB, (topB & 1u) != 0, lane, ring.rB0);
+    StoreChunk(ringB, (topB & 1u) == 0, lane, ring.rB1);
   }
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
@@ -436,82 +539,64 @@ __device__ __forceinline__ void DecodeHalfGroups(const uint32_t *tab, uint16_t *
       case 2: __builtin_amdgcn_s_setprio(1); break;
       default: __builtin_amdgcn_s_setprio(0); break;
     }
-    uint32_t acc[16], first = 0;
+    uint32_t acc[16], first = 0, last = 0, none = 0;
 #pragma unroll
     for (uint32_t blk = 0; blk < 64 / kRefillSteps; ++blk) {
 #pragma unroll
       for (uint32_t s = 0; s < kRefillSteps; ++s) {
-        // One LDS read per step: e = f | (slot - cum) << 12 | symbol << 24.
-        const uint32_t fs = tab[x & (kTableSize - 1)];
-        x = __umul24(x >> kTableLog, fs & 0xFFFu) + __builtin_amdgcn_ubfe(fs, 12, 11);
-        const bool need = x < thr;
-        const uint64_t m = __builtin_amdgcn_uicmp(x, thr, 36 /* ULT */);
-        const uint32_t mlo = static_cast<uint32_t>(m), mhi = static_cast<uint32_t>(m >> 32);
-        const uint32_t tlo = __popc(mlo), thi = __popc(mhi);
-        pA -= tlo;
-        pB -= thi;
-        {
-          // Word index p_half + rank: mbcnt over both halves counts the lower half's
-          // bits for upper lanes, so upper lanes start from pB - tlo.  The rank needs
-          // only the ballot, so it runs beside the scalar pointer updates; one
-          // three-operand add joins them.  Every lane reads (a lane that keeps its
-          // state reads a word of the ring it never uses) and a select on the ballot
-          // keeps the new state: no exec-mask round trip through the scalar unit.
-          const uint32_t rank = __builtin_amdgcn_mbcnt_hi(mhi, __builtin_amdgcn_mbcnt_lo(mlo, 0u));
-          const uint32_t widx = rank + pA + (upper & (pB - tlo - pA));
-          const uint32_t xn = (x << 16) | ring_half[widx & (kRingWords - 1)];
-          x = need ? xn : x;
+        // Step 8*blk + s decodes byte 63 - 8*blk - s of the sector, the last first; byte
+        // `at` is the step before's.  v_perm: selector codes 4-7 take bytes of the first
+        // operand, 0-3 bytes of the second, 0x0c is zero.
+        const uint32_t at = 64 - kRefillSteps * blk - s;
+        uint32_t fs;
+        if (at == 64 || (at & 3) == 3)
+          fs = AnsStep<0>(x, thr, tab_at, h, lanes, pA, pB, 0u, 0u, none, 0u);
+        else if ((at & 3) == 2)
+          fs = AnsStep<1>(x, thr, tab_at, h, lanes, pA, pB, first, last, acc[at >> 2], 0x07030C0Cu);
+        else
+          fs = AnsStep<2>(x, thr, tab_at, h, lanes, pA, pB, 0u, last, acc[at >> 2],
+                          (at & 3) == 1 ? 0x0302070Cu : 0x03020107u);
+        first = last;
+        last = fs;
+        // The pointers moved at most 128 words since the last check, so each crossed at most
+        // one chunk's start, and the next 4 steps read only chunks top and top-1 (top =
+        // chunk of pointer - 1).  Per crossed half (uniform branches, all 64 lanes): store
+        // chunk top-2 from the register of its parity, request chunk top-4 (same parity)
+        // into it, and from the first chunk's copy below move on to the second.
+        if ((s + 1) % kCheckSteps == 0 && static_cast<int32_t>((pA - limA) | (pB - limB)) < 0) {
+          const bool crossA = pA < limA, crossB = pB < limB;
+          const bool oddA = (topA & 1u) != 0, oddB = (topB & 1u) != 0;
+          if (crossA && oddA) {
+            StoreChunk(ringA, true, lane, pAO);
+            asm volatile("" ::: "memory");
+            pAO = LoadChunk(rs, topA - 4, cloA, lane);
+          }
+          if (crossA && !oddA) {
+            StoreChunk(ringA, false, lane, pAE);
+            asm volatile("" ::: "memory");
+            pAE = LoadChunk(rs, topA - 4, cloA, lane);
+          }
+          if (GPW == 2 && crossB && oddB) {
+            StoreChunk(ringB, true, lane, pBO);
+            asm volatile("" ::: "memory");
+            pBO = LoadChunk(rs, topB - 4, cloB, lane);
+          }
+          if (GPW == 2 && crossB && !oddB) {
+            StoreChunk(ringB, false, lane, pBE);
+            asm volatile("" ::: "memory");
+            pBE = LoadChunk(rs, topB - 4, cloB, lane);
+          }
+          pA += crossA && !oddA ? kRingWords : 0u;
+          pB += crossB && !oddB ? kRingWords : 0u;
+          limA = crossA ? slotA + (oddA ? 0u : kChunkWords) : limA;
+          limB = crossB ? slotB + (oddB ? 0u : kChunkWords) : limB;
+          topA -= crossA ? 1u : 0u;
+          topB -= crossB ? 1u : 0u;
+          WaveSync();
         }
-        // Step 8*blk + s lands at byte 63 - 8*blk - s of the sector, the last decoded first.
-        // The symbol (byte 3 of fs) goes in with v_perm: selector codes 4-7 take bytes of
-        // the first operand, 0-3 bytes of the second, 0x0c is zero; the first two of a word
-        // go in together.
-        const uint32_t pos = 63 - kRefillSteps * blk - s;
-        if ((pos & 3) == 3) {
-          first = fs;
-        } else {
-          if ((pos & 3) == 2)
-            acc[pos >> 2] = __builtin_amdgcn_perm(first, fs, 0x07030C0Cu);
-          else
-            acc[pos >> 2] = __builtin_amdgcn_perm(fs, acc[pos >> 2], (pos & 3) == 1 ? 0x0302070Cu : 0x03020107u);
-          asm volatile("" : "+v"(acc[pos >> 2]));  // insert now: keeps 64 symbols out of VGPRs
-        }
-      }
-      // Ring refill at the 8-step boundary: the pointer moved at most 256 words, so it
-      // crossed at most one chunk boundary, and the next 8 steps read only chunks
-      // top and top-1 (top = chunk of pointer - 1).
-      const bool crossA = pA < topA * kChunkWords, crossB = pB < topB * kChunkWords;
-      // Per crossed half (uniform branches, all 64 lanes): store chunk top-2 from the
-      // register of its parity and request chunk top-4 (same parity) into it.
-      const bool oddA = (topA & 1u) != 0, oddB = (topB & 1u) != 0;
-      if (crossA && oddA) {
-        StoreChunk(ringA, topA - 2, lane, pAO);
-        asm volatile("" ::: "memory");
-        pAO = LoadChunk(rs, topA - 4, cloA, lane);
-      }
-      if (crossA && !oddA) {
-        StoreChunk(ringA, topA - 2, lane, pAE);
-        asm volatile("" ::: "memory");
-        pAE = LoadChunk(rs, topA - 4, cloA, lane);
-      }
-      if (GPW == 2 && crossB && oddB) {
-        StoreChunk(ringB, topB - 2, lane, pBO);
-        asm volatile("" ::: "memory");
-        pBO = LoadChunk(rs, topB - 4, cloB, lane);
-      }
-      if (GPW == 2 && crossB && !oddB) {
-        StoreChunk(ringB, topB - 2, lane, pBE);
-        asm volatile("" ::: "memory");
-        pBE = LoadChunk(rs, topB - 4, cloB, lane);
-      }
-      topA -= crossA ? 1u : 0u;
-      topB -= crossB ? 1u : 0u;
-      if (crossA || crossB) {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
       }
     }
+    acc[0] = __builtin_amdgcn_perm(last, acc[0], 0x03020107u);
     if (kSum) {
       // Byte sums of the sector's two 32-symbol halves (v_sad_u8 against zero), less
       // the biases.  The sector covers lane positions 192 - 64 sector + [0, 64), so
@@ -535,7 +620,10 @@ __device__ __forceinline__ void DecodeHalfGroups(const uint32_t *tab, uint16_t *
         dst[i] = make_uint4(acc[4 * i], acc[4 * i + 1], acc[4 * i + 2], acc[4 * i + 3]);
     }
   }
-  const bool under = lane < 32 ? (pA < loA || pA > startA) : (pB < loB || pB > startB);
+  // Words each group consumed (modulo 2^32: at most 2^13), against those it has.
+  const uint32_t usedA = startA - (topA * kChunkWords + (pA - limA));
+  const uint32_t usedB = startB - (topB * kChunkWords + (pB - limB));
+  const bool under = lane < 32 ? usedA > mostA : usedB > mostB;
   if (active && under && j == 0) atomicOr(err, kErrStreamOffsets);
   if (kSum) {
     // Inclusive prefix of the lane totals over the half-wave's 32 lanes.
@@ -549,12 +637,6 @@ __device__ __forceinline__ void DecodeHalfGroups(const uint32_t *tab, uint16_t *
     const int32_t total = __shfl(incl, 31, 32);
     if (active && j == 0) *group_sum = total;
   }
-}
-
-// readfirstlane returns a signed int: every use converts through uint32_t so no
-// 64-bit widening can sign-extend a value with bit 31 set.
-__device__ __forceinline__ uint32_t Uniform(uint32_t v) {
-  return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v)));
 }
 
 // Work-groups are dispatched to the 8 XCDs round robin (group b on XCD b % 8), each XCD
@@ -689,14 +771,14 @@ struct AnsLdsSmall {
 template <uint32_t WAVES, bool kPair>
 struct AnsLds {
   uint32_t tab[kPair ? 2 : 1][kTableSize];
-  uint16_t ring[WAVES][2][kRingWords];
+  uint16_t ring[WAVES][2][kRingAlloc];
 };
 
 template <uint32_t WAVES, uint32_t GPW, bool kBuild, bool kPair>
 __device__ __forceinline__ void AnsDecodeUnits(const KernelArgs &a, AnsLds<WAVES, kPair> &L,
                                                AnsLdsSmall &S) {
   static_assert(!kPair || (kBuild && WAVES % 2 == 0), "paired units build their tables in LDS");
-  static_assert(!kBuild || WAVES * 2 * kRingWords * 2 >= 4 * kBuildScratchWords, "build scratch fits the rings");
+  static_assert(!kBuild || WAVES * 2 * kRingAlloc * 2 >= 4 * kBuildScratchWords, "build scratch fits the rings");
   auto &tab = L.tab;
   auto &ring = L.ring;
   uint32_t *const build_scratch = reinterpret_cast<uint32_t *>(&ring[0][0][0]);
@@ -749,8 +831,8 @@ __device__ __forceinline__ void AnsDecodeUnits(const KernelArgs &a, AnsLds<WAVES
     const uint32_t plo = active ? lo >> 1 : 0u;
     const uint32_t pA = __builtin_amdgcn_readlane(p, 0);
     const uint32_t loA = __builtin_amdgcn_readlane(plo, 0);
-    const uint32_t pB = GPW == 2 ? __builtin_amdgcn_readlane(p, 32) : 0u;
-    const uint32_t loB = GPW == 2 ? __builtin_amdgcn_readlane(plo, 32) : 0u;
+    const uint32_t pB = __builtin_amdgcn_readlane(p, 32);  // 0 with one group a wave
+    const uint32_t loB = __builtin_amdgcn_readlane(plo, 32);
     const AnsRing chunks = RequestRing<GPW>(rs, pA, pB, loA, loB, lane);
 
     LdsBarrier();  // every wave is done with the previous unit's tables and rings
@@ -778,16 +860,15 @@ __device__ __forceinline__ void AnsDecodeUnits(const KernelArgs &a, AnsLds<WAVES
     if (__builtin_amdgcn_ballot_w64(active) == 0) continue;
     const uint32_t *const tw = tab[kPair ? seg : 0];
     const GPtr<uint8_t> outp = d.symbols + SymbolOffset(d, k) + static_cast<size_t>(g) * kGroupSyms + j * kSymsPerLane;
-    uint16_t *ring_half = ring[wave][half];
     if (k == 3)
-      DecodeHalfGroups<true, GPW>(tw, ring[wave][0], ring_half, touch_sink, rs, chunks, lane, active, x, pA, pB,
+      DecodeHalfGroups<true, GPW>(tw, ring[wave][0], touch_sink, rs, chunks, lane, active, x, pA, pB,
                                   loA, loB, outp, d.group_sums + g,
                                   d.lane_sums ? d.lane_sums + g * kLanesPerGroup : nullptr,
                                   d.lane_sums ? d.lane_sums + LaneSuffixBase(d.nv) + g * kLanesPerGroup * 8
                                               : nullptr,
                                   a.err);
     else
-      DecodeHalfGroups<false, GPW>(tw, ring[wave][0], ring_half, touch_sink, rs, chunks, lane, active, x, pA, pB,
+      DecodeHalfGroups<false, GPW>(tw, ring[wave][0], touch_sink, rs, chunks, lane, active, x, pA, pB,
                                    loA, loB, outp, nullptr, nullptr, nullptr, a.err);
   }
 }
