@@ -76,9 +76,8 @@ __host__ __device__ inline uint32_t TileRowOf(uint32_t t, uint32_t tile_mul) {
 constexpr uint32_t kRowBlocks = 32;
 __host__ __device__ inline uint32_t LaneSuffixBase(uint32_t nv) { return nv / kSymsPerLane; }
 
-template <typename Desc>
-__host__ __device__ inline uint32_t SymbolOffset(const Desc &d, uint32_t k) {
-  return k == 0 ? 0u : k == 1 ? 2 * d.nv : k == 2 ? 6 * d.nv : 6 * d.nv + d.palette_bytes;
+__host__ __device__ inline uint32_t SymbolOffset(uint32_t nv, uint32_t palette_bytes, uint32_t k) {
+  return k == 0 ? 0u : k == 1 ? 2 * nv : k == 2 ? 6 * nv : 6 * nv + palette_bytes;
 }
 
 // rANS work units.  A unit is up to `per` consecutive groups of one stream (per = waves
@@ -162,24 +161,28 @@ __host__ __device__ inline uint32_t ChainUnitsOf(const Desc &d) {
   return u;
 }
 
-// Unit `local` of an image with these groups per stream: stream k, groups first ..
-// first + count - 1.
-struct ChainUnit {
+// Unit `local`, of up to `per` groups of one stream, of an image with these groups per
+// stream: stream k, groups first .. first + count - 1.
+struct StreamUnit {
   uint32_t k, first, count;
 };
 
-__host__ __device__ inline ChainUnit ChainUnitAt(uint32_t g0, uint32_t g1, uint32_t g2, uint32_t g3,
-                                                 uint32_t local) {
-  const uint32_t e0 = (g0 + kChainGroups - 1) / kChainGroups, e1 = e0 + (g1 + kChainGroups - 1) / kChainGroups;
-  const uint32_t e2 = e1 + (g2 + kChainGroups - 1) / kChainGroups;
-  ChainUnit r;
+__host__ __device__ inline StreamUnit StreamUnitAt(uint32_t per, uint32_t g0, uint32_t g1, uint32_t g2, uint32_t g3,
+                                                   uint32_t local) {
+  const uint32_t e0 = (g0 + per - 1) / per, e1 = e0 + (g1 + per - 1) / per, e2 = e1 + (g2 + per - 1) / per;
+  StreamUnit r;
   r.k = (local >= e0 ? 1u : 0u) + (local >= e1 ? 1u : 0u) + (local >= e2 ? 1u : 0u);
   const uint32_t start = local >= e2 ? e2 : local >= e1 ? e1 : local >= e0 ? e0 : 0u;
   const uint32_t groups = local >= e2 ? g3 : local >= e1 ? g2 : local >= e0 ? g1 : g0;
-  r.first = kChainGroups * (local - start);
-  r.count = groups - r.first < kChainGroups ? groups - r.first : kChainGroups;
+  r.first = per * (local - start);
+  r.count = groups - r.first < per ? groups - r.first : per;
   return r;
 }
+
+// What AnsUnitAt reads of a descriptor.
+struct AnsGroupCounts {
+  uint32_t groups[4];
+};
 
 // `ans_unit_code`: groups per rANS unit, with kAnsPairShort when short remainders pair up.
 __host__ __device__ inline uint32_t StageUnitsOf(const ImageDesc &d, uint32_t stage,

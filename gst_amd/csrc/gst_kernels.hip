@@ -70,6 +70,10 @@ __device__ __forceinline__ Located LocateIn(const uint32_t (&v)[4], uint32_t u) 
     at[k] = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v[k]), static_cast<int>(lo & 63)));
     after[k] = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v[k]), static_cast<int>(cnt & 63)));
   }
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("" : "+s"(at[0]), "+s"(at[1]), "+s"(at[2]), "+s"(at[3]), "+s"(after[0]), "+s"(after[1]),
+               "+s"(after[2]), "+s"(after[3]));
+#endif
   const uint32_t next = cnt < kPrefixInRegs ? Pick4(after, cnt >> 6) : kPrefixPad;
   return {lo, u - Pick4(at, lo >> 6), next != kPrefixPad};
 }
@@ -791,32 +795,44 @@ __device__ __forceinline__ void AnsDecodeUnits(const KernelArgs &a, AnsLds<WAVES
   for (uint32_t u = blockIdx.x;; u += gridDim.x) {
     const Located loc = Locate(a, kStageAns, u, kUnitCode);
     if (!loc.valid) break;
-    const DevDesc d = LoadDesc(a, loc.img);
-    const AnsUnit unit = AnsUnitAt(d, kUnitCode, Uniform(loc.local));
-    // This wave's segment: the unit's only one, or its half of a pair.
-    const uint32_t seg = kPair && unit.pair && wave >= WAVES / 2 ? 1u : 0u;
-    const uint32_t k = Uniform(seg ? unit.k[1] : unit.k[0]);
-    const uint32_t first = Uniform(seg ? unit.first[1] : unit.first[0]);
-    const uint32_t count = Uniform(seg ? unit.count[1] : unit.count[0]);
-    const uint32_t gi = (kPair && unit.pair ? wave % (WAVES / 2) : wave) * GPW + half;
-    const uint32_t G = Uniform(Pick4(d.groups, k));
+    // Scalar loads by index in two trips, the group counts and then the fields of the
+    // unit's stream: no selects over a descriptor in registers.
+    const CPtr<ImageDesc> d = DescAt(a, loc.img);
+    const AnsGroupCounts counts = {{d->groups[0], d->groups[1], d->groups[2], d->groups[3]}};
+    uint32_t k, first, count, k2 = 0, gi = wave * GPW + half, seg = 0;
+    bool second = false;
+    uint32_t k_first;
+    if constexpr (kPair) {
+      const AnsUnit unit = AnsUnitAt(counts, kUnitCode, Uniform(loc.local));
+      // This wave's segment: the unit's only one, or its half of a pair.
+      seg = unit.pair && wave >= WAVES / 2 ? 1u : 0u;
+      k = Uniform(seg ? unit.k[1] : unit.k[0]);
+      first = Uniform(seg ? unit.first[1] : unit.first[0]);
+      count = Uniform(seg ? unit.count[1] : unit.count[0]);
+      if (unit.pair) gi = (wave % (WAVES / 2)) * GPW + half;
+      second = unit.pair && unit.count[1] != 0;
+      k_first = unit.k[0];
+      k2 = unit.k[1];
+    } else {
+      const StreamUnit unit =
+          StreamUnitAt(kGroupsPerUnit, counts.groups[0], counts.groups[1], counts.groups[2], counts.groups[3], loc.local);
+      k = k_first = unit.k;
+      first = unit.first;
+      count = unit.count;
+    }
+    const uint32_t G = d->groups[k], slen = d->stream_len[k];
     const uint32_t g = first + gi;
-    const uint32_t slen = Uniform(Pick4(d.stream_len, k));
-    const __amdgpu_buffer_rsrc_t rs = MakeRsrc(Uniform(Pick4(d.streams, k)), slen);
+    const __amdgpu_buffer_rsrc_t rs = MakeRsrc(d->streams[k], slen);
     // Straight-line loads (out-of-range offsets read zeros): a load under a branch
     // makes the wait for it land at the join, after later loads have gone out.
     const uint32_t end = __builtin_amdgcn_raw_buffer_load_b32(rs, static_cast<int>(4 * g), 0, 0);
     const uint32_t lo_word = __builtin_amdgcn_raw_buffer_load_b32(rs, static_cast<int>(4 * (g - 1)), 0, 0);
     // Frequencies of the unit's table(s): thread t brings symbol t's.
     uint32_t f = 0, f2 = 0;
-    const bool second = kPair && unit.pair && unit.count[1] != 0;
     if constexpr (kBuild) {
-      const GPtr<const uint16_t> fr = Gbl<const uint16_t>(Uniform(d.freqs + 512 * unit.k[0]));
-      f = fr[threadIdx.x & 255];
-      if (kPair && second) {
-        const GPtr<const uint16_t> fr2 = Gbl<const uint16_t>(Uniform(d.freqs + 512 * unit.k[1]));
-        f2 = fr2[threadIdx.x & 255];
-      }
+      const GPtr<const uint16_t> fr = Gbl<const uint16_t>(d->freqs);
+      f = fr[256 * k_first + (threadIdx.x & 255)];
+      if (kPair && second) f2 = fr[256 * k2 + (threadIdx.x & 255)];
     }
     const uint32_t lo = g == 0 ? 4 * G : lo_word;
     const bool ok = ((end | lo) & 3) == 0 && end <= slen && lo >= 4 * G && lo <= end &&
@@ -846,7 +862,7 @@ __device__ __forceinline__ void AnsDecodeUnits(const KernelArgs &a, AnsLds<WAVES
       if (kPair && second)
         table_ok = BuildTableInLds<WAVES * 64>(f2, build_scratch, put(tab[kPair ? 1 : 0])) && table_ok;
     } else {
-      const uint32_t tix = Uniform(d.table_base + k);
+      const uint32_t tix = d->table_base + k;
       const GPtr<const uint32_t> src = Gbl<const uint32_t>(a.tables + static_cast<size_t>(tix) * kTableSize);
       for (uint32_t i = threadIdx.x; i < kTableSize; i += WAVES * 64) tab[0][i] = src[i];
       table_ok = Gbl<const uint32_t>(a.table_status)[tix] != 0;
@@ -859,17 +875,17 @@ __device__ __forceinline__ void AnsDecodeUnits(const KernelArgs &a, AnsLds<WAVES
     // that do.  It goes straight to the next unit's barrier.
     if (__builtin_amdgcn_ballot_w64(active) == 0) continue;
     const uint32_t *const tw = tab[kPair ? seg : 0];
-    const GPtr<uint8_t> outp = d.symbols + SymbolOffset(d, k) + static_cast<size_t>(g) * kGroupSyms + j * kSymsPerLane;
-    if (k == 3)
-      DecodeHalfGroups<true, GPW>(tw, ring[wave][0], touch_sink, rs, chunks, lane, active, x, pA, pB,
-                                  loA, loB, outp, d.group_sums + g,
-                                  d.lane_sums ? d.lane_sums + g * kLanesPerGroup : nullptr,
-                                  d.lane_sums ? d.lane_sums + LaneSuffixBase(d.nv) + g * kLanesPerGroup * 8
-                                              : nullptr,
-                                  a.err);
-    else
-      DecodeHalfGroups<false, GPW>(tw, ring[wave][0], touch_sink, rs, chunks, lane, active, x, pA, pB,
-                                   loA, loB, outp, nullptr, nullptr, nullptr, a.err);
+    const GPtr<uint8_t> outp = Gbl<uint8_t>(d->symbols + SymbolOffset(d->nv, d->palette_bytes, k)) +
+                               static_cast<size_t>(g) * kGroupSyms + j * kSymsPerLane;
+    if (k == 3) {
+      const GPtr<int32_t> sums = Gbl<int32_t>(d->lane_sums);
+      DecodeHalfGroups<true, GPW>(tw, ring[wave][0], touch_sink, rs, chunks, lane, active, x, pA, pB, loA, loB, outp,
+                                  Gbl<int32_t>(d->group_sums) + g, sums ? sums + g * kLanesPerGroup : nullptr,
+                                  sums ? sums + LaneSuffixBase(d->nv) + g * kLanesPerGroup * 8 : nullptr, a.err);
+    } else {
+      DecodeHalfGroups<false, GPW>(tw, ring[wave][0], touch_sink, rs, chunks, lane, active, x, pA, pB, loA, loB, outp,
+                                   nullptr, nullptr, nullptr, a.err);
+    }
   }
 }
 
@@ -1131,7 +1147,7 @@ __global__ __launch_bounds__(kChainWaves * 64, 4) void AnsChainKernel(KernelArgs
     const Located loc = Locate(a, kStageChain, w, 0);
     if (!loc.valid) break;
     const CPtr<ImageDesc> d = DescAt(a, loc.img);
-    const ChainUnit unit = ChainUnitAt(d->groups[0], d->groups[1], d->groups[2], d->groups[3], loc.local);
+    const StreamUnit unit = StreamUnitAt(kChainGroups, d->groups[0], d->groups[1], d->groups[2], d->groups[3], loc.local);
     const uint32_t k = unit.k, g = unit.first + wave;
     const uint32_t G = d->groups[k], slen = d->stream_len[k], nv = d->nv;
     const __amdgpu_buffer_rsrc_t rs = MakeRsrc(d->streams[k], slen);
@@ -1166,8 +1182,7 @@ __global__ __launch_bounds__(kChainWaves * 64, 4) void AnsChainKernel(KernelArgs
     StoreChainChunk(lds.tab, ring, kChunkWords, false, lane, c1);
     WaveSync();
     const uint32_t ring_at = sizeof(lds.tab) + wave * sizeof(lds.ring[0]);
-    const uint32_t at = k == 0 ? 0u : k == 1 ? 2 * nv : k == 2 ? 6 * nv : 6 * nv + d->palette_bytes;
-    const GPtr<uint8_t> outp = Gbl<uint8_t>(d->symbols + at) + static_cast<size_t>(g) * kGroupSyms;
+    const GPtr<uint8_t> outp = Gbl<uint8_t>(d->symbols + SymbolOffset(nv, d->palette_bytes, k)) + static_cast<size_t>(g) * kGroupSyms;
     uint32_t y = x, q, used;
     if (k == 3) {
       const GPtr<int32_t> sums = Gbl<int32_t>(d->lane_sums);
@@ -1276,7 +1291,7 @@ __global__ __launch_bounds__(256) void DecodeIndicesKernel(KernelArgs a) {
       if (lane == 0) gprefix = s;
     }
     const GPtr<const uint4> diffs =
-        (GPtr<const uint4>)(d.symbols + SymbolOffset(d, 3) + static_cast<size_t>(g) * kGroupSyms + 32 * t);
+        (GPtr<const uint4>)(d.symbols + SymbolOffset(d.nv, d.palette_bytes, 3) + static_cast<size_t>(g) * kGroupSyms + 32 * t);
     const uint4 q0 = diffs[0];
     const uint4 q1 = diffs[1];
     const uint32_t words[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
@@ -1637,7 +1652,7 @@ __global__ __launch_bounds__(256) void AssembleDxtKernel(KernelArgs a) {
     for (int p = 0; p < 6; ++p)
       pw[p] = *(GPtr<const uint32_t>)(d.planes + static_cast<size_t>(p) * nv + b0);
     const int4 ix = *(GPtr<const int4>)(d.indices + b0);
-    const GPtr<const uint32_t> pal = (GPtr<const uint32_t>)(d.symbols + SymbolOffset(d, 2));
+    const GPtr<const uint32_t> pal = (GPtr<const uint32_t>)(d.symbols + SymbolOffset(d.nv, d.palette_bytes, 2));
     const uint32_t words = d.palette_bytes / 4;
     const int idx[4] = {ix.x, ix.y, ix.z, ix.w};
     uint32_t o[8];
@@ -1696,8 +1711,8 @@ __global__ __launch_bounds__(WAVES * 64) void AssembleFusedKernel(KernelArgs a) 
     int32_t base = 0;
     for (uint32_t i = lane; i < g; i += 64) base += d.group_sums[i];
     base = WaveSum64(base) + GroupLocalPrefix(d, b0);
-    const GPtr<const uint8_t> diffs = d.symbols + SymbolOffset(d, 3);
-    const GPtr<const uint32_t> pal = (GPtr<const uint32_t>)(d.symbols + SymbolOffset(d, 2));
+    const GPtr<const uint8_t> diffs = d.symbols + SymbolOffset(d.nv, d.palette_bytes, 3);
+    const GPtr<const uint32_t> pal = (GPtr<const uint32_t>)(d.symbols + SymbolOffset(d.nv, d.palette_bytes, 2));
     const uint32_t words = d.palette_bytes / 4;
     bool bad = false;
 #pragma unroll
@@ -1761,7 +1776,7 @@ __global__ __launch_bounds__(WAVES * 64) void AssembleFusedWideKernel(KernelArgs
     const uint32_t nv = d.nv;
     const uint32_t b0 = loc.local * kAssembleBlocksPerUnit;
     const uint32_t blk = b0 + kPerLane * lane;
-    const uint4 dv = *(GPtr<const uint4>)(d.symbols + SymbolOffset(d, 3) + blk);
+    const uint4 dv = *(GPtr<const uint4>)(d.symbols + SymbolOffset(d.nv, d.palette_bytes, 3) + blk);
     uint4 pv[6];
 #pragma unroll
     for (int p = 0; p < 6; ++p)
@@ -1784,7 +1799,7 @@ __global__ __launch_bounds__(WAVES * 64) void AssembleFusedWideKernel(KernelArgs
       if (lane >= static_cast<uint32_t>(off)) incl += n;
     }
     const int32_t before = base + incl - acc;
-    const GPtr<const uint32_t> pal = (GPtr<const uint32_t>)(d.symbols + SymbolOffset(d, 2));
+    const GPtr<const uint32_t> pal = (GPtr<const uint32_t>)(d.symbols + SymbolOffset(d.nv, d.palette_bytes, 2));
     const uint32_t words = d.palette_bytes / 4;
     bool bad = false;
     const GPtr<uint4> dst = (GPtr<uint4>)(d.out + 8 * static_cast<size_t>(blk));
@@ -2138,7 +2153,7 @@ __global__ __launch_bounds__(256) void AssembleRgbKernel(KernelArgs a) {
     for (int p = 0; p < 6; ++p)
       pw[p] = *(GPtr<const uint32_t>)(d.planes + static_cast<size_t>(p) * nv + b0);
     const int4 ix = *(GPtr<const int4>)(d.indices + b0);
-    const GPtr<const uint32_t> pal = (GPtr<const uint32_t>)(d.symbols + SymbolOffset(d, 2));
+    const GPtr<const uint32_t> pal = (GPtr<const uint32_t>)(d.symbols + SymbolOffset(d.nv, d.palette_bytes, 2));
     const uint32_t words = d.palette_bytes / 4;
     const int idx[4] = {ix.x, ix.y, ix.z, ix.w};
     bool bad = false;
