@@ -945,12 +945,18 @@ __global__ __launch_bounds__(kAutoWaves * 64, 6) void AnsAutoKernel(KernelArgs a
 // times the popcount while the read is in flight; each 8 steps it is compared with the
 // chunk's end, and a crossing writes the chunk requested two crossings earlier.
 //
-// A step is bound by that chain: 123 cycles with the refills, about 52 of them the LDS read,
-// against some 280 in AnsAutoKernel (two LDS round trips, 12 dependent VALU, two scalar
-// hops).  Stage times, this kernel against AnsAutoKernel: one 512x512 image 16.9 / 33.0 us,
+// A step is bound by that chain: 101 cycles, about 52 of them the LDS read, and 440 a refill
+// (133 a step with an index stream's 13 refills), against some 280 in AnsAutoKernel (two LDS
+// round trips, 12 dependent VALU, two scalar hops).  Stage times, this kernel against
+// AnsAutoKernel when it came in, at 123 cycles a step: one 512x512 image 16.9 / 33.0 us,
 // 1024x1024 images by the dozen: 8 (480 groups) 21.6 / 35.4, 34 (2,040) 28.7 / 39.8, 68
 // (4,080, four waves a SIMD) 34.5 / 44.1.  LDS holds four work-groups a CU; a second pass
 // loses the gain (4,620 groups: 43.5 / 44.5; 7,200: 55.0 / 48.8).
+//
+// With the four steps of a symbol word in one block and one test a ring check: one 4096x4096
+// image 21.8 -> 21.0 us, 24 images 24.3 -> 23.1, 16 512x512 images 20.3 -> 19.4, 24 groups of
+// AnsGroupsKernel 20.8 -> 19.4 (three sets of inputs in turn).  16 steps a loop iteration
+// instead of 64, for a quarter of the code, was slower: 27,900 -> 29,200 cycles a group.
 constexpr uint32_t kChainWaves = kChainGroups;
 constexpr uint32_t kChainRing = 3 * kChunkWords;  // entries per wave
 
@@ -971,9 +977,8 @@ __device__ __forceinline__ void StoreChainChunk(const u32x2 *tab, u32x2 *ring, u
   for (uint32_t k = 0; k < 4; ++k) e[k] = tab[word[k] & (kTableSize - 1)];
 #pragma unroll
   for (uint32_t k = 0; k < 4; ++k) {
-    const uint32_t f = e[k].x & 0xFFFFFFu;
-    const uint32_t lo = (f << 5) | (e[k].x & 0xFF000000u);
-    const uint32_t hi = __umul24(word[k] >> kTableLog, f) + e[k].y;
+    const uint32_t lo = __builtin_amdgcn_perm(e[k].x, e[k].x << 5, 0x07020100u);  // 32 f, the symbol on top
+    const uint32_t hi = __umul24(word[k] >> kTableLog, e[k].x) + e[k].y;
     const uint32_t pos = 3 - k;
     o[pos >> 1][(pos & 1) * 2] = lo;
     o[pos >> 1][(pos & 1) * 2 + 1] = hi;
@@ -987,52 +992,48 @@ __device__ __forceinline__ void StoreChainChunk(const u32x2 *tab, u32x2 *ring, u
   }
 }
 
-// The reading half of a step: the lane's entry {multiplier | symbol << 24, addend} and the
-// state's multiplicand `mul`; moves q past the words the wave's lanes take, and (kInsert)
-// puts the previous step's symbol (bits 24-31 of `last`) into `acc`.  One block in a fixed
-// order: the address chain first, what fits behind it while the read is in flight, and
-// the wait (left to the compiler a step took 135 cycles, this way 123; a read of either
-// entry under its own exec mask, without the address select, also 135).  Two instructions
-// stand between the compare and the first vector read of its vcc_lo, the wait states that
-// this chip asks for and that nothing checks inside the block.  LDS addresses are those of
-// AnsChainLds at address 0, the kernel's only LDS object.
-template <bool kInsert>
-__device__ __forceinline__ u32x2 ChainStep(const uint32_t &y, uint32_t thr, uint32_t &q, uint32_t &mul,
-                                           uint32_t last, uint32_t &acc, uint32_t sel) {
-  u32x2 e;
+// Four steps, whose symbols are the returned word (the first in byte 3): moves the state y,
+// and q past the words the wave's lanes take.  `thr0` is the first step's threshold.
+//
+// One block in a fixed order: the address chain first, what fits behind it while the read is
+// in flight, the wait, the update, and the symbol's insertion where the update's latency
+// would idle.  (A step left to the compiler took 135 cycles, a block a step 123, of which a
+// wait state that the compiler puts behind every block and the 18 scalar instructions of a
+// ring check; see DecodeGroupChain.  A read of either entry under its own exec mask, without
+// the address select, also took 135.)  Two instructions stand between the compare and the
+// first vector read of its vcc_lo, the wait states that this chip asks for and that nothing
+// checks inside the block.  LDS addresses are those of AnsChainLds at address 0, the
+// kernel's only LDS object; the entry is in fixed registers because its halves have no name
+// otherwise.
+__device__ __forceinline__ uint32_t ChainSteps(uint32_t &y, uint32_t thr0, uint32_t thr, uint32_t &q) {
+  uint32_t word = 0;
 #if defined(__HIP_DEVICE_COMPILE__)
-  uint32_t slot, rank, moved;
-#define GST_CHAIN_ADDRESS                          \
-  "v_cmp_lt_u32 vcc, %[y], %[thr]\n\t"             \
-  "v_lshlrev_b32 %[slot], 3, %[y]\n\t"             \
-  "v_and_b32 %[slot], 0x3ff8, %[slot]\n\t"         \
-  "v_mbcnt_lo_u32_b32 %[rank], vcc_lo, 0\n\t"      \
-  "v_lshl_add_u32 %[rank], %[rank], 3, %[q]\n\t"   \
-  "v_cndmask_b32 %[slot], %[slot], %[rank], vcc\n\t" \
-  "ds_read_b64 %[e], %[slot]\n\t"
-#define GST_CHAIN_BEHIND                           \
-  "v_lshrrev_b32 %[mul], 11, %[y]\n\t"             \
-  "s_bcnt1_i32_b32 %[moved], vcc_lo\n\t"           \
-  "v_cndmask_b32 %[mul], %[mul], %[y], vcc\n\t"    \
-  "s_lshl_b32 %[moved], %[moved], 3\n\t"           \
-  "s_add_u32 %[q], %[q], %[moved]\n\t"             \
-  "s_waitcnt lgkmcnt(0)"
-  if constexpr (kInsert)
-    asm volatile(GST_CHAIN_ADDRESS "v_perm_b32 %[acc], %[last], %[acc], %[sel]\n\t" GST_CHAIN_BEHIND
-                 : [e] "=&v"(e), [slot] "=&v"(slot), [rank] "=&v"(rank), [mul] "=&v"(mul), [q] "+s"(q),
-                   [moved] "=&s"(moved), [acc] "+v"(acc)
-                 : [y] "v"(y), [thr] "v"(thr), [last] "v"(last), [sel] "s"(sel)
-                 : "vcc", "scc", "memory");
-  else
-    asm volatile(GST_CHAIN_ADDRESS GST_CHAIN_BEHIND
-                 : [e] "=&v"(e), [slot] "=&v"(slot), [rank] "=&v"(rank), [mul] "=&v"(mul), [q] "+s"(q),
-                   [moved] "=&s"(moved)
-                 : [y] "v"(y), [thr] "v"(thr)
-                 : "vcc", "scc", "memory");
-#undef GST_CHAIN_ADDRESS
-#undef GST_CHAIN_BEHIND
+  uint32_t slot, rank, mul, moved;
+#define GST_CHAIN_STEP(THR, INSERT)                    \
+  "v_cmp_lt_u32 vcc, %[y], " THR "\n\t"                \
+  "v_lshlrev_b32 %[slot], 3, %[y]\n\t"                 \
+  "v_and_b32 %[slot], 0x3ff8, %[slot]\n\t"             \
+  "v_mbcnt_lo_u32_b32 %[rank], vcc_lo, 0\n\t"          \
+  "v_lshl_add_u32 %[rank], %[rank], 3, %[q]\n\t"       \
+  "v_cndmask_b32 %[slot], %[slot], %[rank], vcc\n\t"   \
+  "ds_read_b64 v[120:121], %[slot]\n\t"                \
+  "v_lshrrev_b32 %[mul], 11, %[y]\n\t"                 \
+  "s_bcnt1_i32_b32 %[moved], vcc_lo\n\t"               \
+  "v_cndmask_b32 %[mul], %[mul], %[y], vcc\n\t"        \
+  "s_lshl3_add_u32 %[q], %[moved], %[q]\n\t"           \
+  "s_waitcnt lgkmcnt(0)\n\t"                           \
+  "v_mad_u32_u24 %[y], %[mul], v120, v121\n\t" INSERT "\n\t"
+  asm volatile(GST_CHAIN_STEP("%[thr0]", "v_mov_b32 %[word], v120")
+               GST_CHAIN_STEP("%[thr]", "v_perm_b32 %[word], v120, %[word], %[s2]")
+               GST_CHAIN_STEP("%[thr]", "v_perm_b32 %[word], v120, %[word], %[s1]")
+               GST_CHAIN_STEP("%[thr]", "v_perm_b32 %[word], v120, %[word], %[s0]")
+               : [y] "+v"(y), [q] "+s"(q), [word] "=&v"(word), [slot] "=&v"(slot), [rank] "=&v"(rank),
+                 [mul] "=&v"(mul), [moved] "=&s"(moved)
+               : [thr0] "v"(thr0), [thr] "v"(thr), [s2] "s"(0x03070100u), [s1] "s"(0x03020700u), [s0] "s"(0x03020107u)
+               : "vcc", "scc", "memory", "v120", "v121");
+#undef GST_CHAIN_STEP
 #endif
-  return e;
+  return word;
 }
 
 // One group of n <= 32 streams: lanes 0 .. n - 1 decode streams n - 1 .. 0 from state y,
@@ -1058,51 +1059,34 @@ __device__ __forceinline__ uint32_t DecodeGroupChain(const AnsChainLds &lds, u32
   uint32_t limit = end0, wraps = 0;
   int32_t sum = 0;
   for (uint32_t sector = 0; sector < kSymsPerLane / 64; ++sector) {
-    uint32_t acc[16], last = 0, none = 0;
+    uint32_t acc[16];
 #pragma unroll
-    for (uint32_t i = 0; i < 16; ++i) acc[i] = 0;
-#pragma unroll
-    for (uint32_t blk = 0; blk < 64 / kRefillSteps; ++blk) {
-#pragma unroll
-      for (uint32_t s = 0; s < kRefillSteps; ++s) {
-        // The last step's symbol goes in while this step's read is in flight: byte `at` of
-        // the sector (the first step's has no predecessor in it).
-        const uint32_t at = 64 - kRefillSteps * blk - s;
-        const uint32_t sel = (0x03020100u & ~(0xFFu << (8 * (at & 3)))) | (7u << (8 * (at & 3)));
-        uint32_t mul;
-        u32x2 e;
-        if (at == 64)
-          e = ChainStep<false>(y, thr, q, mul, 0u, none, sel);
-        else
-          e = ChainStep<true>(y, thr, q, mul, last, acc[at >> 2], sel);
-        y = __umul24(mul, e.x) + e.y;
-        last = e.x;
-        if (at == 64) thr = full;
-        if (s == kRefillSteps - 1) {
-          // 8 steps read at most 256 words, so at most one chunk's end was crossed.  Two
-          // uniform branches, not an if/else, so that each request stays in its register.
-          const bool cross0 = q >= limit && limit == end0, cross1 = q >= limit && limit == end1;
-          if (cross0) {
-            StoreChainChunk(lds.tab, ring, 0, true, lane, pE);
-            asm volatile("" ::: "memory");
-            pE = LoadChunk(rs, top - 4, clo, lane);
-            limit = end1;
-            --top;
-          }
-          if (cross1) {
-            StoreChainChunk(lds.tab, ring, kChunkWords, false, lane, pO);
-            asm volatile("" ::: "memory");
-            pO = LoadChunk(rs, top - 4, clo, lane);
-            limit = end0;
-            --top;
-            q -= 16 * kChunkWords;
-            ++wraps;
-          }
-          WaveSync();
+    for (uint32_t w = 0; w < 16; ++w) {
+      acc[15 - w] = ChainSteps(y, thr, full, q);
+      thr = full;
+      // 8 steps read at most 256 words, so at most one chunk's end was crossed.  One test
+      // on the way past (two scalar instructions; both cases' tests there took 18, 100
+      // cycles of each 8 steps), and behind it two uniform branches, not an if/else, so that
+      // each request stays in its register.
+      if (w % 2 == 1 && __builtin_expect(q >= limit, 0)) {
+        const bool first = limit == end0, second = limit == end1;
+        if (first) {
+          StoreChainChunk(lds.tab, ring, 0, true, lane, pE);
+          asm volatile("" ::: "memory");
+          pE = LoadChunk(rs, top - 4, clo, lane);
         }
+        if (second) {
+          StoreChainChunk(lds.tab, ring, kChunkWords, false, lane, pO);
+          asm volatile("" ::: "memory");
+          pO = LoadChunk(rs, top - 4, clo, lane);
+          q -= 16 * kChunkWords;
+          ++wraps;
+        }
+        limit = first ? end1 : end0;
+        --top;
+        WaveSync();
       }
     }
-    acc[0] = __builtin_amdgcn_perm(last, acc[0], 0x03020107u);
     if (kSum) {
       // As in DecodeHalfGroups: the sector's suffix sums from 32-symbol steps.
       uint32_t lo = 0, hi = 0;
@@ -1124,13 +1108,15 @@ __device__ __forceinline__ uint32_t DecodeGroupChain(const AnsChainLds &lds, u32
     }
   }
   if (kSum) {
-    // Inclusive prefix over the 32 streams, which run down the lanes.
-    int32_t incl = sum;
-#pragma unroll
-    for (uint32_t off = 1; off < 32; off <<= 1) {
-      const int32_t n_below = __shfl_down(incl, off, 32);
-      if (j >= off) incl += n_below;
-    }
+    // Inclusive prefix over the 32 streams, which run down the lanes: within each row of 16
+    // by DPP row shifts, then the upper row's total to the lower.
+    uint32_t v = static_cast<uint32_t>(sum);
+    v = DppAdd<0x101, 0xF>(v);  // row_shl:1, 2, 4, 8
+    v = DppAdd<0x102, 0xF>(v);
+    v = DppAdd<0x104, 0xF>(v);
+    v = DppAdd<0x108, 0xF>(v);
+    const uint32_t upper = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), 16));
+    const int32_t incl = static_cast<int32_t>(lane < 16 ? v + upper : v);
     if (active && lane_sum) lane_sum[j] = incl;
     if (lane == 0) *group_sum = incl;
   }
@@ -1253,12 +1239,13 @@ __global__ __launch_bounds__(kChainWaves * 64, 4) void AnsGroupsKernel(const uin
   StoreChainChunk(lds.tab, ring, kChunkWords, false, lane, c1);
   WaveSync();
   const bool active = lane < n;
-  uint32_t y = active ? x : 0u, q, mul, unused = 0;
-  DecodeGroupChain<false>(lds, ring, sizeof(lds.tab) + wave * sizeof(lds.ring[0]), rs, lane, n, y, q, p, 0, pE, pO,
-                          dst, nullptr, nullptr, nullptr);
+  uint32_t y = active ? x : 0u, q;
+  const uint32_t ring_at = sizeof(lds.tab) + wave * sizeof(lds.ring[0]);
+  DecodeGroupChain<false>(lds, ring, ring_at, rs, lane, n, y, q, p, 0, pE, pO, dst, nullptr, nullptr, nullptr);
   // The final state is 2^15: y itself, or y = 0 renormalised with the word 2^15, which its
   // ring entry tells from every other word (slot 0, 16 above it: an rANS step is one to one).
-  const u32x2 e = ChainStep<false>(y, active ? kStateL : 0u, q, mul, 0u, unused, 0u);
+  const uint64_t ends = __builtin_amdgcn_ballot_w64(active && y < kStateL);
+  const u32x2 e = ring[(q - ring_at) / 8 + __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(ends), 0u)];
   const uint32_t f = lds.tab[0].x & 0xFFFFFFu;
   const bool last = y >= kStateL ? y == kStateL
                                  : y == 0 && e.x == ((f << 5) | (lds.tab[0].x & 0xFF000000u)) && e.y == 16 * f;
