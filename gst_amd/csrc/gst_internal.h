@@ -199,8 +199,9 @@ __host__ __device__ inline uint32_t StageUnitsOf(const ImageDesc &d, uint32_t st
 
 // Device plan for batched decodes of up to `cap` images, n of them bound: the header
 // (padded to 64 bytes), then prefix[kNumUnitKinds][cap + 1] (work units per stage and of
-// AnsChainKernel, so that either rANS kernel decodes any plan; exclusive prefix over the images; entries past index n hold 0xFFFFFFFF), then
-// ImageDesc[cap], of which the first n are used.  Every offset depends on cap alone,
+// AnsChainKernel, so that either rANS kernel decodes any plan; exclusive prefix over the
+// images; entries past index n hold 0xFFFFFFFF), then ImageDesc[cap], of which the first n
+// are used.  Every offset depends on cap alone,
 // which the kernels receive as an argument, so a kernel reads the header and the
 // prefix in one round trip; the used bytes (everything up to the n-th descriptor)
 // are one contiguous copy.
@@ -253,9 +254,9 @@ struct StageConfig {
   uint32_t fused_wide;           // fused kernel layout: 0 = 4 blocks per lane x 4 segments,
                                  // 1 = 16 consecutive blocks per lane
   uint32_t tile_fused;           // 1: the wavelet and the index scan run inside the DXT1
-                                 // assembly (two tile positions per 3-wave work-group);
+                                 // or RGB8 assembly (two tile positions per 3-wave work-group);
                                  // the wavelet and index stages launch nothing
-  uint32_t rgb;                  // 1: RGB8 assembly
+  uint32_t rgb;                  // 1: RGB8 output
 };
 
 // Work-groups that give every unit of `units` its own pass (no grid-stride repeat).

@@ -24,15 +24,11 @@ template <typename T>
 using GPtr = __attribute__((address_space(1))) T *;
 template <typename T>
 using CPtr = __attribute__((address_space(4))) const T *;
-template <typename T>
-using LPtr = __attribute__((address_space(3))) T *;
 #else
 template <typename T>
 using GPtr = T *;
 template <typename T>
 using CPtr = const T *;
-template <typename T>
-using LPtr = T *;
 #endif
 
 template <typename T, typename U>
@@ -63,7 +59,7 @@ __device__ __forceinline__ Located LocateIn(const uint32_t (&v)[4], uint32_t u) 
 #pragma unroll
   for (uint32_t k = 0; k < 4; ++k) cnt += Popc64(__builtin_amdgcn_ballot_w64(v[k] <= u));
   const uint32_t lo = cnt - 1;  // prefix[0] = 0 <= u
-  // Reads of a lane and scalar selects: no branches over the four registers.
+  // Reads of a lane and scalar selects, pinned so that the selects don't become branches.
   uint32_t at[4], after[4];
 #pragma unroll
   for (uint32_t k = 0; k < 4; ++k) {
@@ -1201,7 +1197,7 @@ __global__ __launch_bounds__(kChainWaves * 64, 4) void AnsChainKernel(KernelArgs
 // output of a group with a malformed end offset is zeros.  data, out and status may be
 // pinned host memory: every chunk is read once, two chunks ahead.
 //
-// 24 groups of 32 streams: 16.3 us, where a wave per group with two LDS round trips a step
+// 24 groups of 32 streams: 15 us, where a wave per group with two LDS round trips a step
 // and the words copied to LDS two bytes a lane took 87 us.
 __global__ __launch_bounds__(kChainWaves * 64, 4) void AnsGroupsKernel(const uint32_t *table, const uint8_t *data,
                                                                        uint32_t data_len, uint32_t groups,
@@ -1940,7 +1936,8 @@ __device__ __forceinline__ TilePair PairAt(CPtr<ImageDesc> d, uint32_t t0) {
 // of the 53 us at 4.5 waves a SIMD): pairs of planes that the conversion takes as they lie,
 // no read back of the last level's rows, addresses with a scalar base, signed dot products
 // for the running indices and the palette's range check in the buffer: 20.8 M, 49.6 us (24
-// textures 13.4, one 512x512 image 7.6 -> 7.0, 4096x4096 11.4 -> 10.3).
+// textures 13.4, one 512x512 image 7.6 -> 7.0, 4096x4096 11.4 -> 10.3); with the coarse
+// levels by all lanes (SplitPass) 19.2 M, 47.2 us (12.8, 6.7, 10.1).
 //
 // At most 96 VGPRs: 5 waves per SIMD, about what the 26 KiB of LDS allows.
 template <bool kRgb>
@@ -2008,7 +2005,11 @@ __global__ __launch_bounds__(kTileFusedWaves * 64, 5) void WaveletAssembleKernel
     int32_t gpre = 0;
     if (few_groups) {
       int32_t before = gb;
-      for (uint32_t i = lane + 64; i < g_min; i += 64) before += cur.group_sums[i];
+      if (g_min > 64) {
+        uint32_t i = lane + 64;
+        asm volatile("" : "+v"(i));  // made here: kept through the unit loop, it was spilled
+        for (; i < g_min; i += 64) before += cur.group_sums[i];
+      }
       before = static_cast<int32_t>(WaveTotal(static_cast<uint32_t>(before)));
       gpre = before + static_cast<int32_t>(WaveInclusiveSum(static_cast<uint32_t>(gs))) - gs;
     }

@@ -222,7 +222,7 @@ typedef struct gst_batch_config {
   uint32_t assembly_wide;           /* fused assembly with 16 consecutive blocks per lane
                                        (one scan per 1024 blocks) instead of 4 x 4 */
   uint32_t separate_wavelet;        /* 1: the inverse wavelet as its own launch; 0: it runs
-                                       inside the DXT1 assembly (planes stay in LDS) */
+                                       inside the assembly (planes stay in LDS) */
   uint32_t ans_form;                /* rANS kernel with 4 waves x 2 groups and tables built in
                                        LDS (the default shape): GST_ANS_FORM_* */
 } gst_batch_config;
@@ -277,7 +277,7 @@ typedef struct gst_tune_result {
   float stage_ms[5];                 /* median time of the chosen shape per stage; NaN for a
                                         stage the chosen shapes fold into another launch */
   float total_ms;
-  uint32_t wavelet_fused;            /* 1: wavelet + index scan + DXT1 assembly in one kernel */
+  uint32_t wavelet_fused;            /* 1: wavelet + index scan + assembly in one kernel */
   uint32_t ans_form;                 /* GST_ANS_FORM_PAIRED, _PLAIN or _AUTO (8-group units in
                                         the kernel that also runs PAIRED, or the kernel with a
                                         wave per group, which later binds choose again) of the
@@ -289,7 +289,7 @@ typedef struct gst_tune_result {
  * rANS streams per wavefront {32, 64} x waves per work-group {1, 2, 4, 8} x grid,
  * wavelet waves per work-group {1, 2, 4} x grid, and the index scan + assembly either
  * fused (waves per work-group {1, 2, 4} x grid) or as two launches (grid each); then
- * the wavelet inside the DXT1 assembly (grid) replaces the last three stages when it
+ * the wavelet inside the assembly (grid) replaces the last three stages when it
  * beats their sum.  The
  * bound images are decoded along the way.  Drops a captured graph
  * (capture again afterwards).  Blocking. */
