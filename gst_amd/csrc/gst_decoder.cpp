@@ -219,7 +219,17 @@ uint32_t *ErrWord(hipStream_t s) {
   if (it != g.err_words.end()) return it->second;
   uint32_t *w = nullptr;
   if (hipMalloc(&w, sizeof(uint32_t)) != hipSuccess) return nullptr;
-  if (hipMemset(w, 0, sizeof(uint32_t)) != hipSuccess) {
+  // Cleared on a stream of its own and waited for: a clear on the null stream may still be on
+  // its way when kernels of a non-blocking stream set bits, and would take them back.
+  hipStream_t clear = nullptr;
+  hipError_t e = hipStreamCreateWithFlags(&clear, hipStreamNonBlocking);
+  if (e == hipSuccess) {
+    e = hipMemsetAsync(w, 0, sizeof(uint32_t), clear);
+    const hipError_t done = hipStreamSynchronize(clear);
+    if (e == hipSuccess) e = done;
+    (void)hipStreamDestroy(clear);
+  }
+  if (e != hipSuccess) {
     (void)hipFree(w);
     return nullptr;
   }

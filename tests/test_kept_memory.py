@@ -22,7 +22,7 @@ def _threads(n, body):
     def run(i):
         try:
             body(i)
-        except Exception as e:  # reported by the test's own thread
+        except BaseException as e:  # pytest's own failures too: reported by the test's thread
             errors.append(e)
     threads = [threading.Thread(target=run, args=(i,)) for i in range(n)]
     for t in threads:
