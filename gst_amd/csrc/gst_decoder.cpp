@@ -178,10 +178,11 @@ bool AutoPairs(const ImageDesc *descs, uint32_t n) {
 }
 
 // Whether GST_ANS_FORM_AUTO takes AnsChainKernel: while its work-groups of four groups fit
-// the device in one pass (four a CU, by LDS).  Up to there it is faster throughout (one
-// image 16.9 against 33.0 us, 4,080 groups 34.5 against 44.1); with a second pass the two
-// meet (4,620 groups 43.5 against 44.5) and AnsAutoKernel, whose waves carry two groups,
-// is ahead (7,200 groups 48.8 against 55.0).
+// the device in one pass (four a CU, by LDS).  Up to there it is far ahead; a few in a second
+// pass take most of that back, and many lose, since AnsAutoKernel's waves carry two groups.
+// Batches of 1024x1024 images, us a decode with it and with AnsAutoKernel: 480 groups 26.8 /
+// 41.6, 2,040 41.0 / 53.5, 4,080 (4 a CU) 54.7 / 66.0, 4,620 64.4 / 67.8, 5,400 69.5 / 70.9,
+// 7,200 83.2 / 80.7.
 bool ChainFits(const ImageDesc *descs, uint32_t n) {
   uint64_t units = 0;
   for (uint32_t i = 0; i < n; ++i) units += gst::ChainUnitsOf(descs[i]);
