@@ -69,7 +69,8 @@ def build_encoder():
 def build_cpp_tests():
     """tests/cpp/codec_test and tests/cpp/ans_ocl_test: the reference's end-to-end decoder
     test and its ANS decoder tests against the C++ API; tests/cpp/encoder_test: the
-    encoder's C++ API; tests/cpp/ans_units_test: the rANS work-unit enumeration."""
+    encoder's C++ API; tests/cpp/ans_units_test: the rANS work-unit enumeration;
+    tests/cpp/host_runtime_test: the library's host code on a stand-in for the HIP runtime."""
     outs = []
     for name in ("codec_test", "ans_ocl_test"):
         src = os.path.join(ROOT, "tests", "cpp", name + ".cpp")
@@ -88,6 +89,12 @@ def build_cpp_tests():
     outs.append(_atomic_build(os.path.join(ROOT, "tests", "cpp", "ans_units_test"), lambda o: [
         cxx, "-std=c++17", "-O2", "-Wall", "-Wextra", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
         "-I" + CSRC, "-I" + INCLUDE, src, "-o", o]))
+    # The library's host sources without HIP or a GPU: the test brings its own runtime.
+    srcs = [os.path.join(ROOT, "tests", "cpp", "host_runtime_test.cpp")]
+    srcs += [os.path.join(CSRC, n) for n in ("gst_decoder.cpp", "gst_ans.cpp", "gst_serve.cpp")]
+    outs.append(_atomic_build(os.path.join(ROOT, "tests", "cpp", "host_runtime_test"), lambda o: [
+        cxx, "-std=c++17", "-O1", "-g", "-Wall", "-Wextra", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+        "-I" + CSRC, "-I" + INCLUDE, *srcs, "-o", o, "-lpthread"]))
     return outs
 
 

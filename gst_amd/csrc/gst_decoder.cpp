@@ -220,17 +220,7 @@ uint32_t *ErrWord(hipStream_t s) {
   if (it != g.err_words.end()) return it->second;
   uint32_t *w = nullptr;
   if (hipMalloc(&w, sizeof(uint32_t)) != hipSuccess) return nullptr;
-  // Cleared on a stream of its own and waited for: a clear on the null stream may still be on
-  // its way when kernels of a non-blocking stream set bits, and would take them back.
-  hipStream_t clear = nullptr;
-  hipError_t e = hipStreamCreateWithFlags(&clear, hipStreamNonBlocking);
-  if (e == hipSuccess) {
-    e = hipMemsetAsync(w, 0, sizeof(uint32_t), clear);
-    const hipError_t done = hipStreamSynchronize(clear);
-    if (e == hipSuccess) e = done;
-    (void)hipStreamDestroy(clear);
-  }
-  if (e != hipSuccess) {
+  if (gst::ClearAndWait(w, sizeof(uint32_t)) != hipSuccess) {
     (void)hipFree(w);
     return nullptr;
   }
@@ -751,6 +741,16 @@ class HostCalls {
 
 int gst::EnsureDecoderInit() { return EnsureInit(); }
 
+hipError_t gst::ClearAndWait(void *p, size_t n) {
+  hipStream_t s = nullptr;
+  hipError_t e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
+  if (e != hipSuccess) return e;
+  e = hipMemsetAsync(p, 0, n, s);
+  const hipError_t done = hipStreamSynchronize(s);
+  (void)hipStreamDestroy(s);
+  return e == hipSuccess ? done : e;
+}
+
 hipError_t gst::TakePinned(size_t bytes, PinnedBuffer *out) { return PinnedPool::Get().Take(bytes, out); }
 void gst::GivePinned(const PinnedBuffer &b) { PinnedPool::Get().Give(b); }
 
@@ -1222,7 +1222,7 @@ int gst_batch_create(const gst_batch_config *cfg, gst_batch **out) {
   off += b->scratch_cap;
   b->dbytes = off;
   hipError_t e = hipMalloc(&b->dmem, b->dbytes);
-  if (e == hipSuccess) e = hipMemset(b->dmem, 0, b->scratch_off);
+  if (e == hipSuccess) e = gst::ClearAndWait(b->dmem, b->scratch_off);
   if (e == hipSuccess) e = hipHostMalloc(&b->h_blob, b->blob_bytes, hipHostMallocCoherent);
   if (e == hipSuccess) e = hipHostGetDevicePointer(&b->h_blob_dev, b->h_blob, 0);
   // As in PinnedRing: the event only tells when the blob was read.

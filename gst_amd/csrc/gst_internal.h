@@ -342,6 +342,11 @@ uint8_t *NoAllocScratch(int device);
 // The decoder library's one-time device set-up (gst_initialize_decoder(0) on first use).
 int EnsureDecoderInit();
 
+// Zeroes fresh device memory on a stream of its own and waits for it.  hipMemset is queued on
+// the null stream and returns: a stream that the null stream does not order (hipStreamNonBlocking)
+// may write the memory first and lose what it wrote to the late clear.
+hipError_t ClearAndWait(void *p, size_t n);
+
 // Coherent pinned host memory that host-to-host calls pass their data through.  A few
 // buffers are kept for later calls, each with one call at a time (gst_free_decompressor
 // gives them back); allocating one takes some hundred microseconds.

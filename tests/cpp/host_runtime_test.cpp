@@ -1,0 +1,255 @@
+// The library's host code (gst_decoder.cpp, gst_ans.cpp, gst_serve.cpp) on a stand-in for the
+// HIP runtime and for the kernels' launches: what a call leaves behind it, and what it does
+// when the runtime refuses it something.  One check an argument; no GPU and no HIP library.
+//
+// The stand-in keeps device and pinned memory in ordinary memory that is never given back, so
+// no two allocations share an address.  Work on created streams is done at once; hipMemset on
+// the null stream is done as late as HIP allows: when something waits for that stream or runs
+// on it.  The "kernels" write kBlock to every output byte.
+#include <hip/hip_runtime.h>
+
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <functional>
+#include <map>
+#include <mutex>
+#include <set>
+#include <string>
+#include <vector>
+
+#include "gst_ans.h"
+#include "gst_decoder.h"
+#include "gst_internal.h"
+#include "gst_serve.h"
+
+#define CHECK(x)                                                        \
+  do {                                                                  \
+    if (!(x)) {                                                         \
+      std::printf("%s:%d: %s\n", __FILE__, __LINE__, #x);               \
+      std::exit(1);                                                     \
+    }                                                                   \
+  } while (0)
+
+namespace {
+
+constexpr uint8_t kBlock = 0x5A;
+
+struct Fake {
+  std::mutex mu;
+  std::vector<std::function<void()>> late;  // null-stream clears that were not waited for
+  std::set<void *> freed;
+  int streams = 0;
+  uint32_t raise = 0;    // error bits the next decodes set
+  uint32_t images = 0;   // images the last rANS launch found in its plan
+
+  void RunLate() {
+    std::vector<std::function<void()>> work;
+    {
+      std::lock_guard<std::mutex> lk(mu);
+      work.swap(late);
+    }
+    for (auto &w : work) w();
+  }
+  void Before(hipStream_t s) {
+    if (!s) RunLate();
+  }
+};
+Fake &F() {
+  static Fake f;
+  return f;
+}
+
+hipError_t NewMemory(void **p, size_t n) {
+  *p = std::aligned_alloc(4096, (n + 4095) / 4096 * 4096);
+  std::memset(*p, 0xA5, n);
+  return hipSuccess;
+}
+
+}  // namespace
+
+extern "C" {
+
+hipError_t hipGetDeviceCount(int *n) { *n = 1; return hipSuccess; }
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipGetDevice(int *d) { *d = 0; return hipSuccess; }
+hipError_t hipGetDeviceProperties(hipDeviceProp_t *p, int) {
+  std::memset(p, 0, sizeof(*p));
+  std::strcpy(p->gcnArchName, "gfx950:sramecc+:xnack-");
+  p->maxThreadsPerBlock = 1024;
+  p->sharedMemPerBlock = 65536;
+  p->multiProcessorCount = 256;
+  return hipSuccess;
+}
+hipError_t hipGetLastError() { return hipSuccess; }
+
+hipError_t hipMalloc(void **p, size_t n) { return NewMemory(p, n); }
+hipError_t hipFree(void *p) { F().freed.insert(p); return hipSuccess; }
+hipError_t hipMallocAsync(void **p, size_t n, hipStream_t) { return NewMemory(p, n); }
+hipError_t hipFreeAsync(void *p, hipStream_t) { F().freed.insert(p); return hipSuccess; }
+hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return NewMemory(p, n); }
+hipError_t hipHostFree(void *p) { F().freed.insert(p); return hipSuccess; }
+hipError_t hipHostGetDevicePointer(void **d, void *h, unsigned) { *d = h; return hipSuccess; }
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t *, const void *) { return hipErrorInvalidValue; }
+hipError_t hipMemGetAddressRange(hipDeviceptr_t *, size_t *, hipDeviceptr_t) { return hipErrorInvalidValue; }
+
+hipError_t hipMemset(void *p, int v, size_t n) {
+  std::lock_guard<std::mutex> lk(F().mu);
+  F().late.push_back([=] { std::memset(p, v, n); });
+  return hipSuccess;
+}
+hipError_t hipMemsetAsync(void *p, int v, size_t n, hipStream_t s) {
+  if (!s) return hipMemset(p, v, n);
+  std::memset(p, v, n);
+  return hipSuccess;
+}
+hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) {
+  F().RunLate();
+  std::memcpy(d, s, n);
+  return hipSuccess;
+}
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t st) {
+  F().Before(st);
+  std::memcpy(d, s, n);
+  return hipSuccess;
+}
+
+hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned flags) {
+  CHECK(flags == hipStreamNonBlocking);
+  *s = reinterpret_cast<hipStream_t>(static_cast<uintptr_t>(0x1000 + 16 * ++F().streams));
+  return hipSuccess;
+}
+hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t s) { F().Before(s); return hipSuccess; }
+hipError_t hipDeviceSynchronize() { F().RunLate(); return hipSuccess; }
+hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
+hipError_t hipEventCreate(hipEvent_t *e) { *e = reinterpret_cast<hipEvent_t>(0x10); return hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return hipEventCreate(e); }
+hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t s) { F().Before(s); return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventQuery(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) { *ms = 0.f; return hipSuccess; }
+hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipErrorNotSupported; }
+hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t *) { return hipErrorNotSupported; }
+hipError_t hipGraphInstantiate(hipGraphExec_t *, hipGraph_t, hipGraphNode_t *, char *, size_t) { return hipErrorNotSupported; }
+hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return hipErrorNotSupported; }
+hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
+hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
+
+}  // extern "C"
+
+namespace gst {
+
+hipError_t LaunchStage(uint32_t stage, const KernelArgs &a, uint32_t, const StageConfig &, hipStream_t s) {
+  F().Before(s);
+  if (stage == kStageAns) {
+    F().images = a.plan ? a.plan->n_images : 1;
+    *a.err |= F().raise;
+  }
+  if (stage != kStageAssemble) return hipSuccess;
+  const uint32_t n = a.plan ? a.plan->n_images : 1;
+  for (uint32_t i = 0; i < n; ++i) {
+    const ImageDesc &d = a.plan ? reinterpret_cast<const ImageDesc *>(reinterpret_cast<const uint8_t *>(a.plan) +
+                                                                      PlanImagesOffset(a.plan_cap))[i]
+                                : a.single;
+    std::memset(d.out, kBlock, 8 * static_cast<size_t>(d.nv));
+  }
+  return hipSuccess;
+}
+hipError_t LaunchAnsGroups(const uint32_t *, const uint8_t *, uint32_t, uint32_t groups, uint32_t n, uint8_t *out,
+                           uint32_t *status, hipStream_t s) {
+  F().Before(s);
+  std::memset(out, kBlock, static_cast<size_t>(groups) * n * kSymsPerLane);
+  std::memset(status, 0, 4 * static_cast<size_t>(groups));
+  return hipSuccess;
+}
+hipError_t LaunchExportBits(uint32_t *bits, uint32_t *host, hipStream_t s) {
+  F().Before(s);
+  *host = *bits;
+  *bits = 0;
+  return hipSuccess;
+}
+hipError_t LaunchGather(const GatherArgs &a, hipStream_t s) {
+  F().Before(s);
+  for (uint32_t i = 0; i < a.n; ++i) std::memcpy(a.job[i].dst, a.job[i].src, a.job[i].bytes);
+  return hipSuccess;
+}
+hipError_t LaunchCompare(const CompareArgs &, hipStream_t) { return hipSuccess; }
+hipError_t ResolveNoAllocScratch(int) { return hipSuccess; }
+uint8_t *NoAllocScratch(int) { return nullptr; }
+
+}  // namespace gst
+
+namespace {
+
+// A file of the smallest legal size whose streams hold no words (the stand-in decodes nothing).
+std::vector<uint8_t> File(uint32_t width = 128, uint32_t height = 1024) {
+  gst_header h{};
+  h.width = width;
+  h.height = height;
+  h.palette_bytes = 8192;
+  const uint32_t groups = width * height / 131072;
+  h.y_cmp_sz = 2 * groups * 132;
+  h.chroma_cmp_sz = 4 * groups * 132;
+  h.palette_sz = 132;
+  h.indices_sz = groups * 132;
+  std::vector<uint8_t> f(sizeof(h) + 2048 + h.y_cmp_sz + h.chroma_cmp_sz + h.palette_sz + h.indices_sz);
+  std::memcpy(f.data(), &h, sizeof(h));
+  return f;
+}
+
+gst_header Header(const std::vector<uint8_t> &f) {
+  gst_header h;
+  std::memcpy(&h, f.data(), sizeof(h));
+  return h;
+}
+
+hipStream_t NewStream() {
+  hipStream_t s;
+  CHECK(hipStreamCreateWithFlags(&s, hipStreamNonBlocking) == hipSuccess);
+  return s;
+}
+
+gst_batch *NewBatch(const gst_header &h) {
+  gst_batch_config c{};
+  c.capacity_images = 1;
+  c.capacity_blocks = h.width / 4 * (h.height / 4);
+  gst_batch *b = nullptr;
+  CHECK(gst_batch_create(&c, &b) == GST_OK);
+  return b;
+}
+
+void Bind(gst_batch *b, const gst_header &h, const std::vector<uint8_t> &f, std::vector<uint8_t> *out, hipStream_t s) {
+  const void *in[1] = {f.data()};
+  void *o[1] = {out->data()};
+  CHECK(gst_batch_bind(b, &h, 1, in, o, s) == GST_OK);
+}
+
+// A batch made while the null stream is busy, bound on a stream that does not wait for it.
+void BatchPlanSurvives() {
+  const auto f = File();
+  const gst_header h = Header(f);
+  std::vector<uint8_t> out(h.width * h.height / 2);
+  gst_batch *b = NewBatch(h);
+  hipStream_t s = NewStream();
+  Bind(b, h, f, &out, s);
+  F().RunLate();
+  CHECK(gst_batch_decode(b, s) == GST_OK);
+  CHECK(F().images == 1);
+  for (uint8_t v : out) CHECK(v == kBlock);
+  gst_batch_destroy(b);
+}
+
+const std::map<std::string, void (*)()> kChecks = {
+    {"batch_plan", BatchPlanSurvives},
+};
+
+}  // namespace
+
+int main(int argc, char **argv) {
+  if (argc != 2 || !kChecks.count(argv[1])) return 2;
+  kChecks.at(argv[1])();
+  std::puts("ok");
+  return 0;
+}
