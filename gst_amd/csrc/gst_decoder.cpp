@@ -228,6 +228,22 @@ uint32_t *ErrWord(hipStream_t s) {
   return w;
 }
 
+// Reads a word of error bits after the stream's work and clears it, all in the stream's own
+// order: a clear on the null stream could still be on its way when the stream's next kernels
+// set bits, and would take them back.  Waiting first refuses a stream under capture before
+// anything is recorded.
+int ReadAndClear(uint32_t *w, hipStream_t s, uint32_t *bits) {
+  GST_HIP(hipStreamSynchronize(s));
+  uint32_t got = 0;
+  hipError_t e = hipMemcpyAsync(&got, w, sizeof(uint32_t), hipMemcpyDeviceToHost, s);
+  if (e == hipSuccess) e = hipMemsetAsync(w, 0, sizeof(uint32_t), s);
+  const hipError_t done = hipStreamSynchronize(s);  // also after an error: the copy's target is on this stack
+  GST_HIP(e);
+  GST_HIP(done);
+  *bits = got;
+  return GST_OK;
+}
+
 // Pinned host staging for small descriptor uploads: slots recycled once the copy
 // that last used them has completed.
 class PinnedRing {
@@ -836,10 +852,7 @@ int gst_read_error_bits(gst_stream stream, uint32_t *bits) {
   hipStream_t s = static_cast<hipStream_t>(stream);
   uint32_t *w = ErrWord(s);
   if (!w) return GST_ERR_HIP;
-  GST_HIP(hipStreamSynchronize(s));
-  GST_HIP(hipMemcpy(bits, w, sizeof(uint32_t), hipMemcpyDeviceToHost));
-  GST_HIP(hipMemset(w, 0, sizeof(uint32_t)));
-  return GST_OK;
+  return ReadAndClear(w, s, bits);
 }
 
 int gst_read_error_bits_async(gst_stream stream, uint32_t *host_bits) {
@@ -1561,10 +1574,7 @@ int gst_batch_decode_timed(gst_batch *b, gst_stream stream, float ms[5]) {
 int gst_batch_error_bits(gst_batch *b, gst_stream stream, uint32_t *bits) {
   if (!b || !bits) return GST_ERR_INVALID_ARGUMENT;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  GST_HIP(hipStreamSynchronize(s));
-  GST_HIP(hipMemcpy(bits, b->dmem + b->err_off, sizeof(uint32_t), hipMemcpyDeviceToHost));
-  GST_HIP(hipMemset(b->dmem + b->err_off, 0, sizeof(uint32_t)));
-  return GST_OK;
+  return ReadAndClear(reinterpret_cast<uint32_t *>(b->dmem + b->err_off), s, bits);
 }
 
 int gst_batch_error_bits_async(gst_batch *b, gst_stream stream, uint32_t *host_bits) {

@@ -241,8 +241,45 @@ void BatchPlanSurvives() {
   gst_batch_destroy(b);
 }
 
+// Bits that a decode sets after they were read and cleared are there for the next read.
+void BatchErrorBitsSurvive() {
+  const auto f = File();
+  const gst_header h = Header(f);
+  std::vector<uint8_t> out(h.width * h.height / 2);
+  gst_batch *b = NewBatch(h);
+  F().RunLate();
+  hipStream_t s = NewStream();
+  Bind(b, h, f, &out, s);
+  for (uint32_t bits : {4u, 2u, 0u, 6u}) {
+    F().raise = bits;
+    CHECK(gst_batch_decode(b, s) == GST_OK);
+    F().RunLate();
+    uint32_t got = ~0u;
+    CHECK(gst_batch_error_bits(b, s, &got) == GST_OK);
+    CHECK(got == bits);
+  }
+  gst_batch_destroy(b);
+}
+
+void StreamErrorBitsSurvive() {
+  const auto f = File();
+  const gst_header h = Header(f);
+  std::vector<uint8_t> out(h.width * h.height / 2), staging(512 + f.size());
+  hipStream_t s = NewStream();
+  for (uint32_t bits : {4u, 2u, 0u, 6u}) {
+    F().raise = bits;
+    CHECK(gst_load_compressed_dxt(&h, s, staging.data(), out.data(), 0, nullptr, nullptr) == GST_OK);
+    F().RunLate();
+    uint32_t got = ~0u;
+    CHECK(gst_read_error_bits(s, &got) == GST_OK);
+    CHECK(got == bits);
+  }
+}
+
 const std::map<std::string, void (*)()> kChecks = {
     {"batch_plan", BatchPlanSurvives},
+    {"batch_error_bits", BatchErrorBitsSurvive},
+    {"stream_error_bits", StreamErrorBitsSurvive},
 };
 
 }  // namespace
