@@ -737,7 +737,7 @@ int gst_server_create(const gst_server_config *cfg, gst_server **out) {
       if (e == hipSuccess) *slot.err_host = 0;
       if (e == hipSuccess) e = hipHostMalloc(&slot.flags_host, sizeof(uint32_t) * max_images, hipHostMallocDefault);
       if (e == hipSuccess) e = hipMalloc(&slot.flags_dev, sizeof(uint32_t) * max_images);
-      if (e == hipSuccess) e = hipMemset(slot.flags_dev, 0, sizeof(uint32_t) * max_images);
+      if (e == hipSuccess) e = gst::ClearAndWait(slot.flags_dev, sizeof(uint32_t) * max_images);
       if (e == hipSuccess && !s->cfg.plain) {
         gst_batch_config bc{};
         bc.capacity_images = s->cfg.max_batch_images;

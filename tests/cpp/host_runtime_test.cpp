@@ -276,10 +276,24 @@ void StreamErrorBitsSurvive() {
   }
 }
 
+// The server's comparison flags and plans are cleared before its first request.
+void ServerLeavesNothingBehind() {
+  gst_server_config c{};
+  c.hbm_budget_bytes = 1 << 20;
+  c.host_staging_bytes = 1 << 20;
+  c.max_batch_images = 4;
+  c.max_batch_blocks = 1 << 16;
+  gst_server *s = nullptr;
+  CHECK(gst_server_create(&c, &s) == GST_OK);
+  CHECK(F().late.empty());
+  gst_server_destroy(s);
+}
+
 const std::map<std::string, void (*)()> kChecks = {
     {"batch_plan", BatchPlanSurvives},
     {"batch_error_bits", BatchErrorBitsSurvive},
     {"stream_error_bits", StreamErrorBitsSurvive},
+    {"server_flags", ServerLeavesNothingBehind},
 };
 
 }  // namespace
