@@ -161,7 +161,7 @@ int gst_ans_decode(const gst_ans_decoder *d, const uint32_t *states, uint32_t nu
     const uint32_t *const status = reinterpret_cast<const uint32_t *>(packed + status_at);
     for (uint32_t i = 0; i < n_data; ++i) err |= status[i];
   }
-  gst::GivePinned(buf);
+  gst::GivePinned(buf, s == hipSuccess);
   if (e != hipSuccess) return HipFail(e);
   return err ? GST_ERR_CORRUPT_STREAM : GST_OK;
 }

@@ -618,8 +618,8 @@ class PinnedPool {
     *out = {static_cast<uint8_t *>(h), static_cast<uint8_t *>(d), cap};
     return hipSuccess;
   }
-  void Give(const gst::PinnedBuffer &b) {
-    if (b.cap <= kKeptBytes) {
+  void Give(const gst::PinnedBuffer &b, bool keep) {
+    if (keep && b.cap <= kKeptBytes) {
       std::lock_guard<std::mutex> lk(mu_);
       if (idle_.size() < kKept) {
         idle_.push_back(b);
@@ -768,7 +768,7 @@ hipError_t gst::ClearAndWait(void *p, size_t n) {
 }
 
 hipError_t gst::TakePinned(size_t bytes, PinnedBuffer *out) { return PinnedPool::Get().Take(bytes, out); }
-void gst::GivePinned(const PinnedBuffer &b) { PinnedPool::Get().Give(b); }
+void gst::GivePinned(const PinnedBuffer &b, bool keep) { PinnedPool::Get().Give(b, keep); }
 
 // ---------------------------------------------------------------------------
 // C ABI
@@ -1057,7 +1057,7 @@ int gst_decompress_dxt(const uint8_t *file, size_t len, uint8_t *out, size_t out
     memcpy(out, pin.host + out_at, dxt);
     rc = *c->bits ? GST_ERR_CORRUPT_STREAM : GST_OK;
   }
-  gst::GivePinned(pin);
+  gst::GivePinned(pin, sync == hipSuccess);
   HostCalls::Get().Give(c, e == hipSuccess && (rc == GST_OK || rc == GST_ERR_CORRUPT_STREAM));
   return e != hipSuccess ? HipFail(e) : rc;
 }

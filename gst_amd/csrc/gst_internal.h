@@ -356,6 +356,8 @@ struct PinnedBuffer {
   size_t cap = 0;
 };
 hipError_t TakePinned(size_t bytes, PinnedBuffer *out);
-void GivePinned(const PinnedBuffer &b);  // nothing reads or writes it any more
+// keep: the wait for its stream succeeded, so nothing reads or writes it any more.  After a
+// failed wait a kernel may still be writing to it, and no other call may get it.
+void GivePinned(const PinnedBuffer &b, bool keep);
 
 }  // namespace gst

@@ -42,6 +42,8 @@ struct Fake {
   int streams = 0;
   uint32_t raise = 0;    // error bits the next decodes set
   uint32_t images = 0;   // images the last rANS launch found in its plan
+  int fail_waits = 0;    // hipStreamSynchronize fails this many times
+  void *out = nullptr;   // where the last kernel wrote its output
 
   void RunLate() {
     std::vector<std::function<void()>> work;
@@ -120,7 +122,12 @@ hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned flags) {
   return hipSuccess;
 }
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
-hipError_t hipStreamSynchronize(hipStream_t s) { F().Before(s); return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t s) {
+  F().Before(s);
+  if (F().fail_waits == 0) return hipSuccess;
+  --F().fail_waits;
+  return hipErrorUnknown;
+}
 hipError_t hipDeviceSynchronize() { F().RunLate(); return hipSuccess; }
 hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
 hipError_t hipEventCreate(hipEvent_t *e) { *e = reinterpret_cast<hipEvent_t>(0x10); return hipSuccess; }
@@ -154,6 +161,7 @@ hipError_t LaunchStage(uint32_t stage, const KernelArgs &a, uint32_t, const Stag
                                                                       PlanImagesOffset(a.plan_cap))[i]
                                 : a.single;
     std::memset(d.out, kBlock, 8 * static_cast<size_t>(d.nv));
+    F().out = d.out;
   }
   return hipSuccess;
 }
@@ -162,6 +170,7 @@ hipError_t LaunchAnsGroups(const uint32_t *, const uint8_t *, uint32_t, uint32_t
   F().Before(s);
   std::memset(out, kBlock, static_cast<size_t>(groups) * n * kSymsPerLane);
   std::memset(status, 0, 4 * static_cast<size_t>(groups));
+  F().out = out;
   return hipSuccess;
 }
 hipError_t LaunchExportBits(uint32_t *bits, uint32_t *host, hipStream_t s) {
@@ -289,11 +298,40 @@ void ServerLeavesNothingBehind() {
   gst_server_destroy(s);
 }
 
+// A call whose wait failed may leave a kernel writing to its buffer: no later call gets it.
+void PinnedAfterFailedWait() {
+  const auto f = File();
+  std::vector<uint8_t> out(Header(f).width * Header(f).height / 2);
+  CHECK(gst_decompress_dxt(f.data(), f.size(), out.data(), out.size()) == GST_OK);
+  void *const first = F().out;
+  F().fail_waits = 1;
+  CHECK(gst_decompress_dxt(f.data(), f.size(), out.data(), out.size()) == GST_ERR_HIP);
+  CHECK(F().out == first);  // kept after the call that succeeded
+  CHECK(gst_decompress_dxt(f.data(), f.size(), out.data(), out.size()) == GST_OK);
+  CHECK(F().out != first);
+
+  const uint32_t counts[2] = {1, 1};
+  gst_ans_decoder *d = nullptr;
+  CHECK(gst_ans_decoder_create(counts, 2, 1, &d) == GST_OK);
+  const uint32_t state = 1u << 15;
+  const uint8_t word[2] = {};
+  const uint8_t *const data[1] = {word};
+  const size_t len[1] = {2};
+  uint8_t syms[GST_ANS_SYMBOLS_PER_STREAM];
+  F().fail_waits = 1;
+  CHECK(gst_ans_decode(d, &state, 1, data, len, 1, syms) == GST_ERR_HIP);
+  void *const failed = F().out;
+  CHECK(gst_ans_decode(d, &state, 1, data, len, 1, syms) == GST_OK);
+  CHECK(F().out != failed);
+  gst_ans_decoder_destroy(d);
+}
+
 const std::map<std::string, void (*)()> kChecks = {
     {"batch_plan", BatchPlanSurvives},
     {"batch_error_bits", BatchErrorBitsSurvive},
     {"stream_error_bits", StreamErrorBitsSurvive},
     {"server_flags", ServerLeavesNothingBehind},
+    {"pinned_after_failed_wait", PinnedAfterFailedWait},
 };
 
 }  // namespace
