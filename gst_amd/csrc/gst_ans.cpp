@@ -7,7 +7,9 @@
 
 #include <algorithm>
 #include <cstring>
+#include <memory>
 #include <mutex>
+#include <new>
 #include <vector>
 
 #include "gst_ans.h"
@@ -133,12 +135,20 @@ int gst_ans_decode(const gst_ans_decoder *d, const uint32_t *states, uint32_t nu
   const size_t out_bytes = static_cast<size_t>(num_streams) * GST_ANS_SYMBOLS_PER_STREAM;
   const size_t out_at = RoundUp256(total), status_at = out_at + RoundUp256(out_bytes);
   const size_t all = status_at + 4 * static_cast<size_t>(n_data);
+  std::lock_guard<std::mutex> lock(d->mu);
   // The kernel reads the packed data and writes the symbols and status words in pinned
-  // memory itself: one launch and one wait a call.
+  // memory itself: one launch and one wait a call.  Without pinned memory they pass through
+  // device memory and the runtime's copies.
   gst::PinnedBuffer buf;
   hipError_t e = gst::TakePinned(all, &buf);
-  if (e != hipSuccess) return HipFail(e);
-  std::lock_guard<std::mutex> lock(d->mu);
+  const bool pinned = e == hipSuccess;
+  std::unique_ptr<uint8_t[]> host;
+  if (!pinned) {
+    host.reset(new (std::nothrow) uint8_t[all]);
+    if (!host) return GST_ERR_OUT_OF_MEMORY;
+    buf.host = host.get();
+    ANS_HIP(hipMallocAsync(reinterpret_cast<void **>(&buf.dev), all, d->stream));
+  }
   uint8_t *const packed = buf.host;
   size_t at = 4 * static_cast<size_t>(n_data);
   for (uint32_t i = 0; i < n_data; ++i) {
@@ -151,8 +161,15 @@ int gst_ans_decode(const gst_ans_decoder *d, const uint32_t *states, uint32_t nu
     const uint32_t end32 = static_cast<uint32_t>(at);
     std::memcpy(packed + 4 * static_cast<size_t>(i), &end32, 4);
   }
-  e = gst::LaunchAnsGroups(d->d_tables, buf.dev, static_cast<uint32_t>(total), n_data, lanes,
-                           buf.dev + out_at, reinterpret_cast<uint32_t *>(buf.dev + status_at), d->stream);
+  e = pinned ? hipSuccess : hipMemcpyAsync(buf.dev, packed, total, hipMemcpyHostToDevice, d->stream);
+  if (e == hipSuccess)
+    e = gst::LaunchAnsGroups(d->d_tables, buf.dev, static_cast<uint32_t>(total), n_data, lanes,
+                             buf.dev + out_at, reinterpret_cast<uint32_t *>(buf.dev + status_at), d->stream);
+  if (!pinned) {
+    if (e == hipSuccess)
+      e = hipMemcpyAsync(packed + out_at, buf.dev + out_at, all - out_at, hipMemcpyDeviceToHost, d->stream);
+    (void)hipFreeAsync(buf.dev, d->stream);
+  }
   const hipError_t s = hipStreamSynchronize(d->stream);
   if (e == hipSuccess) e = s;
   uint32_t err = 0;
@@ -161,7 +178,7 @@ int gst_ans_decode(const gst_ans_decoder *d, const uint32_t *states, uint32_t nu
     const uint32_t *const status = reinterpret_cast<const uint32_t *>(packed + status_at);
     for (uint32_t i = 0; i < n_data; ++i) err |= status[i];
   }
-  gst::GivePinned(buf, s == hipSuccess);
+  if (pinned) gst::GivePinned(buf, s == hipSuccess);
   if (e != hipSuccess) return HipFail(e);
   return err ? GST_ERR_CORRUPT_STREAM : GST_OK;
 }

@@ -11,7 +11,9 @@
 #include <atomic>
 #include <cstring>
 #include <map>
+#include <memory>
 #include <mutex>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -226,6 +228,18 @@ uint32_t *ErrWord(hipStream_t s) {
   }
   g.err_words[s] = w;
   return w;
+}
+
+// A stream of the library's own, with its error word.
+void DestroyStream(hipStream_t s) {
+  Globals &g = G();
+  std::lock_guard<std::mutex> lk(g.mu);
+  auto it = g.err_words.find(s);
+  if (it != g.err_words.end()) {
+    (void)hipFree(it->second);
+    g.err_words.erase(it);
+  }
+  (void)hipStreamDestroy(s);
 }
 
 // Reads a word of error bits after the stream's work and clears it, all in the stream's own
@@ -737,21 +751,41 @@ class HostCalls {
     if (c->bits) (void)hipHostFree(c->bits);
     if (c->scratch.ptr) (void)hipFree(c->scratch.ptr);
     if (c->d_cmp) (void)hipFree(c->d_cmp);
-    if (c->stream) {
-      Globals &g = G();
-      std::lock_guard<std::mutex> lk(g.mu);
-      auto it = g.err_words.find(c->stream);
-      if (it != g.err_words.end()) {
-        (void)hipFree(it->second);
-        g.err_words.erase(it);
-      }
-      (void)hipStreamDestroy(c->stream);
-    }
+    if (c->stream) DestroyStream(c->stream);
     delete c;
   }
   std::mutex mu_;
   std::vector<Call *> idle_;
 };
+
+// gst_decompress_dxt without pinned memory or anything kept: ordinary host memory, copies by
+// the runtime, and a stream and device memory for this call alone.
+int DecompressUnpinned(const gst_header &h, const uint8_t *file, size_t len, uint8_t *out, size_t staging) {
+  std::unique_ptr<uint8_t[]> host(new (std::nothrow) uint8_t[staging]);
+  if (!host) return GST_ERR_OUT_OF_MEMORY;
+  const uint8_t *const files[1] = {file};
+  const size_t lens[1] = {len};
+  int rc = gst_pack_staging(files, lens, 1, host.get(), staging);
+  if (rc != GST_OK) return rc;
+  const size_t dxt = static_cast<size_t>(h.width) * h.height / 2;
+  hipStream_t s = nullptr;
+  GST_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
+  void *d_cmp = nullptr, *d_out = nullptr;
+  hipError_t e = hipMalloc(&d_cmp, staging);
+  if (e == hipSuccess) e = hipMalloc(&d_out, dxt);
+  if (e == hipSuccess) e = hipMemcpyAsync(d_cmp, host.get(), staging, hipMemcpyHostToDevice, s);
+  if (e == hipSuccess) rc = DecodeStaging(&h, 1, s, d_cmp, d_out, false, 0, nullptr, nullptr);
+  if (e == hipSuccess && rc == GST_OK) e = hipMemcpyAsync(out, d_out, dxt, hipMemcpyDeviceToHost, s);
+  uint32_t bits = 0;
+  if (e == hipSuccess && rc == GST_OK) rc = gst_read_error_bits(s, &bits);
+  const hipError_t done = hipStreamSynchronize(s);
+  if (e == hipSuccess) e = done;
+  if (d_cmp) (void)hipFree(d_cmp);
+  if (d_out) (void)hipFree(d_out);
+  DestroyStream(s);
+  if (e != hipSuccess) return HipFail(e);
+  return rc == GST_OK && bits ? GST_ERR_CORRUPT_STREAM : rc;
+}
 
 }  // namespace
 
@@ -1025,13 +1059,13 @@ int gst_decompress_dxt(const uint8_t *file, size_t len, uint8_t *out, size_t out
   // codec/decoder.cpp:430-476: offsets block of 512 B, then the file minus its header.
   const size_t staging = 512 + 2048 + StreamBytes(h);
   HostCalls::Call *c = HostCalls::Get().Take(staging);
-  if (!c) return GST_ERR_OUT_OF_MEMORY;
+  if (!c) return DecompressUnpinned(h, file, len, out, staging);
   const size_t out_at = AlignUp(staging, kAlign);
   gst::PinnedBuffer pin;  // [staging][blocks]
   hipError_t e = gst::TakePinned(out_at + dxt, &pin);
   if (e != hipSuccess) {
     HostCalls::Get().Give(c, true);
-    return HipFail(e);
+    return DecompressUnpinned(h, file, len, out, staging);
   }
   const uint8_t *const files[1] = {file};
   const size_t lens[1] = {len};

@@ -43,6 +43,7 @@ struct Fake {
   uint32_t raise = 0;    // error bits the next decodes set
   uint32_t images = 0;   // images the last rANS launch found in its plan
   int fail_waits = 0;    // hipStreamSynchronize fails this many times
+  bool no_pinned = false;  // hipHostMalloc fails
   void *out = nullptr;   // where the last kernel wrote its output
 
   void RunLate() {
@@ -89,7 +90,9 @@ hipError_t hipMalloc(void **p, size_t n) { return NewMemory(p, n); }
 hipError_t hipFree(void *p) { F().freed.insert(p); return hipSuccess; }
 hipError_t hipMallocAsync(void **p, size_t n, hipStream_t) { return NewMemory(p, n); }
 hipError_t hipFreeAsync(void *p, hipStream_t) { F().freed.insert(p); return hipSuccess; }
-hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return NewMemory(p, n); }
+hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
+  return F().no_pinned ? hipErrorOutOfMemory : NewMemory(p, n);
+}
 hipError_t hipHostFree(void *p) { F().freed.insert(p); return hipSuccess; }
 hipError_t hipHostGetDevicePointer(void **d, void *h, unsigned) { *d = h; return hipSuccess; }
 hipError_t hipPointerGetAttributes(hipPointerAttribute_t *, const void *) { return hipErrorInvalidValue; }
@@ -298,6 +301,24 @@ void ServerLeavesNothingBehind() {
   gst_server_destroy(s);
 }
 
+// One stand-alone stream of one word.
+struct AnsCall {
+  gst_ans_decoder *d = nullptr;
+  uint8_t syms[GST_ANS_SYMBOLS_PER_STREAM] = {};
+  AnsCall() {
+    const uint32_t counts[2] = {1, 1};
+    CHECK(gst_ans_decoder_create(counts, 2, 1, &d) == GST_OK);
+  }
+  ~AnsCall() { gst_ans_decoder_destroy(d); }
+  int Decode() {
+    const uint32_t state = 1u << 15;
+    const uint8_t word[2] = {};
+    const uint8_t *const data[1] = {word};
+    const size_t len[1] = {2};
+    return gst_ans_decode(d, &state, 1, data, len, 1, syms);
+  }
+};
+
 // A call whose wait failed may leave a kernel writing to its buffer: no later call gets it.
 void PinnedAfterFailedWait() {
   const auto f = File();
@@ -310,20 +331,31 @@ void PinnedAfterFailedWait() {
   CHECK(gst_decompress_dxt(f.data(), f.size(), out.data(), out.size()) == GST_OK);
   CHECK(F().out != first);
 
-  const uint32_t counts[2] = {1, 1};
-  gst_ans_decoder *d = nullptr;
-  CHECK(gst_ans_decoder_create(counts, 2, 1, &d) == GST_OK);
-  const uint32_t state = 1u << 15;
-  const uint8_t word[2] = {};
-  const uint8_t *const data[1] = {word};
-  const size_t len[1] = {2};
-  uint8_t syms[GST_ANS_SYMBOLS_PER_STREAM];
+  AnsCall a;
   F().fail_waits = 1;
-  CHECK(gst_ans_decode(d, &state, 1, data, len, 1, syms) == GST_ERR_HIP);
+  CHECK(a.Decode() == GST_ERR_HIP);
   void *const failed = F().out;
-  CHECK(gst_ans_decode(d, &state, 1, data, len, 1, syms) == GST_OK);
+  CHECK(a.Decode() == GST_OK);
   CHECK(F().out != failed);
-  gst_ans_decoder_destroy(d);
+}
+
+// Host-to-host calls go on without pinned memory: from the first, and when it runs out.
+void NoPinnedMemory() {
+  const auto f = File();
+  AnsCall a;
+  for (bool none : {true, false, true}) {
+    F().no_pinned = none;
+    if (none) gst_free_decompressor();
+    std::vector<uint8_t> out(Header(f).width * Header(f).height / 2);
+    CHECK(gst_decompress_dxt(f.data(), f.size(), out.data(), out.size()) == GST_OK);
+    for (uint8_t v : out) CHECK(v == kBlock);
+    F().raise = 4;
+    CHECK(gst_decompress_dxt(f.data(), f.size(), out.data(), out.size()) == GST_ERR_CORRUPT_STREAM);
+    F().raise = 0;
+    std::memset(a.syms, 0, sizeof(a.syms));
+    CHECK(a.Decode() == GST_OK);
+    for (uint8_t v : a.syms) CHECK(v == kBlock);
+  }
 }
 
 const std::map<std::string, void (*)()> kChecks = {
@@ -332,6 +364,7 @@ const std::map<std::string, void (*)()> kChecks = {
     {"stream_error_bits", StreamErrorBitsSurvive},
     {"server_flags", ServerLeavesNothingBehind},
     {"pinned_after_failed_wait", PinnedAfterFailedWait},
+    {"no_pinned_memory", NoPinnedMemory},
 };
 
 }  // namespace
