@@ -480,9 +480,11 @@ int TakeScratch(size_t bytes, hipStream_t s, KeptScratch *own, Scratch *out) {
     }
   }
   if (own && bytes <= kKeptScratchBytes) {
-    GST_HIP(GrowScratch(own, bytes, s));
-    out->ptr = own->ptr;
-    return GST_OK;
+    if (GrowScratch(own, bytes, s) == hipSuccess) {
+      out->ptr = own->ptr;
+      return GST_OK;
+    }
+    (void)hipGetLastError();  // kept scratch comes in powers of two: exactly `bytes` may still fit
   }
   if (!s && (out->slot = DefaultStreamScratch::Get().Take(bytes)) != nullptr) {
     out->ptr = out->slot->ptr;

@@ -43,6 +43,7 @@ struct Fake {
   uint32_t raise = 0;    // error bits the next decodes set
   uint32_t images = 0;   // images the last rANS launch found in its plan
   int fail_waits = 0;    // hipStreamSynchronize fails this many times
+  size_t most = ~size_t{0};  // the largest device allocation that succeeds
   bool no_pinned = false;  // hipHostMalloc fails
   void *out = nullptr;   // where the last kernel wrote its output
 
@@ -86,9 +87,9 @@ hipError_t hipGetDeviceProperties(hipDeviceProp_t *p, int) {
 }
 hipError_t hipGetLastError() { return hipSuccess; }
 
-hipError_t hipMalloc(void **p, size_t n) { return NewMemory(p, n); }
+hipError_t hipMalloc(void **p, size_t n) { return n > F().most ? hipErrorOutOfMemory : NewMemory(p, n); }
 hipError_t hipFree(void *p) { F().freed.insert(p); return hipSuccess; }
-hipError_t hipMallocAsync(void **p, size_t n, hipStream_t) { return NewMemory(p, n); }
+hipError_t hipMallocAsync(void **p, size_t n, hipStream_t) { return hipMalloc(p, n); }
 hipError_t hipFreeAsync(void *p, hipStream_t) { F().freed.insert(p); return hipSuccess; }
 hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
   return F().no_pinned ? hipErrorOutOfMemory : NewMemory(p, n);
@@ -358,6 +359,18 @@ void NoPinnedMemory() {
   }
 }
 
+// A call that fits the device's memory goes on where the size it would keep does not.
+void LittleDeviceMemory() {
+  const auto f = File();
+  const gst_header h = Header(f);
+  std::vector<uint8_t> out(h.width * h.height / 2), staging(512 + f.size());
+  CHECK(gst_decompress_dxt(f.data(), f.size(), out.data(), out.size()) == GST_OK);
+  gst_free_decompressor();
+  F().most = size_t{300} << 10;  // the scratch is 177 KiB, kept scratch at least 1 MiB
+  CHECK(gst_decompress_dxt(f.data(), f.size(), out.data(), out.size()) == GST_OK);
+  CHECK(gst_load_compressed_dxt(&h, nullptr, staging.data(), out.data(), 0, nullptr, nullptr) == GST_OK);
+}
+
 const std::map<std::string, void (*)()> kChecks = {
     {"batch_plan", BatchPlanSurvives},
     {"batch_error_bits", BatchErrorBitsSurvive},
@@ -365,6 +378,7 @@ const std::map<std::string, void (*)()> kChecks = {
     {"server_flags", ServerLeavesNothingBehind},
     {"pinned_after_failed_wait", PinnedAfterFailedWait},
     {"no_pinned_memory", NoPinnedMemory},
+    {"little_device_memory", LittleDeviceMemory},
 };
 
 }  // namespace
