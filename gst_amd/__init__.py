@@ -214,9 +214,8 @@ def _events(init):
     return len(init), ctypes.cast(arr, _P)
 
 
-_PyBytes = ctypes.pythonapi.PyBytes_FromStringAndSize
-_PyBytes.argtypes = [_P, ctypes.c_ssize_t]
-_PyBytes.restype = ctypes.py_object
+# A prototype of its own: ctypes.pythonapi's function object belongs to the whole process.
+_PyBytes = ctypes.PYFUNCTYPE(ctypes.py_object, _P, ctypes.c_ssize_t)(("PyBytes_FromStringAndSize", ctypes.pythonapi))
 
 
 def _new_bytes(n):
