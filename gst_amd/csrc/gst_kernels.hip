@@ -997,18 +997,17 @@ __device__ __forceinline__ void StoreChainChunk(const u32x2 *tab, u32x2 *ring, u
 // wait state that the compiler puts behind every block and the 18 scalar instructions of a
 // ring check; see DecodeGroupChain.  A read of either entry under its own exec mask, without
 // the address select, also took 135.)  Two instructions stand between the compare and the
-// first vector read of its vcc_lo, the wait states that this chip asks for and that nothing
-// checks inside the block.  LDS addresses are those of AnsChainLds at address 0, the
-// kernel's only LDS object; the entry is in fixed registers because its halves have no name
-// otherwise.
-__device__ __forceinline__ uint32_t ChainSteps(uint32_t &y, uint32_t thr0, uint32_t thr, uint32_t &q) {
+// first vector read of its vcc_lo, the wait states that this chip asks for and that the
+// compiler does not add inside the block.  tab_at is the table's LDS address, q the next
+// word's entry's; the entry is in fixed registers because its halves have no name otherwise.
+__device__ __forceinline__ uint32_t ChainSteps(uint32_t &y, uint32_t thr0, uint32_t thr, uint32_t tab_at, uint32_t &q) {
   uint32_t word = 0;
 #if defined(__HIP_DEVICE_COMPILE__)
   uint32_t slot, rank, mul, moved;
 #define GST_CHAIN_STEP(THR, INSERT)                    \
   "v_cmp_lt_u32 vcc, %[y], " THR "\n\t"                \
-  "v_lshlrev_b32 %[slot], 3, %[y]\n\t"                 \
-  "v_and_b32 %[slot], 0x3ff8, %[slot]\n\t"             \
+  "v_and_b32 %[slot], 0x7ff, %[y]\n\t"                 \
+  "v_lshl_add_u32 %[slot], %[slot], 3, %[tab]\n\t"     \
   "v_mbcnt_lo_u32_b32 %[rank], vcc_lo, 0\n\t"          \
   "v_lshl_add_u32 %[rank], %[rank], 3, %[q]\n\t"       \
   "v_cndmask_b32 %[slot], %[slot], %[rank], vcc\n\t"   \
@@ -1025,7 +1024,8 @@ __device__ __forceinline__ uint32_t ChainSteps(uint32_t &y, uint32_t thr0, uint3
                GST_CHAIN_STEP("%[thr]", "v_perm_b32 %[word], v120, %[word], %[s0]")
                : [y] "+v"(y), [q] "+s"(q), [word] "=&v"(word), [slot] "=&v"(slot), [rank] "=&v"(rank),
                  [mul] "=&v"(mul), [moved] "=&s"(moved)
-               : [thr0] "v"(thr0), [thr] "v"(thr), [s2] "s"(0x03070100u), [s1] "s"(0x03020700u), [s0] "s"(0x03020107u)
+               : [thr0] "v"(thr0), [thr] "v"(thr), [tab] "s"(tab_at), [s2] "s"(0x03070100u), [s1] "s"(0x03020700u),
+                 [s0] "s"(0x03020107u)
                : "vcc", "scc", "memory", "v120", "v121");
 #undef GST_CHAIN_STEP
 #endif
@@ -1038,7 +1038,7 @@ __device__ __forceinline__ uint32_t ChainSteps(uint32_t &y, uint32_t thr0, uint3
 // renormalisation in y and the ring address of the next word in q; returns how many words
 // the group consumed before that renormalisation.
 template <bool kSum>
-__device__ __forceinline__ uint32_t DecodeGroupChain(const AnsChainLds &lds, u32x2 *ring, uint32_t ring_at,
+__device__ __forceinline__ uint32_t DecodeGroupChain(const AnsChainLds &lds, u32x2 *ring,
                                                      __amdgpu_buffer_rsrc_t rs, uint32_t lane, uint32_t n,
                                                      uint32_t &y, uint32_t &q, uint32_t p, uint32_t clo, u32x2 pE,
                                                      u32x2 pO, GPtr<uint8_t> outp, GPtr<int32_t> group_sum,
@@ -1049,6 +1049,7 @@ __device__ __forceinline__ uint32_t DecodeGroupChain(const AnsChainLds &lds, u32
   uint32_t thr = 0;  // a group's first step never renormalises: its states come as stored
   asm volatile("" : "+v"(thr));
   uint32_t top = p ? (p - 1) / kChunkWords : 0u;
+  const uint32_t tab_at = Uniform(LdsAddress(&lds.tab[0])), ring_at = Uniform(LdsAddress(ring));
   const uint32_t q0 = ring_at + 8 * (kChunkWords - 1 - ((p - 1) & (kChunkWords - 1)));
   q = Uniform(q0);
   const uint32_t end0 = ring_at + 8 * kChunkWords, end1 = ring_at + 16 * kChunkWords;
@@ -1058,7 +1059,7 @@ __device__ __forceinline__ uint32_t DecodeGroupChain(const AnsChainLds &lds, u32
     uint32_t acc[16];
 #pragma unroll
     for (uint32_t w = 0; w < 16; ++w) {
-      acc[15 - w] = ChainSteps(y, thr, full, q);
+      acc[15 - w] = ChainSteps(y, thr, full, tab_at, q);
       thr = full;
       // 8 steps read at most 256 words, so at most one chunk's end was crossed.  One test
       // on the way past (two scalar instructions; both cases' tests there took 18, 100
@@ -1163,16 +1164,15 @@ __global__ __launch_bounds__(kChainWaves * 64, 4) void AnsChainKernel(KernelArgs
     StoreChainChunk(lds.tab, ring, 0, false, lane, c0);
     StoreChainChunk(lds.tab, ring, kChunkWords, false, lane, c1);
     WaveSync();
-    const uint32_t ring_at = sizeof(lds.tab) + wave * sizeof(lds.ring[0]);
     const GPtr<uint8_t> outp = Gbl<uint8_t>(d->symbols + SymbolOffset(nv, d->palette_bytes, k)) + static_cast<size_t>(g) * kGroupSyms;
     uint32_t y = x, q, used;
     if (k == 3) {
       const GPtr<int32_t> sums = Gbl<int32_t>(d->lane_sums);
-      used = DecodeGroupChain<true>(lds, ring, ring_at, rs, lane, kLanesPerGroup, y, q, p, clo, pE, pO, outp,
+      used = DecodeGroupChain<true>(lds, ring, rs, lane, kLanesPerGroup, y, q, p, clo, pE, pO, outp,
                                     Gbl<int32_t>(d->group_sums) + g, sums ? sums + g * kLanesPerGroup : nullptr,
                                     sums ? sums + LaneSuffixBase(nv) + g * kLanesPerGroup * 8 : nullptr);
     } else {
-      used = DecodeGroupChain<false>(lds, ring, ring_at, rs, lane, kLanesPerGroup, y, q, p, clo, pE, pO, outp,
+      used = DecodeGroupChain<false>(lds, ring, rs, lane, kLanesPerGroup, y, q, p, clo, pE, pO, outp,
                                      nullptr, nullptr, nullptr);
     }
     used += Popc64(__builtin_amdgcn_ballot_w64(lane < kLanesPerGroup && y < kStateL));  // the last renormalisation's
@@ -1236,12 +1236,11 @@ __global__ __launch_bounds__(kChainWaves * 64, 4) void AnsGroupsKernel(const uin
   WaveSync();
   const bool active = lane < n;
   uint32_t y = active ? x : 0u, q;
-  const uint32_t ring_at = sizeof(lds.tab) + wave * sizeof(lds.ring[0]);
-  DecodeGroupChain<false>(lds, ring, ring_at, rs, lane, n, y, q, p, 0, pE, pO, dst, nullptr, nullptr, nullptr);
+  DecodeGroupChain<false>(lds, ring, rs, lane, n, y, q, p, 0, pE, pO, dst, nullptr, nullptr, nullptr);
   // The final state is 2^15: y itself, or y = 0 renormalised with the word 2^15, which its
   // ring entry tells from every other word (slot 0, 16 above it: an rANS step is one to one).
   const uint64_t ends = __builtin_amdgcn_ballot_w64(active && y < kStateL);
-  const u32x2 e = ring[(q - ring_at) / 8 + __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(ends), 0u)];
+  const u32x2 e = ring[(q - LdsAddress(ring)) / 8 + __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(ends), 0u)];
   const uint32_t f = lds.tab[0].x & 0xFFFFFFu;
   const bool last = y >= kStateL ? y == kStateL
                                  : y == 0 && e.x == ((f << 5) | (lds.tab[0].x & 0xFF000000u)) && e.y == 16 * f;
