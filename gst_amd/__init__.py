@@ -17,7 +17,6 @@ raises GstError on a non-zero status.  The library must be built
 """
 import array
 import ctypes
-import itertools
 import math
 import os
 import struct
@@ -454,15 +453,17 @@ def NormalizeFrequencies(counts, M=ANS_TABLE_SIZE):
     return [int(v) for v in out[:n]]
 
 
-# 32 streams' symbols at a time, a third of the time of a slice each.  (One format for a whole
+# 64 streams' symbols at a time, a third of the time of a slice each.  (One format for a whole
 # call would stay in struct's cache: 24 bytes a stream for each of up to 100 sizes.)
-_STREAMS = struct.Struct("%ds" % ANS_SYMBOLS_PER_STREAM * 32)
+_STREAMS = struct.Struct("%ds" % ANS_SYMBOLS_PER_STREAM * 64)
 
 
 def _split_streams(raw):
     whole = len(raw) // _STREAMS.size * _STREAMS.size
-    out = list(itertools.chain.from_iterable(_STREAMS.iter_unpack(memoryview(raw)[:whole])))
-    out += [raw[i:i + ANS_SYMBOLS_PER_STREAM] for i in range(whole, len(raw), ANS_SYMBOLS_PER_STREAM)]
+    out = []
+    for at in range(0, whole, _STREAMS.size):
+        out += _STREAMS.unpack_from(raw, at)
+    out += struct.unpack_from("%ds" % ANS_SYMBOLS_PER_STREAM * ((len(raw) - whole) // ANS_SYMBOLS_PER_STREAM), raw, whole)
     return out
 
 
