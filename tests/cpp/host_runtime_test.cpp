@@ -8,6 +8,7 @@
 // on it.  The "kernels" write kBlock to every output byte.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -44,6 +45,7 @@ struct Fake {
   uint32_t images = 0;   // images the last rANS launch found in its plan
   int fail_waits = 0;    // hipStreamSynchronize fails this many times
   size_t most = ~size_t{0};  // the largest device allocation that succeeds
+  size_t pinned = 0;     // the largest pinned allocation so far
   bool no_pinned = false;  // hipHostMalloc fails
   void *out = nullptr;   // where the last kernel wrote its output
 
@@ -92,6 +94,7 @@ hipError_t hipFree(void *p) { F().freed.insert(p); return hipSuccess; }
 hipError_t hipMallocAsync(void **p, size_t n, hipStream_t) { return hipMalloc(p, n); }
 hipError_t hipFreeAsync(void *p, hipStream_t) { F().freed.insert(p); return hipSuccess; }
 hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
+  F().pinned = std::max(F().pinned, n);
   return F().no_pinned ? hipErrorOutOfMemory : NewMemory(p, n);
 }
 hipError_t hipHostFree(void *p) { F().freed.insert(p); return hipSuccess; }
@@ -371,6 +374,26 @@ void LittleDeviceMemory() {
   CHECK(gst_load_compressed_dxt(&h, nullptr, staging.data(), out.data(), 0, nullptr, nullptr) == GST_OK);
 }
 
+// Calls too large for a buffer that is kept pin nothing for themselves.
+void LargeHostCalls() {
+  const auto f = File(16384, 8192);
+  std::vector<uint8_t> out(size_t{16384} * 8192 / 2);
+  CHECK(gst_decompress_dxt(f.data(), f.size(), out.data(), out.size()) == GST_OK);
+  for (uint8_t v : out) CHECK(v == kBlock);
+  const uint32_t groups = 8192, lanes = 32, counts[2] = {1, 1};
+  gst_ans_decoder *d = nullptr;
+  CHECK(gst_ans_decoder_create(counts, 2, lanes, &d) == GST_OK);
+  const uint8_t word[2] = {};
+  const std::vector<uint32_t> states(groups * lanes, 1u << 15);
+  const std::vector<const uint8_t *> data(groups, word);
+  const std::vector<size_t> lens(groups, 2);
+  std::vector<uint8_t> syms(states.size() * GST_ANS_SYMBOLS_PER_STREAM);
+  CHECK(gst_ans_decode(d, states.data(), groups * lanes, data.data(), lens.data(), groups, syms.data()) == GST_OK);
+  for (uint8_t v : syms) CHECK(v == kBlock);
+  gst_ans_decoder_destroy(d);
+  CHECK(F().pinned <= size_t{64} << 20);
+}
+
 const std::map<std::string, void (*)()> kChecks = {
     {"batch_plan", BatchPlanSurvives},
     {"batch_error_bits", BatchErrorBitsSurvive},
@@ -379,6 +402,7 @@ const std::map<std::string, void (*)()> kChecks = {
     {"pinned_after_failed_wait", PinnedAfterFailedWait},
     {"no_pinned_memory", NoPinnedMemory},
     {"little_device_memory", LittleDeviceMemory},
+    {"large_host_calls", LargeHostCalls},
 };
 
 }  // namespace
