@@ -885,14 +885,13 @@ __device__ __forceinline__ void AnsDecodeUnits(const KernelArgs &a, AnsLds<WAVES
   }
 }
 
-template <uint32_t WAVES, uint32_t GPW, bool kBuild, bool kPair = false>
-// With 4 or 8 waves LDS allows 7 waves per SIMD (6 with the second table); hold the
-// VGPRs to that (at most 72, or 80).
-__global__ __launch_bounds__(WAVES * 64, kPair ? 6 : WAVES >= 4 ? 7 : 1)
+template <uint32_t WAVES, uint32_t GPW, bool kBuild>
+// With 4 or 8 waves LDS allows 7 waves per SIMD; hold the VGPRs to that (at most 72).
+__global__ __launch_bounds__(WAVES * 64, WAVES >= 4 ? 7 : 1)
 void AnsDecodeKernel(KernelArgs a) {
-  __shared__ __align__(16) AnsLds<WAVES, kPair> lds;
+  __shared__ __align__(16) AnsLds<WAVES, false> lds;
   __shared__ AnsLdsSmall small;
-  AnsDecodeUnits<WAVES, GPW, kBuild, kPair>(a, lds, small);
+  AnsDecodeUnits<WAVES, GPW, kBuild, false>(a, lds, small);
 }
 
 // The rANS stage whose work-unit form is data: the plan's unit code (or, for a single
@@ -2190,9 +2189,9 @@ __global__ __launch_bounds__(256) void AssembleRgbKernel(KernelArgs a) {
   }
 }
 
-template <uint32_t WAVES, uint32_t GPW, bool kBuild = false, bool kPair = false>
+template <uint32_t WAVES, uint32_t GPW, bool kBuild = false>
 hipError_t LaunchAns(const KernelArgs &args, uint32_t grid, hipStream_t stream) {
-  hipLaunchKernelGGL((AnsDecodeKernel<WAVES, GPW, kBuild, kPair>), dim3(grid), dim3(WAVES * 64), 0, stream, args);
+  hipLaunchKernelGGL((AnsDecodeKernel<WAVES, GPW, kBuild>), dim3(grid), dim3(WAVES * 64), 0, stream, args);
   return hipGetLastError();
 }
 
