@@ -901,7 +901,7 @@ int gst_read_error_bits_async(gst_stream stream, uint32_t *host_bits) {
   uint32_t *w = ErrWord(s);
   if (!w) return GST_ERR_HIP;
   GST_HIP(hipMemcpyAsync(host_bits, w, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-  GST_HIP(hipMemsetAsync(w, 0, sizeof(uint32_t), s));
+  GST_HIP(gst::LaunchClearWord(w, s));
   return GST_OK;
 }
 
@@ -1621,7 +1621,7 @@ int gst_batch_error_bits_async(gst_batch *b, gst_stream stream, uint32_t *host_b
   if (!b || !host_bits) return GST_ERR_INVALID_ARGUMENT;
   hipStream_t s = static_cast<hipStream_t>(stream);
   GST_HIP(hipMemcpyAsync(host_bits, b->dmem + b->err_off, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-  GST_HIP(hipMemsetAsync(b->dmem + b->err_off, 0, sizeof(uint32_t), s));
+  GST_HIP(gst::LaunchClearWord(reinterpret_cast<uint32_t *>(b->dmem + b->err_off), s));
   return GST_OK;
 }
 

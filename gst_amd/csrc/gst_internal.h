@@ -298,6 +298,10 @@ hipError_t LaunchAnsGroups(const uint32_t *table, const uint8_t *data, uint32_t 
 // without a DMA copy's fixed cost.
 hipError_t LaunchExportBits(uint32_t *bits, uint32_t *host, hipStream_t stream);
 
+// Zeroes a word in stream order, for calls that a caller may capture into a graph: a recorded
+// hipMemsetAsync has given wrong results there on replays after the first.
+hipError_t LaunchClearWord(uint32_t *word, hipStream_t stream);
+
 // Device-side comparison of decoded outputs with expected bytes: the server checks
 // every completion this way under load.  Job i sets flags[job.flag] to 1 when its
 // `bytes` (a multiple of 16, both pointers 16-byte aligned) differ anywhere.

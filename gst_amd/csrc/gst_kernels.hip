@@ -2401,6 +2401,15 @@ __global__ __launch_bounds__(64) void ExportBitsKernel(uint32_t *bits, uint32_t 
   Gbl<uint32_t>(bits)[0] = 0;
 }
 
+__global__ __launch_bounds__(64) void ClearWordKernel(uint32_t *word) {
+  if (threadIdx.x == 0) Gbl<uint32_t>(word)[0] = 0;
+}
+
+hipError_t LaunchClearWord(uint32_t *word, hipStream_t stream) {
+  hipLaunchKernelGGL(ClearWordKernel, dim3(1), dim3(64), 0, stream, word);
+  return hipGetLastError();
+}
+
 hipError_t LaunchExportBits(uint32_t *bits, uint32_t *host, hipStream_t stream) {
   hipLaunchKernelGGL(ExportBitsKernel, dim3(1), dim3(64), 0, stream, bits, host);
   return hipGetLastError();

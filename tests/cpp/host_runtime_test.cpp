@@ -41,6 +41,7 @@ struct Fake {
   std::vector<std::function<void()>> late;  // null-stream clears that were not waited for
   std::set<void *> freed;
   int streams = 0;
+  int memsets = 0;       // hipMemsetAsync calls on created streams
   uint32_t raise = 0;    // error bits the next decodes set
   uint32_t images = 0;   // images the last rANS launch found in its plan
   int fail_waits = 0;    // hipStreamSynchronize fails this many times
@@ -109,6 +110,7 @@ hipError_t hipMemset(void *p, int v, size_t n) {
 }
 hipError_t hipMemsetAsync(void *p, int v, size_t n, hipStream_t s) {
   if (!s) return hipMemset(p, v, n);
+  ++F().memsets;
   std::memset(p, v, n);
   return hipSuccess;
 }
@@ -184,6 +186,11 @@ hipError_t LaunchExportBits(uint32_t *bits, uint32_t *host, hipStream_t s) {
   F().Before(s);
   *host = *bits;
   *bits = 0;
+  return hipSuccess;
+}
+hipError_t LaunchClearWord(uint32_t *word, hipStream_t s) {
+  F().Before(s);
+  *word = 0;
   return hipSuccess;
 }
 hipError_t LaunchGather(const GatherArgs &a, hipStream_t s) {
@@ -292,6 +299,30 @@ void StreamErrorBitsSurvive() {
   }
 }
 
+// What a caller may record into a graph holds no hipMemsetAsync.
+void AsyncErrorBits() {
+  const auto f = File();
+  const gst_header h = Header(f);
+  std::vector<uint8_t> out(h.width * h.height / 2), staging(512 + f.size());
+  gst_batch *b = NewBatch(h);
+  hipStream_t s = NewStream();
+  Bind(b, h, f, &out, s);
+  uint32_t got = 0;
+  CHECK(gst_read_error_bits(s, &got) == GST_OK);  // the stream's word is there from here on
+  const int before = F().memsets;
+  for (uint32_t bits : {4u, 0u, 6u}) {
+    F().raise = bits;
+    CHECK(gst_load_compressed_dxt(&h, s, staging.data(), out.data(), 0, nullptr, nullptr) == GST_OK);
+    CHECK(gst_read_error_bits_async(s, &got) == GST_OK);
+    CHECK(got == bits);
+    CHECK(gst_batch_decode(b, s) == GST_OK);
+    CHECK(gst_batch_error_bits_async(b, s, &got) == GST_OK);
+    CHECK(got == bits);
+  }
+  CHECK(F().memsets == before);
+  gst_batch_destroy(b);
+}
+
 // The server's comparison flags and plans are cleared before its first request.
 void ServerLeavesNothingBehind() {
   gst_server_config c{};
@@ -398,6 +429,7 @@ const std::map<std::string, void (*)()> kChecks = {
     {"batch_plan", BatchPlanSurvives},
     {"batch_error_bits", BatchErrorBitsSurvive},
     {"stream_error_bits", StreamErrorBitsSurvive},
+    {"async_error_bits", AsyncErrorBits},
     {"server_flags", ServerLeavesNothingBehind},
     {"pinned_after_failed_wait", PinnedAfterFailedWait},
     {"no_pinned_memory", NoPinnedMemory},
