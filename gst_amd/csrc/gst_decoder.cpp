@@ -827,9 +827,9 @@ int gst_initialize_decoder(int device) {
   hipDeviceProp_t prop;
   GST_HIP(hipGetDeviceProperties(&prop, device));
   if (std::string(prop.gcnArchName).rfind("gfx950", 0) != 0) return GST_ERR_NOT_INITIALIZED;
-  // The kernels need 256-thread work-groups and 16 KiB + 8.4 KiB of LDS
-  // (codec/decoder.cpp:558-591 checks the work-group sizes of the reference's).
-  if (prop.maxThreadsPerBlock < 512 || prop.sharedMemPerBlock < 32768) return GST_ERR_NOT_INITIALIZED;
+  // The kernels need work-groups of up to 512 threads and 40 KiB of LDS (AnsChainKernel;
+  // codec/decoder.cpp:558-591 checks the work-group sizes of the reference's).
+  if (prop.maxThreadsPerBlock < 512 || prop.sharedMemPerBlock < 40960) return GST_ERR_NOT_INITIALIZED;
   // The no-allocation entry point's static scratch on this device (current here).
   GST_HIP(gst::ResolveNoAllocScratch(device));
   g.device = device;

@@ -40,6 +40,7 @@ struct Fake {
   std::mutex mu;
   std::vector<std::function<void()>> late;  // null-stream clears that were not waited for
   std::set<void *> freed;
+  size_t lds = 65536;
   int streams = 0;
   int memsets = 0;       // hipMemsetAsync calls on created streams
   uint32_t raise = 0;    // error bits the next decodes set
@@ -84,7 +85,7 @@ hipError_t hipGetDeviceProperties(hipDeviceProp_t *p, int) {
   std::memset(p, 0, sizeof(*p));
   std::strcpy(p->gcnArchName, "gfx950:sramecc+:xnack-");
   p->maxThreadsPerBlock = 1024;
-  p->sharedMemPerBlock = 65536;
+  p->sharedMemPerBlock = F().lds;
   p->multiProcessorCount = 256;
   return hipSuccess;
 }
@@ -247,6 +248,14 @@ void Bind(gst_batch *b, const gst_header &h, const std::vector<uint8_t> &f, std:
   const void *in[1] = {f.data()};
   void *o[1] = {out->data()};
   CHECK(gst_batch_bind(b, &h, 1, in, o, s) == GST_OK);
+}
+
+// A device without the LDS that the largest kernel asks for is refused when it is set up.
+void DeviceWithLittleLds() {
+  F().lds = 40959;
+  CHECK(gst_initialize_decoder(0) == GST_ERR_NOT_INITIALIZED);
+  F().lds = 40960;
+  CHECK(gst_initialize_decoder(0) == GST_OK);
 }
 
 // A batch made while the null stream is busy, bound on a stream that does not wait for it.
@@ -426,6 +435,7 @@ void LargeHostCalls() {
 }
 
 const std::map<std::string, void (*)()> kChecks = {
+    {"little_lds", DeviceWithLittleLds},
     {"batch_plan", BatchPlanSurvives},
     {"batch_error_bits", BatchErrorBitsSurvive},
     {"stream_error_bits", StreamErrorBitsSurvive},

@@ -13,7 +13,7 @@ EXE = os.path.join(ROOT, "tests", "cpp", "host_runtime_test")
 
 @pytest.mark.parametrize("check", ["batch_plan", "batch_error_bits", "stream_error_bits", "server_flags",
                                    "pinned_after_failed_wait", "no_pinned_memory", "little_device_memory",
-                                   "large_host_calls", "async_error_bits"])
+                                   "large_host_calls", "async_error_bits", "little_lds"])
 def test_host_code(check):
     proc = subprocess.run([EXE, check], capture_output=True, text=True, timeout=60)
     assert proc.returncode == 0, proc.stdout + proc.stderr
