@@ -455,15 +455,19 @@ def NormalizeFrequencies(counts, M=ANS_TABLE_SIZE):
 
 # 64 streams' symbols at a time, a third of the time of a slice each.  (One format for a whole
 # call would stay in struct's cache: 24 bytes a stream for each of up to 100 sizes.)
-_STREAMS = struct.Struct("%ds" % ANS_SYMBOLS_PER_STREAM * 64)
+_STREAM = "%ds" % ANS_SYMBOLS_PER_STREAM
+_STREAMS = struct.Struct(_STREAM * 64)
 
 
 def _split_streams(raw):
-    whole = len(raw) // _STREAMS.size * _STREAMS.size
+    n = len(raw) // ANS_SYMBOLS_PER_STREAM
+    if n < 64:
+        return list(struct.unpack(_STREAM * n, raw))
     out = []
-    for at in range(0, whole, _STREAMS.size):
+    for at in range(0, n // 64 * _STREAMS.size, _STREAMS.size):
         out += _STREAMS.unpack_from(raw, at)
-    out += struct.unpack_from("%ds" % ANS_SYMBOLS_PER_STREAM * ((len(raw) - whole) // ANS_SYMBOLS_PER_STREAM), raw, whole)
+    if n % 64:
+        out += struct.unpack_from(_STREAM * (n % 64), raw, n // 64 * _STREAMS.size)
     return out
 
 
