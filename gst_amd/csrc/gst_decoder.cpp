@@ -151,7 +151,7 @@ StageConfig DefaultStageConfig(bool rgb) {
   s.fused_waves = rgb ? 0 : 4;
   s.tile_fused = 1;
   s.ans_build_tables = 1;
-  s.ans_auto = 1;  // GST_ANS_FORM_AUTO: the caller sets ans_pair_short from AutoPairs
+  s.ans_auto = 1;  // GST_ANS_FORM_AUTO: the caller chooses the kernel and its form (SetAutoForm)
   s.ans_pair_short = 0;
   s.rgb = rgb ? 1 : 0;
   return s;
@@ -159,9 +159,9 @@ StageConfig DefaultStageConfig(bool rgb) {
 
 // The rANS forms of the 4-wave x 2-group shape with tables built in LDS
 // (GST_ANS_FORM_*): PLAIN is AnsDecodeKernel<4, 2, true> (units of 8 groups of one
-// stream, 7 work-groups per CU); PAIRED and AUTO run AnsAutoKernel, which reads the
-// unit code of its plan: AUTO pairs short remainders only when the 8-group units would
-// not fit the device in one pass at 6 work-groups per CU.
+// stream, 7 work-groups per CU); PAIRED runs AnsAutoKernel, which reads the unit code of its
+// plan.  AUTO, set by SetAutoForm once the images are known, is AnsChainKernel (ChainFits) or
+// AnsAutoKernel, with short remainders paired (AutoPairs) or not.
 void SetAnsForm(StageConfig *s, uint32_t form, bool pair = true) {
   s->ans_auto = (form == GST_ANS_FORM_PAIRED || form == GST_ANS_FORM_AUTO) ? 1 : 0;
   s->ans_pair_short = (form == GST_ANS_FORM_PAIRED || (form == GST_ANS_FORM_AUTO && pair)) ? 1 : 0;
@@ -180,11 +180,23 @@ bool AutoPairs(const ImageDesc *descs, uint32_t n) {
 }
 
 // Whether GST_ANS_FORM_AUTO takes AnsChainKernel: while its work-groups of four groups fit
-// the device in one pass (four a CU, by LDS).  Up to there it is far ahead; a few in a second
-// pass take most of that back, and many lose, since AnsAutoKernel's waves carry two groups.
-// Batches of 1024x1024 images, us a decode with it and with AnsAutoKernel: 480 groups 26.8 /
-// 41.6, 2,040 41.0 / 53.5, 4,080 (4 a CU) 54.7 / 66.0, 4,620 64.4 / 67.8, 5,400 69.5 / 70.9,
-// 7,200 83.2 / 80.7.
+// the device in one pass (four a CU, by LDS).  Up to there it is far ahead of AnsAutoKernel for
+// a plan alone; a second pass takes most of that back at once.  From 4 to 5 work-groups a CU it
+// still leads by up to 4 %, but there several plans in flight, which share the CUs, are slower
+// with it by 6 to 13 %, so the line stays where the one pass ends.
+// Batches of 1024x1024 images (uneven ones from 512x512 to 2048x2048 lie within 2 %), us a
+// decode with it / with AnsAutoKernel, for a plan alone, then 2 and 4 plans on streams of their
+// own:
+//     480 groups, 0.5 a CU   27.1 / 42.1   14.8 / 22.0   10.4 / 13.0
+//   2,040         2.0        40.9 / 53.4   26.8 / 30.5   22.3 / 20.3
+//   3,600         3.5        53.3 / 60.0   38.0 / 36.6   34.5 / 30.3
+//   4,080         4.0        55.4 / 64.6   40.9 / 39.3   38.5 / 33.8
+//   4,380         4.3        63.0 / 65.9   43.0 / 40.7   47.0 / 44.5
+//   4,620         4.5        65.5 / 66.5   45.2 / 41.9   43.8 / 39.1
+//   5,100         5.0        67.8 / 67.9   48.7 / 45.8   49.1 / 44.0
+//   7,200         7.0        82.7 / 78.3   66.0 / 56.6   69.9 / 63.6
+// A bind cannot know what else will run.  A program that keeps 4 plans of 2 or more work-groups
+// a CU in flight at once decodes faster with GST_ANS_FORM_PLAIN.
 bool ChainFits(const ImageDesc *descs, uint32_t n) {
   uint64_t units = 0;
   for (uint32_t i = 0; i < n; ++i) units += gst::ChainUnitsOf(descs[i]);
@@ -666,7 +678,7 @@ class PinnedPool {
 // What a host-to-host decode needs beside pinned memory: a stream of its own with scratch
 // for it, a pinned word for the error bits and the staging buffer on the device.  Creating them all
 // took most of a call's time (a 1024x1024 file 163 us in the library, of which the GPU's
-// part is 35; with them kept 72).  At most kKept stay for later calls, each with one call
+// part is 35; with them kept 72; in all 229 us without anything kept, 69 with).  At most kKept stay for later calls, each with one call
 // at a time; gst_free_decompressor gives them back.
 class HostCalls {
  public:
@@ -1314,7 +1326,8 @@ int gst_batch_bind(gst_batch *b, const gst_header *hdrs, uint32_t n, const void 
              static_cast<uint8_t *>(d_outs[i]), b->stage.rgb != 0, &descs[i]);
     off += c.total;
   }
-  // The form travels in the plan, so a captured graph replays whichever one a bind picks.
+  // AUTO picks one of two kernels here.  The plan carries AnsAutoKernel's form; which kernel is
+  // the launches' matter: gst_batch_launch_graph replays exec[ans_chain].
   if (b->auto_form) SetAutoForm(&b->stage, descs.data(), n);
   b->bound = std::move(descs);
   uint32_t units[gst::kNumUnitKinds];

@@ -246,8 +246,9 @@ struct StageConfig {
                                  // (4 waves x 2 groups, tables built in LDS)
   uint32_t ans_auto;             // 1: AnsAutoKernel (4 waves x 2 groups, tables built in LDS),
                                  // which takes the form (ans_pair_short) from the unit code
-  uint32_t ans_chain;            // 1, with ans_auto: AnsChainKernel on the same units instead
-                                 // (few groups: a wave per group, one LDS round trip a step)
+  uint32_t ans_chain;            // 1, with ans_auto: AnsChainKernel instead, on units of its own
+                                 // (kStageChain; few groups: a wave per group, one LDS round
+                                 // trip a step)
   uint32_t wavelet_waves;        // waves per wavelet work-group (1, 2, 4); a wave takes 2 units
   uint32_t fused_waves;          // 0: separate index scan and assembly; else waves per
                                  // work-group of the fused scan + DXT1 assembly (1, 2, 4)
@@ -353,7 +354,8 @@ hipError_t ClearAndWait(void *p, size_t n);
 
 // Coherent pinned host memory that host-to-host calls pass their data through.  A few
 // buffers are kept for later calls, each with one call at a time (gst_free_decompressor
-// gives them back); allocating one takes some hundred microseconds.
+// gives them back); allocating one takes some hundred microseconds.  TakePinned fails above 64
+// MiB and where the runtime has none to give: the calls go on without it.
 struct PinnedBuffer {
   uint8_t *host = nullptr;
   uint8_t *dev = nullptr;  // its address for device code

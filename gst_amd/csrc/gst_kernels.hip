@@ -942,11 +942,11 @@ __global__ __launch_bounds__(kAutoWaves * 64, 6) void AnsAutoKernel(KernelArgs a
 //
 // A step is bound by that chain: 101 cycles, about 52 of them the LDS read, and 440 a refill
 // (133 a step with an index stream's 13 refills), against some 280 in AnsAutoKernel (two LDS
-// round trips, 12 dependent VALU, two scalar hops).  Stage times, this kernel against
-// AnsAutoKernel when it came in, at 123 cycles a step: one 512x512 image 16.9 / 33.0 us,
-// 1024x1024 images by the dozen: 8 (480 groups) 21.6 / 35.4, 34 (2,040) 28.7 / 39.8, 68
-// (4,080, four waves a SIMD) 34.5 / 44.1.  LDS holds four work-groups a CU; a second pass
-// loses the gain (4,620 groups: 43.5 / 44.5; 7,200: 55.0 / 48.8).
+// round trips, 12 dependent VALU, two scalar hops).  Stage times by events, which add 1.5 us,
+// this kernel / AnsAutoKernel: one 512x512 image 18.6 / 33.6 us, 1024x1024 images by the dozen:
+// 8 (480 groups) 20.9 / 36.0, 34 (2,040) 27.8 / 39.8, 68 (4,080, four waves a SIMD) 35.7 / 43.2.
+// LDS holds four work-groups a CU; a second pass loses the gain (4,620 groups: 43.6 / 44.2;
+// 7,200: 53.7 / 47.4).
 //
 // With the four steps of a symbol word in one block and one test a ring check: one 4096x4096
 // image 21.8 -> 21.0 us, 24 images 24.3 -> 23.1, 16 512x512 images 20.3 -> 19.4, 24 groups of
@@ -1196,8 +1196,9 @@ __global__ __launch_bounds__(kChainWaves * 64, 4) void AnsChainKernel(KernelArgs
 // output of a group with a malformed end offset is zeros.  data, out and status may be
 // pinned host memory: every chunk is read once, two chunks ahead.
 //
-// 24 groups of 32 streams: 15 us, where a wave per group with two LDS round trips a step
-// and the words copied to LDS two bytes a lane took 87 us.
+// 24 groups of 32 streams: 19.0 us with data, output and status in pinned memory, 16.4 with all
+// of them in device memory, where a wave per group with two LDS round trips a step and the words
+// copied to LDS two bytes a lane took 87 us.
 __global__ __launch_bounds__(kChainWaves * 64, 4) void AnsGroupsKernel(const uint32_t *table, const uint8_t *data,
                                                                        uint32_t data_len, uint32_t groups,
                                                                        uint32_t n, uint8_t *out, uint32_t *status) {

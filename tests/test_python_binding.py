@@ -36,7 +36,7 @@ class Library:
 gst_amd.lib = lambda: Library
 d = gst_amd.AnsDecoder.__new__(gst_amd.AnsDecoder)
 d._h = None
-for n in (1, 31, 32, 33, 768):
+for n in (1, 31, 32, 33, 63, 64, 65, 127, 128, 768):
     got = d.decode([0] * n, b"")
     assert len(got) == n and {type(g) for g in got} == {bytes}
     assert b"".join(got) == bytes(i % 251 for i in range(256 * n))
