@@ -182,8 +182,8 @@ bool AutoPairs(const ImageDesc *descs, uint32_t n) {
 // Whether GST_ANS_FORM_AUTO takes AnsChainKernel: while its work-groups of four groups fit
 // the device in one pass (four a CU, by LDS).  Up to there it is far ahead of AnsAutoKernel for
 // a plan alone; a second pass takes most of that back at once.  From 4 to 5 work-groups a CU it
-// still leads by up to 4 %, but there several plans in flight, which share the CUs, are slower
-// with it by 6 to 13 %, so the line stays where the one pass ends.
+// still leads by up to 5 %, but there several plans in flight, which share the CUs, are slower
+// with it by 6 to 12 %, so the line stays where the one pass ends.
 // Batches of 1024x1024 images (uneven ones from 512x512 to 2048x2048 lie within 2 %), us a
 // decode with it / with AnsAutoKernel, for a plan alone, then 2 and 4 plans on streams of their
 // own:

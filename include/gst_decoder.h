@@ -73,7 +73,9 @@ int gst_parse_header(const uint8_t *file, size_t len, gst_header *hdr);
 
 /* Replaces GenTC::DecompressDXT (codec/decoder.h:16-17, codec/decoder.cpp:487-532):
  * host .gtc bytes in, host DXT1 blocks out (out_len >= w*h/2).  Blocking.  Returns
- * GST_ERR_CORRUPT_STREAM when the kernels raised an error bit. */
+ * GST_ERR_CORRUPT_STREAM when the kernels raised an error bit.  File and blocks pass through
+ * kept pinned memory while both fit 64 MiB (and the runtime has it), else through ordinary
+ * memory with the runtime's copies. */
 int gst_decompress_dxt(const uint8_t *file, size_t len, uint8_t *out, size_t out_len);
 
 /* Replaces GenTC::LoadCompressedDXT (codec/decoder.h:19-21, codec/decoder.cpp:534-538).
@@ -230,7 +232,9 @@ typedef struct gst_batch_config {
 /* rANS work-group forms (gst_batch_config.ans_form, gst_tune_result.ans_form). */
 #define GST_ANS_FORM_AUTO 0   /* chosen at each bind: a kernel with a wave per group and one
                                  LDS round trip a step while its work-groups of 4 groups
-                                 fit the device in one pass at 4 per CU; else work-groups
+                                 fit the device in one pass at 4 per CU (programs that keep
+                                 4 plans of that size in flight at once are faster with
+                                 PLAIN); else work-groups
                                  of 8 groups of one stream while those fit at 6 per CU,
                                  else PAIRED (gst_batch_launch_graph replays whichever the
                                  bind chose; launches that a caller captured keep their
@@ -247,8 +251,9 @@ int gst_batch_bind(gst_batch *b, const gst_header *hdrs, uint32_t n, const void 
                    void *const *d_outs, gst_stream stream);
 /* Enqueues the five stages for the bound images. */
 int gst_batch_decode(gst_batch *b, gst_stream stream);
-/* Captures the five launches of the bound plan into a hipGraph (once); later
- * gst_batch_launch_graph replays it for whatever batch is bound. */
+/* Captures the launches of the bound plan into a hipGraph (once; with GST_ANS_FORM_AUTO into
+ * two, one with each rANS kernel that a bind may choose); later gst_batch_launch_graph replays
+ * it for whatever batch is bound. */
 int gst_batch_capture_graph(gst_batch *b, gst_stream stream);
 int gst_batch_launch_graph(gst_batch *b, gst_stream stream);
 /* Per-stage kernel time (ms) of one decode, measured with hipEvents on `stream`:
