@@ -184,7 +184,7 @@ bool AutoPairs(const ImageDesc *descs, uint32_t n) {
 // a plan alone; a second pass takes most of that back at once.  From 4 to 5 work-groups a CU it
 // still leads by up to 5 %, but there several plans in flight, which share the CUs, are slower
 // with it by 6 to 12 %, so the line stays where the one pass ends.
-// Batches of 1024x1024 images (uneven ones from 512x512 to 2048x2048 lie within 2 %), us a
+// Batches of 1024x1024 images (uneven ones from 512x512 to 2048x2048 lie within 3 %), us a
 // decode with it / with AnsAutoKernel, for a plan alone, then 2 and 4 plans on streams of their
 // own:
 //     480 groups, 0.5 a CU   27.1 / 42.1   14.8 / 22.0   10.4 / 13.0
